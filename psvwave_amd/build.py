@@ -15,7 +15,7 @@ LIB = os.path.join(HERE, "libpsvwave_amd.so")
 ARCH = os.environ.get("PSV_OFFLOAD_ARCH", "gfx950")
 ROCM = os.environ.get("ROCM_PATH", "/opt/rocm")
 
-SOURCES = ["psv_config.cpp", "psv_kernels.hip", "psv_model.hip",
+SOURCES = ["psv_config.cpp", "psv_kernels.hip", "psv_loop.hip", "psv_model.hip",
            "psv_batch.hip", "psv_conv.hip", "psv_capi.cpp"]
 
 # -ffp-contract=off: every multiply and add rounds separately, as in the

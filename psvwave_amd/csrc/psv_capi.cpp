@@ -568,6 +568,10 @@ int psv_synchronize(psv_model *m) {
   return guard([&] { M(m); });
 }
 
+int psv_refuse_resident_loops(psv_model *m) {
+  return guard([&] { M(m).refuse_next_loops(); });
+}
+
 int psv_set_checkpointing(psv_model *m, int every) {
   return guard([&] { M(m).set_checkpointing(every); });
 }

@@ -341,10 +341,14 @@ hipError_t launch_adjoint_sources(const double *sx, const double *sz,
                                   double *ax, double *az, long long n,
                                   hipStream_t s);
 // Adds deferred correlation terms [slot][rho, lam, mu][nx * nz] to the
-// kernels over the kernel region, slots from last to first.
+// kernels over the kernel region, slots from last to first.  With `poison`
+// (see LoopLaunch) it does nothing when the word is set, and else writes 1
+// to *status (host memory).
 hipError_t launch_replay_correlation(double *rho_k, double *lam_k, double *mu_k,
                                      const double *d, int nslots, long long ngrid, int nx,
-                                     int kx0, int kx1, int kz0, int kz1, hipStream_t s);
+                                     int kx0, int kx1, int kz0, int kz1, hipStream_t s,
+                                     const unsigned *poison = nullptr,
+                                     unsigned *status = nullptr);
 hipError_t launch_map_kernels(const double *vp, const double *vs,
                               const double *rho, const double *lam_k,
                               const double *mu_k, const double *rho_l,

@@ -2996,9 +2996,14 @@ hipError_t launch_step(int variant, const StepArgs &a, hipStream_t s,
 __global__ void replay_correlation_kernel(double *rho_k, double *lam_k, double *mu_k,
                                           const double *__restrict__ d, int nslots,
                                           long long ngrid, int nx, int kx0, int kx1,
-                                          int kz0, int kz1) {
+                                          int kz0, int kz1, const unsigned *poison,
+                                          unsigned *status) {
   const long long w = kx1 - kx0;
   const long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x;
+  if (poison) {
+    if (*poison) return;
+    if (i == 0) *status = 1;
+  }
   if (i >= w * (kz1 - kz0)) return;
   const long long ci = (long long)(kz0 + i / w) * nx + kx0 + i % w;
   double r = rho_k[ci], l = lam_k[ci], m = mu_k[ci];
@@ -3015,11 +3020,15 @@ __global__ void replay_correlation_kernel(double *rho_k, double *lam_k, double *
 
 hipError_t launch_replay_correlation(double *rho_k, double *lam_k, double *mu_k,
                                      const double *d, int nslots, long long ngrid, int nx,
-                                     int kx0, int kx1, int kz0, int kz1, hipStream_t s) {
+                                     int kx0, int kx1, int kz0, int kz1, hipStream_t s,
+                                     const unsigned *poison, unsigned *status) {
   const long long n = (long long)(kx1 - kx0) * (kz1 - kz0);
-  if (n <= 0 || nslots <= 0) return hipSuccess;
+  if (n <= 0 || nslots <= 0) {
+    if (status) *status = 1;
+    return hipSuccess;
+  }
   hipLaunchKernelGGL(replay_correlation_kernel, dim3(blocks_for(n, 256)), dim3(256), 0, s,
-                     rho_k, lam_k, mu_k, d, nslots, ngrid, nx, kx0, kx1, kz0, kz1);
+                     rho_k, lam_k, mu_k, d, nslots, ngrid, nx, kx0, kx1, kz0, kz1, poison, status);
   return hipGetLastError();
 }
 

@@ -1,0 +1,933 @@
+// psv_loop.hip -- resident time loops.
+//
+// A launch per time step reads and writes the whole state and reads the
+// materials every step (104 B per point) and pays the launch latency.  On
+// this device the state fits on chip: 256 compute units hold 128 MB of
+// registers and 40 MB of LDS.  A resident loop therefore runs all time steps
+// in one launch.  Each block owns one tile for the whole loop; stresses and
+// material factors of its points stay in registers, velocities in LDS, and
+// per step only the velocities on the three-point rim of each tile move, from
+// block to block through memory.  What bounds a step is then FP64 issue
+// (about 125 FP64 instructions per point) plus one exchange latency.
+//
+// Tile.  Eight waves; lane l of every wave is column x0 - 2 + l, wave w holds
+// the rows q = w P .. w P + P - 1 of the tile, row q being z0 - 2 + q.  The
+// velocity update of the own points needs stresses two points beyond them:
+// the two outer lanes on either side and the two outer rows at either end
+// compute those ring stresses redundantly from exchanged velocities, so one
+// exchange per step suffices and every lane runs the same code.  Own points:
+// up to 60 columns and 8 P - 4 rows.
+//
+// Exchange.  A velocity on a tile's rim is sent as one 16-byte cell {low word, tag,
+// high word, tag}: each 8-byte half carries its own tag (the step's number),
+// so a receiver polls the cells themselves and needs no separate flag, no
+// fence and no ordering between stores.  Cells are written and read at
+// device scope (past the XCD's own L2).  Two cell sets alternate: a block
+// overwrites the cells of step k at step k + 2, after it has received every
+// neighbour's step k + 1, which that neighbour sends after consuming step k
+// (neighbours read each other's rims on all sides, so this holds for each
+// pair of tiles that exchange anything; tiles are at least 3 points wide and
+// high, so only adjacent tiles do).
+//
+// All blocks of a launch must be resident at once.  The gate below admits no
+// more blocks than the device holds; should other work in another process
+// keep some of them out, the blocks notice at the start (bounded wait), all
+// of them leave without having written anything, and the host runs the loop
+// with one launch per step instead.
+#include "psv_loop.h"
+
+#include <algorithm>
+#include <mutex>
+#include <string>
+#include <type_traits>
+
+#include "psv_model.h"
+
+namespace psv {
+
+namespace {
+
+typedef const LoopArgs __attribute__((address_space(4))) ConstArgs;
+// Device memory behind a generic pointer that was itself read from memory.
+template <class T>
+using Global = __attribute__((address_space(1))) T;
+template <class T>
+__device__ __forceinline__ Global<T> *gp(T *p) {
+  return (Global<T> *)p;
+}
+
+typedef unsigned u32x4 __attribute__((ext_vector_type(4)));
+
+constexpr int kVW = 67;  // velocity columns -2 .. 64 around the 64 lanes; column
+                         // 65, which no value in use depends on, is the next
+                         // row's column -2, always zero
+constexpr int kDeviceScope = 16;  // buffer cache policy: device scope (sc1)
+
+// A value the compiler cannot see through: what is computed from it in a
+// time step is not kept in registers across all of them.
+__device__ __forceinline__ int fresh(int v) {
+  asm volatile("" : "+v"(v));
+  return v;
+}
+__device__ __forceinline__ double fresh(double v) {
+  asm volatile("" : "+v"(v));
+  return v;
+}
+__device__ __forceinline__ const ConstArgs *fresh(const ConstArgs *v) {
+  asm volatile("" : "+s"(v));
+  return v;
+}
+
+// Divisions x / d by a grid spacing d in [2^-40, 2^40].  All give the
+// correctly rounded quotient; which one a pass may use depends on the values
+// around.  `base` is the difference x was formed from: x itself, or x without
+// its material factor.
+//
+// NormalQuotient: FastDiv's operations (psv_kernels.hip), for x = 0 or
+// 2^-960 <= |x| <= 2^980.
+struct NormalQuotient {
+  double d, y, zh, zl;
+  __device__ bool tiny(double) const { return false; }
+  __device__ double operator()(double x, bool) const {
+    const double q0 = __builtin_fma(x, zl, x * zh);
+    const double r = __builtin_fma(q0, d, -x);
+    return __builtin_fma(-r, y, q0);
+  }
+};
+// SmallQuotient: every |x| <= 2^980, subnormal x and quotients included.
+// Where the difference is below 2^-500, x is scaled by 2^128 first (exactly),
+// and the last operation, a fused multiply-add that in such lanes scales its
+// result by 2^-128 before its one rounding, undoes it (with factors of
+// exponents in [-300, 100], x is below 2^-400 there and above 2^-800 or zero
+// elsewhere).
+struct SmallQuotient {
+  double d, y, zh, zl;
+  __device__ bool tiny(double base) const { return __builtin_fabs(base) < 0x1p-500; }
+  __device__ double operator()(double x, bool t) const {
+    const double xs = __builtin_amdgcn_ldexp(x, fresh(t ? 128 : 0));
+    const double q0 = __builtin_fma(xs, zl, xs * zh);
+    const double r = __builtin_fma(q0, d, -xs);
+    return __builtin_amdgcn_div_fmas(-r, y, q0, t);
+  }
+};
+struct PlainQuotient {
+  double d;
+  __device__ bool tiny(double) const { return false; }
+  __device__ double operator()(double x, bool) const { return x / d; }
+};
+
+// Which division the next pass over some values needs: kNormal if each is
+// zero or of a binary exponent (frexp) in [elimit, 600]; kSmall if only the
+// lower bound fails, as in the numerical precursor ahead of a wavefront;
+// kIeee otherwise (a plain IEEE division for every value: runs that
+// overflow).  Two roundings of differences can cancel to 2^-109 of the
+// smallest value, so with material factors of exponents e_f in [-300, 100] a
+// dividend is zero or at least 2^(elimit - 110 + min(e_f, 0)); elimit =
+// -849 - min(e_f, 0) keeps that above 2^-960.  The upper bound leaves room
+// for one step's growth, so a value that is not finite is never the first
+// one out of range.
+enum : int { kNormal = 0, kSmall = 1, kIeee = 2 };
+constexpr int kExpMax = 600;
+struct Range {
+  int emin = 0, emax = 0;  // of zeros and of values that are not finite: 0
+  __device__ void values(double a, double b) {
+    const int ea = __builtin_amdgcn_frexp_exp(a), eb = __builtin_amdgcn_frexp_exp(b);
+    emin = min(emin, min(ea, eb));
+    emax = max(emax, max(ea, eb));
+  }
+  // also for values that may be infinite or no numbers
+  __device__ void any_values(double a, double b) {
+    values(a, b);
+    if (!(__builtin_fabs(a) + __builtin_fabs(b) < 0x1p800)) emax = 4096;
+  }
+  // adds the wave's need to *word (in LDS): one lane's atomic per wave, not
+  // one per lane, which all hit one bank
+  __device__ void report(int *word, int elimit) const {
+    const unsigned long long small = __ballot(emin < elimit), large = __ballot(emax > kExpMax);
+    if (small | large) {
+      const int m = (small ? kSmall : 0) | (large ? kIeee : 0);
+      if ((int)__ffsll((unsigned long long)__ballot(1)) - 1 == (int)(threadIdx.x & 63))
+        atomicOr(word, m);
+    }
+  }
+};
+
+// Stresses of one point (stress_point's expression trees).  vxx: vx at x-1,
+// x+1, x+2; vxz: vx at z-1, z, z+1, z+2; vzx: vz at x-2, x-1, x+1; vzz: vz
+// at z-2, z-1, z, z+1.  la = lm - 2 mu, dm = dts * mu.
+template <bool FINITE, class D>
+__device__ __forceinline__ void loop_stress(const double (&vxx)[3], double vxm, double vx0,
+                                            double vxp, double vxpp, const double (&vzx)[3],
+                                            double vzmm, double vzm, double vz0, double vzp,
+                                            double lm, double la, double dm, double taper,
+                                            double dts, D divx, D divz, Range &range, double &xx,
+                                            double &zz, double &xz) {
+  const double dvx_x = kC1 * (vxx[1] - vx0) + kC2 * (vxx[0] - vxx[2]);
+  const double dvz_z = kC1 * (vz0 - vzm) + kC2 * (vzmm - vzp);
+  const double dvx_z = kC1 * (vxp - vx0) + kC2 * (vxm - vxpp);
+  const double dvz_x = kC1 * (vz0 - vzx[1]) + kC2 * (vzx[0] - vzx[2]);
+  const bool tx = divx.tiny(dvx_x), tz = divz.tiny(dvz_z);
+  xx = taper * (xx + dts * (divx(lm * dvx_x, tx) + divz(la * dvz_z, tz)));
+  zz = taper * (zz + dts * (divx(la * dvx_x, tx) + divz(lm * dvz_z, tz)));
+  xz = taper * (xz + dm * (divz(dvx_z, divz.tiny(dvx_z)) + divx(dvz_x, divx.tiny(dvz_x))));
+  if (FINITE) {
+    range.values(xx, zz);
+    range.values(xz, xz);
+  } else {
+    range.any_values(xx, zz);
+    range.any_values(xz, xz);
+  }
+}
+
+// Velocities of one point (velocity_point's expression trees).  xxx: txx at
+// x-2, x-1, x+1; xzx: txz at x-1, x+1, x+2.  bd = b * dts.
+template <bool FINITE, class D>
+__device__ __forceinline__ void loop_velocity(const double (&xxx)[3], double xx0,
+                                              const double (&xzx)[3], double xzmm, double xzm,
+                                              double xz0, double xzp, double zzm, double zz0,
+                                              double zzp, double zzpp, double bd, double taper,
+                                              D divx, D divz, Range &range, double &vx,
+                                              double &vz) {
+  const double dxx_x = kC1 * (xx0 - xxx[1]) + kC2 * (xxx[0] - xxx[2]);
+  const double dxz_z = kC1 * (xz0 - xzm) + kC2 * (xzmm - xzp);
+  const double dxz_x = kC1 * (xzx[1] - xz0) + kC2 * (xzx[0] - xzx[2]);
+  const double dzz_z = kC1 * (zzp - zz0) + kC2 * (zzm - zzpp);
+  vx = taper * (vx + bd * (divx(dxx_x, divx.tiny(dxx_x)) + divz(dxz_z, divz.tiny(dxz_z))));
+  vz = taper * (vz + bd * (divx(dxz_x, divx.tiny(dxz_x)) + divz(dzz_z, divz.tiny(dzz_z))));
+  if (FINITE)
+    range.values(vx, vz);
+  else
+    range.any_values(vx, vz);
+}
+
+// Keeps the scheduler from interleaving the stencils of several rows (whose
+// operands would then all be live at once).
+__device__ __forceinline__ void row_fence() { __builtin_amdgcn_sched_barrier(0); }
+
+// min(a, b) of factors that are no NaN (one instruction; fmin adds a quieting
+// one per operand).
+__device__ __forceinline__ double min_factor(double a, double b) {
+  double r;
+  asm("v_min_f64 %0, %1, %2" : "=v"(r) : "v"(a), "v"(b));
+  return r;
+}
+
+// The blocks of a launch meet before any of them writes anything: true when
+// all are resident.  state: 0 waiting, 1 go, 2 leave; exactly one of go and
+// leave is ever decided.
+__device__ bool loop_meet(const LoopLaunch &l) {
+  unsigned *const state = l.sync + 1;
+  if (l.poison && __hip_atomic_load(l.poison, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) {
+    unsigned want = 0;
+    __hip_atomic_compare_exchange_strong(state, &want, 2u, __ATOMIC_RELAXED, __ATOMIC_RELAXED,
+                                         __HIP_MEMORY_SCOPE_AGENT);
+  } else if (__hip_atomic_fetch_add(l.sync, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) +
+                 1 ==
+             (unsigned)l.nblocks) {
+    unsigned want = 0;
+    if (__hip_atomic_compare_exchange_strong(state, &want, 1u, __ATOMIC_RELAXED,
+                                             __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT))
+      __hip_atomic_store(l.status, (unsigned)kLoopRan, __ATOMIC_RELAXED,
+                         __HIP_MEMORY_SCOPE_SYSTEM);
+  }
+  // 0.1 s of the 100 MHz constant clock: the gate lets no other launch of this
+  // process wait here meanwhile
+  const unsigned long long t0 = __builtin_amdgcn_s_memrealtime();
+  for (;;) {
+    const unsigned s = __hip_atomic_load(state, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    if (s) {
+      if (s == 2 && l.poison)
+        __hip_atomic_store(l.poison, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      return s == 1;
+    }
+    if (__builtin_amdgcn_s_memrealtime() - t0 > 10000000ull) {
+      unsigned want = 0;
+      __hip_atomic_compare_exchange_strong(state, &want, 2u, __ATOMIC_RELAXED,
+                                           __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    }
+    __builtin_amdgcn_s_sleep(2);
+  }
+}
+
+template <int KIND, bool ADJ>
+__global__ void __launch_bounds__(64 * kLoopKinds[KIND].waves)
+    __attribute__((amdgpu_waves_per_eu(4, 4)))
+resident_loop(LoopLaunch l) {
+  constexpr int P = kLoopKinds[KIND].rows, NW = kLoopKinds[KIND].waves;
+  constexpr int NT = 64 * NW, SR = NW * P;
+  constexpr int VROWS = SR + 4;  // velocity rows q = -2 .. SR + 1
+  constexpr int NV = VROWS * kVW + 1;
+  // rim and frame cells per thread (own at most 60 x (SR - 4))
+  constexpr int NSEND = (60 * (SR - 4) - 54 * (SR - 10) + NT - 1) / NT;
+  constexpr int NRECV = (66 * (SR + 2) - 60 * (SR - 4) + NT - 1) / NT;
+  constexpr int RIM = loop_rim_cells(KIND);
+  static_assert(NSEND * NT <= RIM, "a tile's rim fits its cells");
+  __shared__ double s_vx[NV], s_vz[NV];
+  __shared__ double s_tz[SR];  // taper factors of the rows
+  // txz of all rows, txx of the own rows 2 .. SR - 3, and of tzz the rows other
+  // waves read, each wave's rows 0, 1 and P - 1
+  constexpr int ZR = P < 3 ? P : 3;
+  __shared__ double s_xz[SR * 64], s_xx[(SR - 4) * 64], s_zz[NW * ZR * 64];
+  // what the next pass over the velocities (by step parity) and over the
+  // stresses needs, kNormal | kSmall | kIeee
+  __shared__ int s_vmode[2], s_smode, s_factor;
+  __shared__ int s_go, s_stall;
+
+  const Global<const int> *const bp = gp((const int *)(l.blocks + blockIdx.x));
+  const struct { int x, y, z; } bt = {bp[0], bp[1], bp[2]};
+  // the arguments do not change while the launch runs: read through the
+  // constant address space, uniform values stay in scalar registers
+  const ConstArgs &A0 = ((const ConstArgs *)l.loops)[bt.x], &A = A0;
+  if (threadIdx.x == 0) {
+    s_go = loop_meet(l);
+    s_stall = 0;
+    s_smode = s_factor = 0;
+  }
+  __syncthreads();
+  if (!s_go) return;
+
+  const int lane = threadIdx.x & 63;
+  const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int nx = A.nx, nz = A.nz, nt = A.nt;
+  const int tile = bt.z * A.ntx + bt.y;
+  const int x0 = (int)((long long)bt.y * nx / A.ntx);
+  const int z0 = (int)((long long)bt.z * nz / A.ntz);
+  const int wt = (int)((long long)(bt.y + 1) * nx / A.ntx) - x0;  // own columns
+  const int ht = (int)((long long)(bt.z + 1) * nz / A.ntz) - z0;  // own rows
+  const int q0 = w * P;         // first row of the strip
+  const int zs = z0 - 2 + q0;   // its grid row
+  const int x = x0 - 2 + lane;
+  const bool own_x = lane >= 2 && lane < 2 + wt;
+  // strip rows with a stress / velocity stencil, and own rows
+  auto clampj = [&](int j) { return min(max(j, 0), P); };
+  const int js0 = clampj(2 - zs), js1 = clampj(min(nz - 2 - zs, ht + 4 - q0));
+  const int jo0 = clampj(2 - q0), jo1 = clampj(ht + 2 - q0);
+  const int jv0 = max(js0, jo0), jv1 = min(jo1, clampj(nz - 2 - zs));
+  const bool xs = x >= 2 && x < nx - 2 && lane < wt + 4;
+  const bool xv = own_x && xs;
+  const double dts = A.dts;
+
+  // ---- the tile's constants and initial state ----
+  double lm[P], la[P], dm[P], bd[P];
+  double xx[P], zz[P], xz[P];
+  int factor_exp = 0;  // smallest of the material factors; -4096: one is too large
+  const double tx = gp(A.taper_x)[min(x, nx + 1)];
+  {
+    const int xc = min(x, nx + 1);
+#pragma unroll
+    for (int j = 0; j < P; ++j) {
+      const int zc = min(zs + j, nz + 1);
+      const long long g = A.origin + (long long)zc * A.pitch + xc;
+      const double m = gp(A.mu)[g];
+      lm[j] = gp(A.lm)[g];
+      la[j] = lm[j] - 2 * m;
+      dm[j] = dts * m;
+      bd[j] = gp(A.b)[g] * dts;
+      for (double f : {lm[j], la[j]})
+        if (f != 0.0) factor_exp = min(factor_exp, __builtin_amdgcn_frexp_exp(f));
+      for (double f : {lm[j], la[j], m, dm[j], bd[j], dts})
+        if (!(__builtin_fabs(f) <= 0x1p100)) factor_exp = -4096;
+      xx[j] = zz[j] = xz[j] = 0.0;
+      if (A.in[0] && x >= 0 && x < nx && zs + j >= 0 && zs + j < nz) {
+        const long long s = A.in_origin + (long long)(zs + j) * A.in_pitch + x;
+        xx[j] = gp(A.in[2])[s];
+        zz[j] = gp(A.in[3])[s];
+        xz[j] = gp(A.in[4])[s];
+      }
+    }
+  }
+  for (int i = threadIdx.x; i < SR; i += NT) s_tz[i] = gp(A.taper_z)[min(z0 - 2 + i, nz + 1)];
+  // a tile with factors out of range divides by the IEEE sequence throughout,
+  // and so does the first step from a given state, whose values are not tested
+  if (factor_exp < 0) atomicMin(&s_factor, factor_exp);
+  if (threadIdx.x == 0) {
+    s_vmode[A.k0 & 1] = kNormal;
+    s_vmode[(A.k0 + 1) & 1] = A.in[0] ? kIeee : kNormal;
+  }
+  for (int i = threadIdx.x; i < NV; i += NT) {
+    const int r = i / kVW, c = i - r * kVW;
+    const int zi = z0 - 2 + r - 2, xi = x0 - 2 + c - 2;
+    double a = 0.0, b = 0.0;
+    if (A.in[0] && xi >= x0 - 3 && xi < x0 + wt + 3 && zi >= z0 - 3 && zi < z0 + ht + 3 &&
+        xi >= 0 && xi < nx && zi >= 0 && zi < nz) {
+      const long long s = A.in_origin + (long long)zi * A.in_pitch + xi;
+      a = gp(A.in[0])[s];
+      b = gp(A.in[1])[s];
+    }
+    s_vx[i] = a;
+    s_vz[i] = b;
+  }
+
+  // ---- this thread's cells ----
+  // A tile's rim cells are numbered along its first three and last three
+  // rows, then the first three columns of the rows between, then the last
+  // three, so that what a neighbour reads lies together;
+  // cell i of component c and set p lies at ((tile * 2 + p) * 2 + c) * RIM +
+  // i.  So a line of cells has one writer, and no tile reads lines that it
+  // writes: with cells of several tiles in one line, a read waited for the
+  // reader's own write to reach memory first (1.7 us instead of 0.7).
+  auto vidx = [](int r, int c) { return (r + 4) * kVW + c + 4; };
+  auto rim_cell = [](int wt, int ht, int r, int c) {
+    if (wt <= 6 || ht <= 6) return r * wt + c;
+    if (r < 3) return r * wt + c;
+    if (r >= ht - 3) return (r - ht + 6) * wt + c;
+    return 6 * wt + (c < 3 ? (r - 3) * 3 + c : (ht + r - 9) * 3 + c - wt + 3);
+  };
+  int send_l[NSEND], recv_l[NRECV];
+  unsigned recv_g[NRECV];
+#pragma unroll
+  for (int s = 0; s < NSEND; ++s) {
+    const int i = threadIdx.x + s * NT;
+    int r, c;
+    bool on;
+    if (wt > 6 && ht > 6) {
+      on = i < 6 * wt + 6 * (ht - 6);
+      if (i < 6 * wt) {
+        const int k = i / wt;
+        r = k < 3 ? k : ht - 6 + k;
+        c = i - k * wt;
+      } else {
+        const int k = (i - 6 * wt) / 3, m = i - 6 * wt - 3 * k;
+        r = 3 + (k < ht - 6 ? k : k - (ht - 6));
+        c = k < ht - 6 ? m : wt - 3 + m;
+      }
+    } else {
+      on = i < wt * ht;
+      r = i / wt;
+      c = i - r * wt;
+    }
+    send_l[s] = on ? vidx(r, c) : -1;
+  }
+#pragma unroll
+  for (int s = 0; s < NRECV; ++s) {
+    const int i = threadIdx.x + s * NT;
+    const int fw = wt + 6, rows = 3 * fw;
+    int r, c;
+    bool on = i < 2 * rows + 6 * ht;
+    if (i < 2 * rows) {
+      const int k = i / fw;
+      r = k < 3 ? k - 3 : ht - 3 + k;
+      c = i - k * fw - 3;
+    } else {
+      const int k = (i - 2 * rows) / 3, m = i - 2 * rows - 3 * k;
+      r = k < ht ? k : k - ht;
+      c = k < ht ? m - 3 : wt + m;
+    }
+    const int xi = x0 + c, zi = z0 + r;
+    on = on && xi >= 0 && xi < nx && zi >= 0 && zi < nz;
+    recv_l[s] = on ? vidx(r, c) : -1;
+    recv_g[s] = 0;
+    if (on) {  // the adjacent tile that owns the point
+      const int ox = bt.y + (c < 0 ? -1 : c >= wt ? 1 : 0);
+      const int oz = bt.z + (r < 0 ? -1 : r >= ht ? 1 : 0);
+      const int ox0 = (int)((long long)ox * nx / A.ntx), oz0 = (int)((long long)oz * nz / A.ntz);
+      const int ow = (int)((long long)(ox + 1) * nx / A.ntx) - ox0;
+      const int oh = (int)((long long)(oz + 1) * nz / A.ntz) - oz0;
+      recv_g[s] = (unsigned)((oz * A.ntx + ox) * 4 * RIM +
+                             rim_cell(ow, oh, zi - oz0, xi - ox0)) * 16u;
+    }
+  }
+  const auto cells =
+      __builtin_amdgcn_make_buffer_rsrc(A.cells, 0, A.cells_bytes, 0x00020000);
+  const unsigned send_g = (unsigned)(tile * 4 * RIM + (int)threadIdx.x) * 16u;
+
+  // ---- this wave's injection targets: target t in lane t ----
+  const int tg0 = __builtin_amdgcn_readfirstlane(gp(A.inj_off)[tile * NW + w]);
+  const int ntg = __builtin_amdgcn_readfirstlane(gp(A.inj_off)[tile * NW + w + 1]) - tg0;
+  auto inj_entry = [](const ConstArgs &A, int e) {
+    const Global<const InjEntry> *const p = gp(A.inj) + e;
+    return InjEntry{p->local, p->comp, p->src, p->pad, p->coef};
+  };
+  auto inj_sample = [&](const ConstArgs &A, const InjEntry &E, int it) {
+    const double *const s = ADJ ? (E.comp ? A.adj_z : A.adj_x) : A.stf;
+    return gp(s)[(long long)E.src * nt + it];
+  };
+  auto inj_term = [](const ConstArgs &A, int comp, double coef, double b, double val) {
+    return ADJ ? A.dt * b * val / A.dxdz : coef * val * A.dt * b / (comp ? A.d4z : A.d4x);
+  };
+  // ---- this thread's receiver ----
+  int rec_l = -1, rec_k = 0;
+  double rec_sx = 0.0, rec_sz = 0.0;
+  if (!ADJ && A.rec_off) {
+    const int r0 = gp(A.rec_off)[tile], nr = gp(A.rec_off)[tile + 1] - r0;
+    if ((int)threadIdx.x < nr) {
+      rec_l = gp(A.rec)[r0 + threadIdx.x].local;
+      rec_k = gp(A.rec)[r0 + threadIdx.x].src;
+    }
+  }
+  __syncthreads();
+
+  const int tile_exp = __builtin_amdgcn_readfirstlane(s_factor);
+  const int floor_mode = tile_exp < -300 ? kIeee : kNormal;
+  const int elimit = -849 - tile_exp;
+  // LDS indices of the strip's first velocity and txz row, and of the rows
+  // above and below it (clamped where no stencil uses them), each to be added
+  // to the lane
+  const int vrow = (q0 + 2) * kVW + 2, srow = q0 * 64;
+  const int up2 = max(q0 - 2, 0) * 64, up1 = max(q0 - 1, 0) * 64;
+  const int dn1 = min(q0 + P, SR - 1) * 64;
+  auto zrow = [](int q) {
+    q = min(max(q, 0), SR - 1);
+    return (P < 3 ? q : q / P * 3 + (q % P == P - 1 ? 2 : q % P)) * 64;
+  };
+  const int zup = zrow(q0 - 1), zdn0 = zrow(q0 + P), zdn1 = zrow(q0 + P + 1);
+  const bool full_s = js0 == 0 && js1 == P, full_v = jv0 == 0 && jv1 == P;
+  unsigned tag = l.tag0;
+
+  // What a step does with the state at its start: receivers, snapshot store,
+  // correlation.  Called between sending the rims and waiting for the
+  // neighbours' (the state then is the next step's), which hides it.
+  int phase = (ADJ ? nt - 1 - A0.k0 : A0.k0) % A0.si;  // of the next step's time index
+  auto begin_step = [&](int k) {
+    const ConstArgs &A = *fresh(&A0);
+    const int it = ADJ ? nt - 1 - k : k;
+    const bool snap_step = phase == 0;
+    phase = ADJ ? (phase == 0 ? A.si : phase) - 1 : (phase + 1 == A.si ? 0 : phase + 1);
+    const int xk = fresh(x), va0 = vrow + fresh(lane);
+    if (rec_l >= 0) {
+      // receiver record at the start of the step (src/fdModel.cpp:576-596)
+      const double ax = A.dt * s_vx[rec_l] / A.dxdz, az = A.dt * s_vz[rec_l] / A.dxdz;
+      rec_sx = k == 0 ? ax : rec_sx + ax;
+      rec_sz = k == 0 ? az : rec_sz + az;
+      const long long at = (long long)fresh(rec_k) * nt + it;
+      gp(A.rtf_x)[at] = rec_sx;
+      gp(A.rtf_z)[at] = rec_sz;
+    }
+    if (snap_step && A.snap[0] && it / A.si % A.slot_every == 0) {
+      const int slot = it / A.si;
+      const long long so = (long long)(slot / A.slot_every - A.slot0) * A.slot_stride;
+      if (!ADJ) {
+        if (own_x)
+#pragma unroll
+          for (int j = 0; j < P; ++j)
+            if (j >= jo0 && j < jo1) {
+              const long long ci = so + (long long)(zs + j) * nx + xk;
+              __builtin_nontemporal_store(s_vx[va0 + j * kVW], gp(A.snap[0]) + ci);
+              __builtin_nontemporal_store(s_vz[va0 + j * kVW], gp(A.snap[1]) + ci);
+              __builtin_nontemporal_store(xx[j], gp(A.snap[2]) + ci);
+              __builtin_nontemporal_store(zz[j], gp(A.snap[3]) + ci);
+              __builtin_nontemporal_store(xz[j], gp(A.snap[4]) + ci);
+            }
+      } else {
+        const long long ko = A.defer_stride * slot;
+        if (own_x && x >= A.kx0 && x < A.kx1)
+#pragma unroll
+          for (int j = 0; j < P; ++j) {
+            const int z = zs + j;
+            if (j >= jo0 && j < jo1 && z >= A.kz0 && z < A.kz1) {
+              const long long c = (long long)z * nx + x, ci = so + c, ck = ko + c;
+              const long long g = A.origin + (long long)z * A.pitch + xk;
+              double r = 0.0, la_k = 0.0, m = 0.0, s[5];
+#pragma unroll
+              for (int f = 0; f < 5; ++f) s[f] = __builtin_nontemporal_load(gp(A.snap[f]) + ci);
+              if (!A.defer_stride) {
+                r = __builtin_nontemporal_load(gp(A.rho_k) + ck);
+                la_k = __builtin_nontemporal_load(gp(A.lam_k) + ck);
+                m = __builtin_nontemporal_load(gp(A.mu_k) + ck);
+              }
+              correlate_point(A.wcorr, lm[j], gp(A.mu)[g], s_vx[va0 + j * kVW], s_vz[va0 + j * kVW],
+                              xx[j], zz[j], xz[j], s[0], s[1], s[2], s[3], s[4], r, la_k, m);
+              __builtin_nontemporal_store(r, gp(A.rho_k) + ck);
+              __builtin_nontemporal_store(la_k, gp(A.lam_k) + ck);
+              __builtin_nontemporal_store(m, gp(A.mu_k) + ck);
+            }
+          }
+      }
+    }
+
+  };
+  begin_step(A.k0);
+
+  for (int k = A.k0; k < A.k1; ++k, ++tag) {
+    const int it = ADJ ? nt - 1 - k : k;
+    const double txk = fresh(tx);
+    // ---- stresses ----
+    auto stress_pass = [&](auto full, auto divx, auto divz) {
+      constexpr bool FULL = decltype(full)::value;
+      constexpr bool FINITE = !std::is_same<decltype(divx), PlainQuotient>::value;
+      const int va = vrow + fresh(lane), ta = fresh(q0);
+      Range range;
+      // vx rows -1 .. P + 1 and vz rows -2 .. P of the lane's column
+      double cx[P + 3], cz[P + 3];
+#pragma unroll
+      for (int j = 0; j < 3; ++j) {
+        cx[j] = s_vx[va + (j - 1) * kVW];
+        cz[j] = s_vz[va + (j - 2) * kVW];
+      }
+#pragma unroll
+      for (int j = 0; j < P; ++j) {
+        const int v = va + j * kVW;
+        cx[j + 3] = s_vx[v + 2 * kVW];
+        cz[j + 3] = s_vz[v + kVW];
+        if (FULL || (j >= js0 && j < js1)) {
+          const double ax[3] = {s_vx[v - 1], s_vx[v + 1], s_vx[v + 2]};
+          const double az[3] = {s_vz[v - 2], s_vz[v - 1], s_vz[v + 1]};
+          loop_stress<FINITE>(ax, cx[j], cx[j + 1], cx[j + 2], cx[j + 3], az, cz[j], cz[j + 1],
+                      cz[j + 2], cz[j + 3], lm[j], la[j], dm[j], min_factor(txk, s_tz[ta + j]),
+                      dts, divx, divz, range, xx[j], zz[j], xz[j]);
+        }
+        row_fence();
+      }
+      range.report(&s_smode, elimit);
+    };
+    const int vmode = max(floor_mode, __builtin_amdgcn_readfirstlane(s_vmode[(k + 1) & 1]));
+    if (xs) {
+      if (vmode == kNormal) {
+        const NormalQuotient dx{A.dx, A.rdx, A.zhx, A.zlx}, dz{A.dz, A.rdz, A.zhz, A.zlz};
+        if (full_s)
+          stress_pass(std::true_type{}, dx, dz);
+        else
+          stress_pass(std::false_type{}, dx, dz);
+      } else if (vmode == kSmall) {
+        const SmallQuotient dx{A.dx, A.rdx, A.zhx, A.zlx}, dz{A.dz, A.rdz, A.zhz, A.zlz};
+        if (full_s)
+          stress_pass(std::true_type{}, dx, dz);
+        else
+          stress_pass(std::false_type{}, dx, dz);
+      } else {
+        stress_pass(std::false_type{}, PlainQuotient{A.dx}, PlainQuotient{A.dz});
+      }
+    }
+    {
+    const int sa0 = srow + fresh(lane);
+#pragma unroll
+    for (int j = 0; j < P; ++j) {
+      if (q0 + j >= 2 && q0 + j < SR - 2) s_xx[sa0 + (j - 2) * 64] = xx[j];
+      s_xz[sa0 + j * 64] = xz[j];
+    }
+#pragma unroll
+    for (int j = 0; j < ZR; ++j) s_zz[w * ZR * 64 - srow + sa0 + j * 64] = zz[j < 2 ? j : P - 1];
+    }
+    __syncthreads();
+
+    // ---- velocities ----
+    // the injection operands of the wave's first 64 targets, in flight during
+    // the pass
+    int inj_at = 0, inj_more = 0;
+    double inj_coef = 0.0, inj_bv = 0.0, inj_val = 0.0;
+    auto inj_fetch = [&](int base) {
+      const ConstArgs &A = *fresh(&A0);
+      const int t = base + fresh(lane);
+      if (t < ntg) {
+        const int e = gp(A.inj_first)[tg0 + t];
+        const InjEntry E = inj_entry(A, e);
+        // LDS index of the point's velocity, and the component
+        inj_at = ((vrow + (E.local >> 6) * kVW + (E.local & 63)) << 1) | E.comp;
+        inj_more = E.pad;
+        inj_coef = E.coef;
+        inj_bv = gp(A.b)[A.origin + (long long)(zs + (E.local >> 6)) * A.pitch + x0 - 2 +
+                     (E.local & 63)];
+        inj_val = inj_sample(A, E, it);
+      }
+    };
+    inj_fetch(0);
+    if (threadIdx.x == 0) s_vmode[(k + 1) & 1] = 0;  // read by all before the barrier
+    auto velocity_pass = [&](auto full, auto divx, auto divz) {
+      constexpr bool FULL = decltype(full)::value;
+      constexpr bool FINITE = !std::is_same<decltype(divx), PlainQuotient>::value;
+      const int ln = fresh(lane), va = vrow + ln, sa = srow + ln, ta = fresh(q0);
+      Range range;
+      const double xzu2 = s_xz[up2 + ln], xzu1 = s_xz[up1 + ln], xzd = s_xz[dn1 + ln];
+      const double zzu = s_zz[zup + ln], zzd0 = s_zz[zdn0 + ln], zzd1 = s_zz[zdn1 + ln];
+      auto XZ = [&](int j) { return j == -2 ? xzu2 : j == -1 ? xzu1 : j == P ? xzd : xz[j]; };
+      auto ZZ = [&](int j) { return j == -1 ? zzu : j == P ? zzd0 : j == P + 1 ? zzd1 : zz[j]; };
+#pragma unroll
+      for (int j = 0; j < P; ++j) {
+        if (FULL || (j >= jv0 && j < jv1)) {
+          const int s = sa + j * 64, x2 = s - 2 * 64;
+          double vx = s_vx[va + j * kVW], vz = s_vz[va + j * kVW];
+          const double ax[3] = {s_xx[x2 - 2], s_xx[x2 - 1], s_xx[x2 + 1]};
+          const double az[3] = {s_xz[s - 1], s_xz[s + 1], s_xz[s + 2]};
+          loop_velocity<FINITE>(ax, xx[j], az, XZ(j - 2), XZ(j - 1), XZ(j), XZ(j + 1), ZZ(j - 1), ZZ(j),
+                        ZZ(j + 1), ZZ(j + 2), bd[j], min_factor(txk, s_tz[ta + j]), divx, divz,
+                        range, vx, vz);
+          s_vx[va + j * kVW] = vx;
+          s_vz[va + j * kVW] = vz;
+        }
+        row_fence();
+      }
+      range.report(&s_vmode[k & 1], elimit);
+    };
+    const int smode = max(floor_mode, __builtin_amdgcn_readfirstlane(s_smode));
+    if (xv) {
+      if (smode == kNormal) {
+        const NormalQuotient dx{A.dx, A.rdx, A.zhx, A.zlx}, dz{A.dz, A.rdz, A.zhz, A.zlz};
+        if (full_v)
+          velocity_pass(std::true_type{}, dx, dz);
+        else
+          velocity_pass(std::false_type{}, dx, dz);
+      } else if (smode == kSmall) {
+        const SmallQuotient dx{A.dx, A.rdx, A.zhx, A.zlx}, dz{A.dz, A.rdz, A.zhz, A.zlz};
+        if (full_v)
+          velocity_pass(std::true_type{}, dx, dz);
+        else
+          velocity_pass(std::false_type{}, dx, dz);
+      } else {
+        velocity_pass(std::false_type{}, PlainQuotient{A.dx}, PlainQuotient{A.dz});
+      }
+    }
+    // injection: lane t adds the terms of target t in list order
+    for (int base = 0; base < ntg; base += 64) {
+      const ConstArgs &A = *fresh(&A0);
+      if (base) inj_fetch(base);
+      if (base + lane < ntg) {
+        double *const v = (inj_at & 1 ? s_vz : s_vx) + (inj_at >> 1);
+        double a = *v + inj_term(A, inj_at & 1, inj_coef, inj_bv, inj_val);
+        if (inj_more) {  // several terms at one point
+          int e = gp(A.inj_first)[tg0 + base + lane];
+          const int e1 = gp(A.inj_first)[tg0 + base + lane + 1];
+          for (++e; e < e1; ++e) {
+            const InjEntry F = inj_entry(A, e);
+            a += inj_term(A, F.comp, F.coef, inj_bv, inj_sample(A, F, it));
+          }
+        }
+        *v = a;
+        Range range;
+        range.any_values(a, a);
+        range.report(&s_vmode[k & 1], elimit);
+      }
+    }
+    __syncthreads();
+
+    // ---- exchange ----
+    if (threadIdx.x == 0) s_smode = 0;  // read by all before the barrier
+    if (k + 1 < A.k1) {
+      const unsigned set = (k & 1) ? 2u * RIM * 16u : 0u;
+#pragma unroll
+      for (int s = 0; s < NSEND; ++s)
+        if (send_l[s] >= 0) {
+          const int at = fresh(send_l[s]);
+          const double a = s_vx[at], b = s_vz[at];
+          const u32x4 ca = {(unsigned)__double2loint(a), tag, (unsigned)__double2hiint(a), tag};
+          const u32x4 cb = {(unsigned)__double2loint(b), tag, (unsigned)__double2hiint(b), tag};
+          __builtin_amdgcn_raw_buffer_store_b128(ca, cells, (int)(send_g + set + s * NT * 16), 0,
+                                                 kDeviceScope);
+          __builtin_amdgcn_raw_buffer_store_b128(cb, cells, (int)(send_g + set + (RIM + s * NT) * 16), 0,
+                                                 kDeviceScope);
+        }
+      begin_step(k + 1);
+      u32x4 ra[NRECV], rb[NRECV];
+      for (unsigned spin = 0;;) {
+        bool ready = true;
+#pragma unroll
+        for (int s = 0; s < NRECV; ++s)
+          if (recv_l[s] >= 0) {
+            ra[s] = __builtin_amdgcn_raw_buffer_load_b128(cells, (int)(set + recv_g[s]), 0,
+                                                          kDeviceScope);
+            rb[s] = __builtin_amdgcn_raw_buffer_load_b128(cells, (int)(set + recv_g[s] + RIM * 16u),
+                                                          0,
+                                                          kDeviceScope);
+          }
+        asm volatile("" ::: "memory");
+#pragma unroll
+        for (int s = 0; s < NRECV; ++s)
+          if (recv_l[s] >= 0)
+            ready = ready && ra[s].y == tag && ra[s].w == tag && rb[s].y == tag && rb[s].w == tag;
+        if (ready) break;
+        // all blocks run, so a neighbour answers within microseconds; a wait
+        // of some seconds means that the device is broken
+        if (++spin > (1u << 23)) {
+          s_stall = 1;
+          break;
+        }
+      }
+      Range range;
+#pragma unroll
+      for (int s = 0; s < NRECV; ++s)
+        if (recv_l[s] >= 0) {
+          const int at = fresh(recv_l[s]);
+          const double a = __hiloint2double((int)ra[s].z, (int)ra[s].x);
+          const double b = __hiloint2double((int)rb[s].z, (int)rb[s].x);
+          s_vx[at] = a;
+          s_vz[at] = b;
+          range.any_values(a, b);
+        }
+      range.report(&s_vmode[k & 1], elimit);
+      __syncthreads();
+      if (s_stall) {
+        if (threadIdx.x == 0)
+          __hip_atomic_store(l.status, (unsigned)kLoopStalled, __ATOMIC_RELAXED,
+                             __HIP_MEMORY_SCOPE_SYSTEM);
+        return;
+      }
+    } else if (A.out[0] && own_x) {
+#pragma unroll
+      for (int j = 0; j < P; ++j)
+        if (j >= jo0 && j < jo1) {
+          const long long g = A.origin + (long long)(zs + j) * A.pitch + x;
+          gp(A.out[0])[g] = s_vx[vrow + lane + j * kVW];
+          gp(A.out[1])[g] = s_vz[vrow + lane + j * kVW];
+          gp(A.out[2])[g] = xx[j];
+          gp(A.out[3])[g] = zz[j];
+          gp(A.out[4])[g] = xz[j];
+        }
+    }
+  }
+}
+
+}  // namespace
+
+namespace {
+
+// Puts a launch's arguments and its zeroed meeting words in place, in stream
+// order before it.
+__global__ void prepare_loop_kernel(LoopArgs *dst, LoopArgs a, unsigned *sync) {
+  const int n = (int)(sizeof(LoopArgs) / 8);
+  const unsigned long long *const src = (const unsigned long long *)&a;
+  for (int i = threadIdx.x; i < n; i += blockDim.x) ((unsigned long long *)dst)[i] = src[i];
+  if (threadIdx.x < 2) sync[threadIdx.x] = 0;
+}
+static_assert(sizeof(LoopArgs) % 8 == 0, "LoopArgs is copied in 8-byte words");
+
+// Blocks of a loop kernel that a compute unit holds, at most two.
+template <int KIND>
+int loop_blocks_per_cu() {
+  int n = 2;
+  for (const void *kernel :
+       {(const void *)resident_loop<KIND, false>, (const void *)resident_loop<KIND, true>}) {
+    int k = 0;
+    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&k, kernel, 64 * kLoopKinds[KIND].waves,
+                                                     0) != hipSuccess)
+      k = 0;
+    n = std::min(n, k);
+  }
+  return n;
+}
+
+constexpr int kMaxDevices = 64;
+constexpr int kXcdCus = 32;  // compute units per XCD
+
+// XCDs of a device and blocks per compute unit of the loop kernels;
+// xcds = 0 where the loops cannot run.
+struct LoopDevice {
+  int xcds = -1;
+  int per_cu[kNumLoopKinds] = {};
+};
+const LoopDevice &loop_device(int dev) {
+  static std::mutex m;
+  static LoopDevice known[kMaxDevices];
+  std::lock_guard<std::mutex> lock(m);
+  LoopDevice &d = known[dev];
+  if (d.xcds < 0) {
+    int cus = 0;
+    d.xcds = hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) == hipSuccess
+                 ? cus / kXcdCus
+                 : 0;
+    d.per_cu[0] = loop_blocks_per_cu<0>();
+    d.per_cu[1] = loop_blocks_per_cu<1>();
+    d.per_cu[2] = loop_blocks_per_cu<2>();
+    d.per_cu[3] = loop_blocks_per_cu<3>();
+    for (int n : d.per_cu)
+      if (n < 1) d.xcds = 0;
+    (void)hipGetLastError();
+  }
+  return d;
+}
+// Loop launches of one device in generations: the launches of a generation
+// fit the device together, and each of them starts after every launch of the
+// generation before, so at no time does the sum of running blocks exceed
+// what can be resident.  One object per device for the whole process (all
+// models, streams and threads launch through it); it holds a few events, no
+// device memory.
+class LoopGate {
+ public:
+  void launch(int kind, bool adjoint, const LoopLaunch &l, hipStream_t s,
+              const LoopDevice &device) {
+    std::lock_guard<std::mutex> lock(m_);
+    // in halves of a compute unit of one XCD; blocks go to the XCDs in turn
+    const int need = (l.nblocks + device.xcds - 1) / device.xcds *
+                     (device.per_cu[kind] == 2 ? 1 : 2);
+    retire(old_);
+    retire(before_);
+    retire(now_);
+    int sum = need;
+    for (const Entry &e : now_) sum += e.need;
+    if (sum > 2 * kXcdCus && !now_.empty()) {
+      // the launches of now_ themselves wait for those of before_
+      old_.insert(old_.end(), before_.begin(), before_.end());
+      before_.swap(now_);
+      now_.clear();
+    }
+    for (const Entry &e : before_) check(hipStreamWaitEvent(s, e.end, 0), "hipStreamWaitEvent");
+    hipEvent_t end;
+    if (free_.empty()) {
+      check(hipEventCreateWithFlags(&end, hipEventDisableTiming), "hipEventCreate");
+    } else {
+      end = free_.back();
+      free_.pop_back();
+    }
+    const hipError_t le = launch_loop(kind, adjoint, l, s);
+    const hipError_t re = hipEventRecord(end, s);
+    now_.push_back({end, need});
+    check(le, "resident time loop");
+    check(re, "hipEventRecord");
+  }
+
+ private:
+  struct Entry {
+    hipEvent_t end;
+    int need;
+  };
+  static void check(hipError_t e, const char *what) {
+    if (e != hipSuccess) throw RuntimeError(std::string(what) + ": " + hipGetErrorString(e));
+  }
+  void retire(std::vector<Entry> &list) {
+    size_t kept = 0;
+    for (const Entry &e : list) {
+      if (hipEventQuery(e.end) == hipSuccess) {
+        free_.push_back(e.end);
+      } else {
+        (void)hipGetLastError();  // not ready is no error of a later call
+        list[kept++] = e;
+      }
+    }
+    list.resize(kept);
+  }
+  std::mutex m_;
+  std::vector<Entry> now_, before_, old_;  // old_: events not yet reusable
+  std::vector<hipEvent_t> free_;
+};
+
+LoopGate *loop_gates() {
+  static LoopGate *const gates = new LoopGate[kMaxDevices];  // lives until the process ends
+  return gates;
+}
+
+}  // namespace
+
+hipError_t launch_loop_prepare(LoopArgs *dst, const LoopArgs &a, unsigned *sync,
+                               hipStream_t s) {
+  hipLaunchKernelGGL(prepare_loop_kernel, dim3(1), dim3(64), 0, s, dst, a, sync);
+  return hipGetLastError();
+}
+
+int loop_capacity(int kind) {
+  int dev = 0;
+  if (hipGetDevice(&dev) != hipSuccess || dev >= kMaxDevices) return 0;
+  const LoopDevice &d = loop_device(dev);
+  return d.xcds * kXcdCus * d.per_cu[kind];
+}
+
+void gated_launch_loop(int kind, bool adjoint, const LoopLaunch &l, hipStream_t s) {
+  int dev = 0;
+  if (l.nblocks > loop_capacity(kind) || hipGetDevice(&dev) != hipSuccess || dev >= kMaxDevices)
+    throw RuntimeError("resident time loop: the device cannot hold its blocks");
+  loop_gates()[dev].launch(kind, adjoint, l, s, loop_device(dev));
+}
+
+hipError_t launch_loop(int kind, bool adjoint, const LoopLaunch &l, hipStream_t s) {
+  const dim3 grid((unsigned)l.nblocks), block(64 * kLoopKinds[kind].waves);
+  auto launch = [&](auto forward, auto backward) {
+    hipLaunchKernelGGL(adjoint ? backward : forward, grid, block, 0, s, l);
+  };
+  switch (kind) {
+    case 0: launch(resident_loop<0, false>, resident_loop<0, true>); break;
+    case 1: launch(resident_loop<1, false>, resident_loop<1, true>); break;
+    case 2: launch(resident_loop<2, false>, resident_loop<2, true>); break;
+    case 3: launch(resident_loop<3, false>, resident_loop<3, true>); break;
+    default: return hipErrorInvalidValue;
+  }
+  return hipGetLastError();
+}
+
+}  // namespace psv

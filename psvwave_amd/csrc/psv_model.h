@@ -13,6 +13,7 @@
 
 #include "psv_config.h"
 #include "psv_kernels.h"
+#include "psv_loop.h"
 
 namespace psv {
 
@@ -111,6 +112,9 @@ class Model {
   }
   void reset_step_timing() { timed_ms_ = 0, timed_ = 0, launches_ = 0; }
   int64_t device_bytes() const { return device_bytes_; }
+  // As if another process held part of the device: the blocks of the next
+  // resident launches leave at once and their loops run step by step (tests).
+  void refuse_next_loops();
 
   // Pieces of a forward time loop for batched launches across models
   // (psv_batch.hip): the arguments of a launch that reads state buffer set
@@ -135,6 +139,19 @@ class Model {
   void ensure_state_sets(int n);
   static constexpr int kMaxStateSets = 8;
   void enqueue_receiver_scan(int i_shot, hipStream_t s) const;
+  // Resident loops of a batch: the tiles of a loop kernel (0: it cannot run
+  // this model) and the arguments of one loop without its exchange cells;
+  // with `snaps` the loop stores to or correlates with the one-shot store.
+  int loop_tile_columns(int kind) {
+    return ensure_loop_tables(kind) ? loop_tables_[kind].ntx : 0;
+  }
+  int loop_tile_rows_of(int kind) {
+    return ensure_loop_tables(kind) ? loop_tables_[kind].ntz : 0;
+  }
+  LoopArgs loop_args(int kind, int i_shot, bool forward) const;
+  // The same loop step by step, with the one-shot snapshot store if it is
+  // allocated and `snaps`.
+  void enqueue_store_loop(int i_shot, bool forward, bool snaps);
   int tile_count() const { return ntiles_; }
   bool lean_ok() const { return lean_ok_; }
   int step_variant() const { return variant_; }
@@ -143,6 +160,12 @@ class Model {
  private:
   void allocate();
   void build_injection_tables();
+  struct InjectionTerm {
+    int x, z, comp, src;  // grid point, 0 = vx / 1 = vz, source or receiver
+    double coef;
+  };
+  std::vector<InjectionTerm> forward_terms(int shot) const;
+  std::vector<InjectionTerm> adjoint_terms() const;
   void ensure_snapshots();
   double *dalloc(size_t n);
   void upload(double *dst, const double *src, size_t n) const;
@@ -264,6 +287,57 @@ class Model {
   void ensure_lane();
   int push_job(int lane, int kind, int shot, bool store, int dep0, int dep1);
   void pump(bool all);
+
+  // Resident time loops (psv_loop.h), the default for grids that fit the
+  // device.  Calls add jobs; the jobs of one direction that are pending
+  // together run as one launch, several shots side by side where the device
+  // holds them: forwards as they are, adjoints with the kernel terms of all
+  // but the first deferred to a buffer each and added afterwards in order.
+  // Everything is enqueued on stream_.
+  struct LoopTables {
+    int state = 0;  // 0 not built, 1 built, -1 the kernel cannot run this model
+    int ntx = 0, ntz = 0;
+    int4 *blocks = nullptr;
+    int *fwd_off = nullptr, *fwd_first = nullptr, *adj_off = nullptr, *adj_first = nullptr;
+    int *rec_off = nullptr;
+    InjEntry *fwd = nullptr, *adj = nullptr, *rec = nullptr;
+    int tiles() const { return ntx * ntz; }
+  };
+  struct LoopJob {
+    int kind, shot;
+    bool store;
+    int defer;  // buffer of the kernel terms (kJobDeferred, kJobReplay)
+    int word;   // its status word
+  };
+  bool resident_ = true;  // until a step variant is chosen
+  LoopTables loop_tables_[kNumLoopKinds];
+  std::vector<LoopJob> loop_jobs_;
+  size_t loop_launched_ = 0;  // jobs already enqueued
+  std::vector<double *> loop_defer_;
+  void *loop_cells_ = nullptr;
+  size_t loop_cells_bytes_ = 0;
+  LoopArgs *loop_args_ = nullptr;
+  int loop_args_n_ = 0;
+  unsigned *loop_sync_ = nullptr, *loop_poison_ = nullptr;
+  unsigned loop_tag_ = 1;
+  unsigned *loop_status_ = nullptr;  // host memory, one word per job
+  static constexpr int kLoopStatusWords = 1024;
+  int loop_skip_ = 0;  // forwards still to run step by step after a refused launch
+  static constexpr int kLoopSkip = 64;
+  void ensure_loop_words();
+  bool resident_path(bool dump);
+  bool ensure_loop_tables(int kind);
+  int loop_kind(int loops);
+  int loop_group(int limit);
+  void release(void *p, size_t bytes);
+  void push_loop(int kind, int shot, bool store);
+  void flush_loops();
+  void settle_loops();
+  void redo_loops(const std::vector<LoopJob> &jobs);
+  void run_resident(int kind, int i_shot, bool store);
+  void enqueue_replay(const double *d, unsigned *status);
+  void enqueue_loop_by_steps(int shot, bool forward, bool snaps, const SlotFn &slot,
+                             double *defer);
 };
 
 }  // namespace psv

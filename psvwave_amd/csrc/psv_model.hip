@@ -81,6 +81,7 @@ Model::Model(const Config &c, hipStream_t shared_stream) : cfg_(c), d_(derive(c)
 Model::Model(const Model &o) : cfg_(o.cfg_), d_(o.d_) {
   lean_ok_ = o.lean_ok_;
   variant_ = o.variant_;
+  resident_ = o.resident_;
   xcd_remap_ = o.xcd_remap_;
   allocate();
   auto cp = [&](double *dst, const double *src, long long n) {
@@ -128,6 +129,7 @@ Model::~Model() {
   destroy_stream(lane_stream_);
   for (void *p : allocations_) (void)hipFree(p);
   if (staging_) (void)hipFree(staging_);
+  if (loop_status_) (void)hipHostFree(loop_status_);
   if (owns_stream_) destroy_stream(stream_);
 }
 
@@ -213,6 +215,37 @@ void Model::allocate() {
   sync();
 }
 
+// The moment-tensor terms of a shot's sources (src/fdModel.cpp:681-751) and
+// the adjoint sources' terms (src/fdModel.cpp:951-958), in reference order.
+std::vector<Model::InjectionTerm> Model::forward_terms(int shot) const {
+  std::vector<InjectionTerm> terms;
+  for (int src : cfg_.which_source_to_fire_in_which_shot[shot]) {
+    const int x = d_.ix_src[src], z = d_.iz_src[src];
+    const double *M = &d_.moment[(size_t)src * 4];
+    const double q01 = 0.25 * M[1], q10 = 0.25 * M[2];
+    terms.push_back({x - 1, z, 0, src, -M[0]});
+    terms.push_back({x, z, 0, src, M[0]});
+    terms.push_back({x, z - 1, 1, src, -M[3]});
+    terms.push_back({x, z, 1, src, M[3]});
+    terms.push_back({x - 1, z + 1, 0, src, q01});
+    terms.push_back({x, z + 1, 0, src, q01});
+    terms.push_back({x - 1, z - 1, 0, src, -q01});
+    terms.push_back({x, z - 1, 0, src, -q01});
+    terms.push_back({x + 1, z - 1, 1, src, q10});
+    terms.push_back({x + 1, z, 1, src, q10});
+    terms.push_back({x - 1, z - 1, 1, src, -q10});
+    terms.push_back({x - 1, z, 1, src, -q10});
+  }
+  return terms;
+}
+
+std::vector<Model::InjectionTerm> Model::adjoint_terms() const {
+  std::vector<InjectionTerm> terms;
+  for (int r = 0; r < cfg_.nr; ++r)
+    for (int comp : {0, 1}) terms.push_back({d_.ix_rec[r], d_.iz_rec[r], comp, r, 0.0});
+  return terms;
+}
+
 // Injection terms in the reference's order, bucketed by owning tile (stable,
 // so terms hitting one point keep their order).  Forward: 12 moment-tensor
 // terms per source (src/fdModel.cpp:681-751); adjoint: one vx and one vz
@@ -221,10 +254,7 @@ void Model::build_injection_tables() {
   tz_ = step_tile_height(variant_);
   ntz_ = (d_.nz + tz_ - 1) / tz_;
   ntiles_ = ntx_ * ntz_;
-  struct Term {
-    int x, z, comp, src;
-    double coef;
-  };
+  using Term = InjectionTerm;
   auto bucket = [&](const std::vector<Term> &terms, std::vector<int> &off,
                     std::vector<InjEntry> &out, int base) {
     std::vector<int> count(ntiles_ + 1, 0);
@@ -250,32 +280,11 @@ void Model::build_injection_tables() {
   std::vector<int> fwd_off, off;
   std::vector<InjEntry> fwd_entries;
   for (int s = 0; s < cfg_.n_shots; ++s) {
-    std::vector<Term> terms;
-    for (int src : cfg_.which_source_to_fire_in_which_shot[s]) {
-      int x = d_.ix_src[src], z = d_.iz_src[src];
-      const double *M = &d_.moment[(size_t)src * 4];
-      double q01 = 0.25 * M[1], q10 = 0.25 * M[2];
-      terms.push_back({x - 1, z, 0, src, -M[0]});
-      terms.push_back({x, z, 0, src, M[0]});
-      terms.push_back({x, z - 1, 1, src, -M[3]});
-      terms.push_back({x, z, 1, src, M[3]});
-      terms.push_back({x - 1, z + 1, 0, src, q01});
-      terms.push_back({x, z + 1, 0, src, q01});
-      terms.push_back({x - 1, z - 1, 0, src, -q01});
-      terms.push_back({x, z - 1, 0, src, -q01});
-      terms.push_back({x + 1, z - 1, 1, src, q10});
-      terms.push_back({x + 1, z, 1, src, q10});
-      terms.push_back({x - 1, z - 1, 1, src, -q10});
-      terms.push_back({x - 1, z, 1, src, -q10});
-    }
+    const std::vector<Term> terms = forward_terms(s);
     bucket(terms, off, fwd_entries, (int)fwd_entries.size());
     fwd_off.insert(fwd_off.end(), off.begin(), off.end());
   }
-  std::vector<Term> aterms;
-  for (int r = 0; r < cfg_.nr; ++r) {
-    aterms.push_back({d_.ix_rec[r], d_.iz_rec[r], 0, r, 0.0});
-    aterms.push_back({d_.ix_rec[r], d_.iz_rec[r], 1, r, 0.0});
-  }
+  const std::vector<Term> aterms = adjoint_terms();
   std::vector<int> adj_off;
   std::vector<InjEntry> adj_entries;
   bucket(aterms, adj_off, adj_entries, 0);
@@ -315,24 +324,7 @@ void Model::build_injection_tables() {
   std::vector<int> fwd_halo_off;
   std::vector<InjEntry> fwd_halo;
   for (int s = 0; s < cfg_.n_shots; ++s) {
-    std::vector<Term> terms;
-    for (int src : cfg_.which_source_to_fire_in_which_shot[s]) {
-      int x = d_.ix_src[src], z = d_.iz_src[src];
-      const double *M = &d_.moment[(size_t)src * 4];
-      double q01 = 0.25 * M[1], q10 = 0.25 * M[2];
-      terms.push_back({x - 1, z, 0, src, -M[0]});
-      terms.push_back({x, z, 0, src, M[0]});
-      terms.push_back({x, z - 1, 1, src, -M[3]});
-      terms.push_back({x, z, 1, src, M[3]});
-      terms.push_back({x - 1, z + 1, 0, src, q01});
-      terms.push_back({x, z + 1, 0, src, q01});
-      terms.push_back({x - 1, z - 1, 0, src, -q01});
-      terms.push_back({x, z - 1, 0, src, -q01});
-      terms.push_back({x + 1, z - 1, 1, src, q10});
-      terms.push_back({x + 1, z, 1, src, q10});
-      terms.push_back({x - 1, z - 1, 1, src, -q10});
-      terms.push_back({x - 1, z, 1, src, -q10});
-    }
+    const std::vector<Term> terms = forward_terms(s);
     halo_bucket(terms, off, fwd_halo, (int)fwd_halo.size());
     fwd_halo_off.insert(fwd_halo_off.end(), off.begin(), off.end());
   }
@@ -393,6 +385,7 @@ void Model::set_step_variant(int variant, int xcd_remap) {
     throw ValueError("step variants 8-20 need dx and dz in [2^-40, 2^40] "
                      "and a taper that grows towards the interior");
   variant_ = variant;
+  resident_ = false;  // an explicit choice: that kernel, step by step
   xcd_remap_ = xcd_remap ? 1 : 0;
   clear_graphs();  // graphs hold pointers into the injection tables
   build_injection_tables();
@@ -765,6 +758,7 @@ void Model::pump(bool all) {
 // Enqueues every pending job, adds pending deferred terms and waits for the
 // device.  Errors of the enqueued work surface here.
 void Model::settle() {
+  settle_loops();
   if (jobs_.empty()) return;
   if (deferred_job_ >= 0) {
     push_job(0, kJobReplay, -1, false, deferred_job_, -1);
@@ -784,6 +778,402 @@ void Model::settle() {
     hip_check(hipStreamWaitEvent(stream_, ev_join_, 0), "hipStreamWaitEvent");
   }
   sync();
+}
+
+// ---- resident time loops ----
+
+// Whether time loops run as resident launches now: the default kernel, no
+// per-launch timing, graph or dump, and a grid that fits the device.
+bool Model::resident_path(bool dump) {
+  if (!resident_ || !lean_ok_ || graph_mode_ || timing_stride_ > 0 || dump || loop_skip_ > 0)
+    return false;
+  return loop_kind(1) >= 0;
+}
+
+void Model::release(void *p, size_t bytes) {
+  if (!p) return;
+  sync();
+  auto it = std::find(allocations_.begin(), allocations_.end(), p);
+  if (it != allocations_.end()) allocations_.erase(it);
+  hip_check(hipFree(p), "hipFree");
+  device_bytes_ -= (int64_t)bytes;
+}
+
+// The kernel for `loops` loops side by side: the smallest tiles with which
+// the device holds them all (-1: none).  Small tiles shorten a step, since
+// each wave advances fewer rows.  A single loop on more than one 28-row tile
+// per compute unit runs on 60-row tiles instead where they fit: two blocks
+// of one loop wait for their neighbours at the same time, so the second
+// hides nothing and only adds rim (1800 x 450: 9.3 against 10.1 us per step).
+int Model::loop_kind(int loops) {
+  auto fits = [&](int k, int per_cu) {
+    const long long cap = loop_capacity(k);
+    const long long room = cap == 2 * loop_capacity(kNumLoopKinds - 1) ? cap * per_cu / 2 : cap;
+    return ensure_loop_tables(k) && (long long)loops * loop_tables_[k].tiles() <= room;
+  };
+  if (d_.nx < 8 || d_.nz < 8) return -1;
+  for (int k = 0; k < kNumLoopKinds; ++k)
+    if (fits(k, k == 2 && loops == 1 ? 1 : 2)) return k;
+  return fits(2, 2) ? 2 : -1;
+}
+
+// Loops per launch when `limit` may run together: as many as the device
+// holds, in launches of even size over the shots.
+int Model::loop_group(int limit) {
+  int most = 1;
+  while (most < std::min(limit, std::max(cfg_.n_shots, 1)) && loop_kind(most + 1) >= 0) ++most;
+  const int launches = (std::max(cfg_.n_shots, 1) + most - 1) / most;
+  return (std::max(cfg_.n_shots, 1) + launches - 1) / launches;
+}
+
+// Injection targets and receivers of every tile of a loop kernel, terms of
+// one target in the reference's order.
+bool Model::ensure_loop_tables(int kind) {
+  LoopTables &t = loop_tables_[kind];
+  if (t.state) return t.state > 0;
+  t.state = -1;
+  if (loop_capacity(kind) == 0) return false;
+  const int P = kLoopKinds[kind].rows, NW = kLoopKinds[kind].waves;
+  const int ntx = t.ntx = loop_tiles_x(d_.nx), ntz = t.ntz = loop_tiles_z(d_.nz, kind);
+  const int ntiles = ntx * ntz;
+  if (ntiles > loop_capacity(kind)) return false;
+  std::vector<int> tile_x(d_.nx), tile_z(d_.nz), x0(ntx), z0(ntz);
+  for (int i = 0; i < ntx; ++i) {
+    x0[i] = (int)((long long)i * d_.nx / ntx);
+    for (int x = x0[i]; x < (int)((long long)(i + 1) * d_.nx / ntx); ++x) tile_x[x] = i;
+  }
+  for (int i = 0; i < ntz; ++i) {
+    z0[i] = (int)((long long)i * d_.nz / ntz);
+    for (int z = z0[i]; z < (int)((long long)(i + 1) * d_.nz / ntz); ++z) tile_z[z] = i;
+  }
+  // receivers, one thread of their tile each
+  std::vector<std::vector<InjEntry>> rec(ntiles);
+  for (int r = 0; r < cfg_.nr; ++r) {
+    const int tx = tile_x[d_.ix_rec[r]], tz = tile_z[d_.iz_rec[r]];
+    InjEntry e;
+    std::memset(&e, 0, sizeof(e));
+    e.local = loop_velocity_index(d_.iz_rec[r] - z0[tz], d_.ix_rec[r] - x0[tx]);
+    e.src = r;
+    rec[tz * ntx + tx].push_back(e);
+  }
+  std::vector<int> roff(1, 0);
+  std::vector<InjEntry> rent;
+  for (const auto &r : rec) {
+    if ((int)r.size() > loop_max_receivers(kind)) return false;
+    rent.insert(rent.end(), r.begin(), r.end());
+    roff.push_back((int)rent.size());
+  }
+  // targets of a term list, by strip (tile * NW + wave) and in the order of
+  // their first term
+  auto bucket = [&](const std::vector<InjectionTerm> &terms, std::vector<int> &off,
+                    std::vector<int> &first, std::vector<InjEntry> &out) {
+    std::vector<std::vector<std::vector<InjEntry>>> strips((size_t)ntiles * NW);
+    for (const InjectionTerm &m : terms) {
+      const int tx = tile_x[m.x], tz = tile_z[m.z];
+      const int q = m.z - z0[tz] + 2, lane = m.x - x0[tx] + 2;
+      auto &targets = strips[(size_t)(tz * ntx + tx) * NW + q / P];
+      InjEntry e;
+      e.local = (q % P) * 64 + lane;
+      e.comp = m.comp;
+      e.src = m.src;
+      e.pad = 0;
+      e.coef = m.coef;
+      auto it = std::find_if(targets.begin(), targets.end(), [&](const auto &g) {
+        return g[0].local == e.local && g[0].comp == e.comp;
+      });
+      if (it == targets.end()) {
+        targets.push_back({e});
+      } else {
+        (*it)[0].pad = 1;
+        it->push_back(e);
+      }
+    }
+    for (const auto &targets : strips) {
+      off.push_back((int)first.size());
+      for (const auto &g : targets) {
+        first.push_back((int)out.size());
+        out.insert(out.end(), g.begin(), g.end());
+      }
+    }
+    off.push_back((int)first.size());
+  };
+  std::vector<int> foff, ffirst, aoff, afirst;
+  std::vector<InjEntry> fent, aent;
+  for (int s = 0; s < cfg_.n_shots; ++s) bucket(forward_terms(s), foff, ffirst, fent);
+  ffirst.push_back((int)fent.size());
+  bucket(adjoint_terms(), aoff, afirst, aent);
+  afirst.push_back((int)aent.size());
+  std::vector<int4> blocks;
+  const int loops = std::min(std::max(cfg_.n_shots, 1), loop_capacity(kind) / ntiles);
+  for (int l = 0; l < loops; ++l)
+    for (int i = 0; i < ntiles; ++i) blocks.push_back(make_int4(l, i % ntx, i / ntx, 0));
+  auto put = [&](auto *&dst, const auto &v) {
+    const size_t bytes = std::max<size_t>(v.size() * sizeof(v[0]), 16);
+    void *p = nullptr;
+    hip_check(hipMalloc(&p, bytes), "hipMalloc");
+    allocations_.push_back(p);
+    device_bytes_ += (int64_t)bytes;
+    dst = (typename std::remove_reference<decltype(dst)>::type)p;
+    if (!v.empty())
+      hip_check(hipMemcpy(p, v.data(), v.size() * sizeof(v[0]), hipMemcpyHostToDevice),
+                "upload");
+  };
+  put(t.blocks, blocks);
+  put(t.fwd_off, foff);
+  put(t.fwd_first, ffirst);
+  put(t.fwd, fent);
+  put(t.adj_off, aoff);
+  put(t.adj_first, afirst);
+  put(t.adj, aent);
+  put(t.rec_off, roff);
+  put(t.rec, rent);
+  t.state = 1;
+  return true;
+}
+
+// Arguments of a whole loop of one shot from the zero state, without its
+// snapshots and exchange cells.
+LoopArgs Model::loop_args(int kind, int i_shot, bool forward) const {
+  const LoopTables &t = loop_tables_[kind];
+  LoopArgs a;
+  std::memset(&a, 0, sizeof(a));
+  const StepArgs b = forward ? forward_args(i_shot) : adjoint_args(i_shot);
+  a.nx = b.nx, a.nz = b.nz, a.pitch = b.pitch, a.origin = b.origin;
+  a.ntx = t.ntx, a.ntz = t.ntz;
+  a.lm = b.lm, a.mu = b.mu, a.b = b.b;
+  a.taper_x = b.taper_x, a.taper_z = b.taper_z;
+  a.dts = b.dts, a.dt = b.dt, a.dx = b.dx, a.dz = b.dz, a.rdx = b.rdx, a.rdz = b.rdz;
+  a.zhx = b.zhx, a.zlx = b.zlx, a.zhz = b.zhz, a.zlz = b.zlz;
+  a.dxdz = b.dxdz, a.d4x = b.d4x, a.d4z = b.d4z;
+  a.nt = b.nt, a.k0 = 0, a.k1 = b.nt;
+  a.si = cfg_.snapshot_interval;
+  a.slot_every = 1;
+  a.slot_stride = ngrid_;
+  a.rho_k = b.rho_k, a.lam_k = b.lam_k, a.mu_k = b.mu_k;
+  a.kx0 = b.kx0, a.kx1 = b.kx1, a.kz0 = b.kz0, a.kz1 = b.kz1;
+  a.wcorr = b.wcorr;
+  if (forward) {
+    a.inj_off = t.fwd_off + (size_t)i_shot * (t.tiles() * kLoopKinds[kind].waves + 1);
+    a.inj_first = t.fwd_first;
+    a.inj = t.fwd;
+    a.rec_off = t.rec_off;
+    a.rec = t.rec;
+  } else {
+    a.inj_off = t.adj_off;
+    a.inj_first = t.adj_first;
+    a.inj = t.adj;
+  }
+  a.stf = b.stf, a.adj_x = b.adj_x, a.adj_z = b.adj_z;
+  a.rtf_x = b.rtf_x, a.rtf_z = b.rtf_z;
+  return a;
+}
+
+// Adds a job; launches the pending ones before a job they cannot share a
+// launch with, and once there are as many as run together.
+void Model::push_loop(int kind, int shot, bool store) {
+  // the second stream, which checkpointed adjoints use beside this one, opens
+  // with the first call as it does for loops by steps
+  if (!lane_stream_) create_stream(&lane_stream_);
+  const bool fwd = kind == kJobForward;
+  bool apart = loop_jobs_.size() + 16 > (size_t)kLoopStatusWords;
+  for (size_t i = loop_launched_; i < loop_jobs_.size(); ++i)
+    apart = apart || (loop_jobs_[i].kind == kJobForward) != fwd ||
+            (fwd && loop_jobs_[i].shot == shot);
+  if (loop_jobs_.size() + 16 > (size_t)kLoopStatusWords)
+    settle_loops();
+  else if (apart)
+    flush_loops();
+  const int pending = (int)(loop_jobs_.size() - loop_launched_);
+  loop_jobs_.push_back({fwd ? kJobForward : pending ? kJobDeferred : kJobAdjoint, shot, store,
+                        pending - 1, 0});
+  int together = std::min(16, loop_group(16));
+  if (!fwd && together > 1) {
+    // a buffer of kernel terms for all but the first: as many as the device
+    // has room for, keeping to a tenth of its memory
+    const long long n = (long long)d_.snapshots * 3 * ngrid_;
+    size_t free_b = 0, total_b = 0;
+    while ((int)loop_defer_.size() < together - 1 &&
+           hipMemGetInfo(&free_b, &total_b) == hipSuccess &&
+           (double)n * sizeof(double) + (double)(2ull << 30) <= (double)free_b &&
+           (double)n * sizeof(double) * (double)(loop_defer_.size() + 1) <= 0.1 * (double)total_b)
+      loop_defer_.push_back(dalloc((size_t)n));
+    together = loop_group((int)loop_defer_.size() + 1);
+  }
+  if (pending + 1 >= together) flush_loops();
+}
+
+void Model::ensure_loop_words() {
+  if (loop_sync_) return;
+  loop_poison_ = (unsigned *)dalloc(1);
+  hip_check(hipHostMalloc((void **)&loop_status_, kLoopStatusWords * sizeof(unsigned),
+                          hipHostMallocDefault),
+            "hipHostMalloc");
+  std::memset(loop_status_, 0, kLoopStatusWords * sizeof(unsigned));
+  loop_sync_ = (unsigned *)dalloc(1);
+}
+
+void Model::refuse_next_loops() {
+  settle();
+  ensure_loop_words();
+  double word = 0.0;
+  const unsigned one = 1;
+  std::memcpy(&word, &one, sizeof(one));
+  upload((double *)loop_poison_, &word, 1);
+}
+
+// Launches the pending jobs side by side, then adds deferred kernel terms.
+void Model::flush_loops() {
+  const int first = (int)loop_launched_, n = (int)loop_jobs_.size() - first;
+  if (n == 0) return;
+  loop_launched_ = loop_jobs_.size();
+  const bool fwd = loop_jobs_[first].kind == kJobForward;
+  const int kind = loop_kind(n);
+  const LoopTables &t = loop_tables_[kind];
+  const size_t cells = loop_cells_bytes(kind, t.tiles());
+  ensure_loop_words();
+  if (loop_args_n_ < n) {
+    release(loop_args_, loop_args_n_ * sizeof(LoopArgs));
+    loop_args_ = (LoopArgs *)dalloc(n * sizeof(LoopArgs) / 8);
+    loop_args_n_ = n;
+  }
+  if (loop_cells_bytes_ < cells * n) {  // new cells are zero: no tag matches
+    release(loop_cells_, loop_cells_bytes_);
+    loop_cells_ = dalloc(cells * n / 8);
+    loop_cells_bytes_ = cells * n;
+  } else if (loop_tag_ + (unsigned)cfg_.nt < loop_tag_) {  // the tags start over
+    hip_check(launch_fill((double *)loop_cells_, (long long)(loop_cells_bytes_ / 8), 0.0, stream_),
+              "clear cells");
+    loop_tag_ = 1;
+  }
+  for (int i = 0; i < n; ++i) {
+    LoopJob &j = loop_jobs_[first + i];
+    j.word = first;
+    LoopArgs a = loop_args(kind, j.shot, fwd);
+    a.slot_every = ckpt_every_;
+    if ((j.store || !fwd) && snap_[0])
+      for (int f = 0; f < 5; ++f)
+        a.snap[f] = snap_[f] + (long long)j.shot * stored_snapshots() * ngrid_;
+    if (j.kind == kJobDeferred) {
+      a.rho_k = loop_defer_[j.defer];
+      a.lam_k = a.rho_k + ngrid_;
+      a.mu_k = a.rho_k + 2 * ngrid_;
+      a.defer_stride = 3 * ngrid_;
+    }
+    a.cells = (char *)loop_cells_ + cells * i;
+    a.cells_bytes = (unsigned)cells;
+    hip_check(launch_loop_prepare(loop_args_ + i, a, loop_sync_, stream_), "prepare loop");
+  }
+  LoopLaunch l;
+  l.loops = loop_args_;
+  l.blocks = t.blocks;
+  l.nblocks = n * t.tiles();
+  l.tag0 = loop_tag_;
+  l.sync = loop_sync_;
+  l.poison = loop_poison_;
+  l.status = loop_status_ + first;
+  gated_launch_loop(kind, !fwd, l, stream_);
+  loop_tag_ += (unsigned)cfg_.nt;
+  launches_ += (int64_t)n * cfg_.nt;
+  for (int i = 1; i < n && !fwd; ++i) {
+    const LoopJob r = {kJobReplay, -1, false, loop_jobs_[first + i].defer,
+                       (int)loop_jobs_.size()};
+    loop_jobs_.push_back(r);
+    ++loop_launched_;
+    enqueue_replay(loop_defer_[r.defer], loop_status_ + r.word);
+  }
+}
+
+// The kernel terms deferred to d, in their adjoint's order.
+void Model::enqueue_replay(const double *d, unsigned *status) {
+  hip_check(launch_replay_correlation(
+                rho_l_, lam_k_, mu_k_, d, d_.snapshots, ngrid_, d_.nx,
+                cfg_.np_boundary + cfg_.nx_inner_boundary,
+                cfg_.np_boundary + cfg_.nx_inner - cfg_.nx_inner_boundary,
+                cfg_.np_boundary + cfg_.nz_inner_boundary,
+                cfg_.np_boundary + cfg_.nz_inner - cfg_.nz_inner_boundary, stream_,
+                status ? loop_poison_ : nullptr, status),
+            "replay correlation");
+}
+
+void Model::settle_loops() {
+  if (loop_jobs_.empty()) return;
+  flush_loops();
+  sync();
+  std::vector<LoopJob> ended;
+  ended.swap(loop_jobs_);
+  loop_launched_ = 0;
+  redo_loops(ended);
+}
+
+// After the device has finished the jobs: runs those that did not take place
+// step by step, in order.  A resident loop does not take place when its
+// blocks were not resident together in time (another process holds part of
+// the device); it then sets the poison word, at which every job after it
+// does nothing either.
+// The next jobs then run step by step from the start, since whoever holds
+// the device is likely still there.
+void Model::redo_loops(const std::vector<LoopJob> &jobs) {
+  const std::vector<unsigned> ran(loop_status_, loop_status_ + jobs.size());
+  std::memset(loop_status_, 0, jobs.size() * sizeof(unsigned));
+  bool missing = false;
+  for (const LoopJob &j : jobs) {
+    if (ran[j.word] == kLoopStalled)
+      throw RuntimeError("a resident time loop made no progress");
+    missing = missing || ran[j.word] == kLoopNotRun;
+  }
+  if (!missing) {
+    loop_skip_ = 0;
+    return;
+  }
+  loop_skip_ = kLoopSkip;
+  hip_check(launch_fill((double *)loop_poison_, 1, 0.0, stream_), "clear poison");
+  for (const LoopJob &j : jobs) {
+    if (ran[j.word] != kLoopNotRun) continue;
+    if (j.kind == kJobReplay) {
+      enqueue_replay(loop_defer_[j.defer], nullptr);
+      continue;
+    }
+    const bool fwd = j.kind == kJobForward;
+    const int shot = j.shot;
+    enqueue_loop_by_steps(shot, fwd, j.store || !fwd,
+                          [this, shot](int it, double **dst) {
+                            return stored_slot(shot, it, dst);
+                          },
+                          j.kind == kJobDeferred ? loop_defer_[j.defer] : nullptr);
+  }
+  sync();
+}
+
+void Model::enqueue_loop_by_steps(int shot, bool forward, bool snaps, const SlotFn &slot,
+                                  double *defer) {
+  StepArgs a = forward ? forward_args(shot) : adjoint_args(shot);
+  a.rec_increments = 0;
+  a.rec_off = adj_off_;
+  a.rec_entries = adj_entries_;
+  enqueue_zero_state(stream_);
+  enqueue_range(a, state_, 0, forward, 0, cfg_.nt, snaps, slot, nullptr, false, stream_, defer);
+}
+
+void Model::enqueue_store_loop(int i_shot, bool forward, bool snaps) {
+  enqueue_loop_by_steps(i_shot, forward, snaps, [this](int it, double **dst) {
+    for (int f = 0; f < 5; ++f)
+      dst[f] = shot_snap_[f] + (long long)(it / cfg_.snapshot_interval) * ngrid_;
+    return true;
+  }, nullptr);
+}
+
+// One loop, waited for; with loop timing, events bracket it.
+void Model::run_resident(int kind, int i_shot, bool store) {
+  settle();
+  auto enqueue = [&] {
+    push_loop(kind, i_shot, store);
+    flush_loops();
+  };
+  if (timing_stride_ < 0)
+    timed_loop(enqueue);
+  else
+    enqueue();
+  settle();
 }
 
 // Adjoint with checkpointing: segments of ckpt_every_ snapshot intervals
@@ -1076,9 +1466,15 @@ void Model::enqueue_receiver_scan(int i_shot, hipStream_t s) const {
 void Model::forward(int i_shot, bool store_fields, bool verbose,
                     bool output_wavefields) {
   check_shot(i_shot);
+  if (loop_skip_ > 0) --loop_skip_;
   if (store_fields && cfg_.nt % cfg_.snapshot_interval != 0)
     throw ValueError("Snapshot interval and size of accumulator don't match!"
                      " (nt must be a multiple of snapshot_interval)");
+  if (resident_path(output_wavefields) && async_ && !verbose && timing_stride_ == 0) {
+    if (store_fields) ensure_snapshots();
+    push_loop(kJobForward, i_shot, store_fields);
+    return;
+  }
   if (async_path(verbose, output_wavefields)) {
     ensure_lane();
     // a pending adjoint may still read this shot's snapshots and a pending
@@ -1097,9 +1493,14 @@ void Model::forward(int i_shot, bool store_fields, bool verbose,
   }
   settle();
   if (store_fields) ensure_snapshots();
-  StepArgs a = forward_args(i_shot);
+  const bool resident = resident_path(output_wavefields);
   auto t0 = std::chrono::steady_clock::now();
-  run_steps(a, i_shot, true, store_fields, output_wavefields);
+  if (resident) {
+    run_resident(kJobForward, i_shot, store_fields);
+  } else {
+    StepArgs a = forward_args(i_shot);
+    run_steps(a, i_shot, true, store_fields, output_wavefields);
+  }
   if (verbose) {
     double s = std::chrono::duration<double>(std::chrono::steady_clock::now() - t0)
                    .count();
@@ -1116,6 +1517,10 @@ void Model::adjoint(int i_shot, bool verbose) {
   if (!snap_[0])
     throw ValueError("adjoint_simulate needs stored forward wavefields; run "
                      "forward_simulate with store_fields=True first");
+  if (resident_path(false) && async_ && !verbose && timing_stride_ == 0 && ckpt_every_ == 1) {
+    push_loop(kJobAdjoint, i_shot, false);
+    return;
+  }
   if (async_path(verbose, false)) {
     ensure_lane();
     if (!defer_ && !no_defer_room_) {
@@ -1158,6 +1563,8 @@ void Model::adjoint(int i_shot, bool verbose) {
                 "hipEventElapsedTime");
       timed_ms_ += ms;
     }
+  } else if (resident_path(false)) {
+    run_resident(kJobAdjoint, i_shot, false);
   } else {
     run_steps(a, i_shot, false, false, false);
   }
@@ -1279,7 +1686,7 @@ void Model::run_model(bool verbose, bool simulate_adjoint) {
     return;
   }
   if (!verbose && (ckpt_every_ == 1 || !simulate_adjoint) && timing_stride_ <= 0 &&
-      cfg_.n_shots > 1) {
+      cfg_.n_shots > 1 && !resident_path(false)) {
     run_model_two_lanes(simulate_adjoint);
     return;
   }
