@@ -110,5 +110,7 @@ int loop_capacity(int kind);
 // Launches through the gate of the current device: the blocks of all loop
 // launches that may run at the same time fit the device together.
 void gated_launch_loop(int kind, bool adjoint, const LoopLaunch &l, hipStream_t s);
+// Before a synchronised stream is destroyed: the gate drops its events.
+void loop_gate_forget(hipStream_t s);
 
 }  // namespace psv

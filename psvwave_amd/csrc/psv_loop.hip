@@ -37,6 +37,7 @@
 #include "psv_loop.h"
 
 #include <algorithm>
+#include <map>
 #include <mutex>
 #include <string>
 #include <type_traits>
@@ -828,7 +829,8 @@ const LoopDevice &loop_device(int dev) {
 // generation before, so at no time does the sum of running blocks exceed
 // what can be resident.  One object per device for the whole process (all
 // models, streams and threads launch through it); it holds a few events, no
-// device memory.
+// device memory.  An event belongs to the stream it is recorded on and goes
+// when that stream goes (forget), under the same lock as every use of it.
 class LoopGate {
  public:
   void launch(int kind, bool adjoint, const LoopLaunch &l, hipStream_t s,
@@ -848,24 +850,45 @@ class LoopGate {
       before_.swap(now_);
       now_.clear();
     }
-    for (const Entry &e : before_) check(hipStreamWaitEvent(s, e.end, 0), "hipStreamWaitEvent");
+    for (const Entry &e : before_)
+      if (e.stream != s) check(hipStreamWaitEvent(s, e.end, 0), "hipStreamWaitEvent");
     hipEvent_t end;
-    if (free_.empty()) {
+    std::vector<hipEvent_t> &spare = spare_[s];
+    if (spare.empty()) {
       check(hipEventCreateWithFlags(&end, hipEventDisableTiming), "hipEventCreate");
     } else {
-      end = free_.back();
-      free_.pop_back();
+      end = spare.back();
+      spare.pop_back();
     }
     const hipError_t le = launch_loop(kind, adjoint, l, s);
     const hipError_t re = hipEventRecord(end, s);
-    now_.push_back({end, need});
+    now_.push_back({end, s, need});
     check(le, "resident time loop");
     check(re, "hipEventRecord");
+  }
+  // Stream s has been synchronised and is about to be destroyed.
+  void forget(hipStream_t s) {
+    std::lock_guard<std::mutex> lock(m_);
+    for (std::vector<Entry> *list : {&now_, &before_, &old_}) {
+      size_t kept = 0;
+      for (const Entry &e : *list) {
+        if (e.stream == s)
+          (void)hipEventDestroy(e.end);
+        else
+          (*list)[kept++] = e;
+      }
+      list->resize(kept);
+    }
+    auto it = spare_.find(s);
+    if (it == spare_.end()) return;
+    for (hipEvent_t e : it->second) (void)hipEventDestroy(e);
+    spare_.erase(it);
   }
 
  private:
   struct Entry {
     hipEvent_t end;
+    hipStream_t stream;
     int need;
   };
   static void check(hipError_t e, const char *what) {
@@ -875,7 +898,7 @@ class LoopGate {
     size_t kept = 0;
     for (const Entry &e : list) {
       if (hipEventQuery(e.end) == hipSuccess) {
-        free_.push_back(e.end);
+        spare_[e.stream].push_back(e.end);
       } else {
         (void)hipGetLastError();  // not ready is no error of a later call
         list[kept++] = e;
@@ -885,7 +908,7 @@ class LoopGate {
   }
   std::mutex m_;
   std::vector<Entry> now_, before_, old_;  // old_: events not yet reusable
-  std::vector<hipEvent_t> free_;
+  std::map<hipStream_t, std::vector<hipEvent_t>> spare_;
 };
 
 LoopGate *loop_gates() {
@@ -906,6 +929,10 @@ int loop_capacity(int kind) {
   if (hipGetDevice(&dev) != hipSuccess || dev >= kMaxDevices) return 0;
   const LoopDevice &d = loop_device(dev);
   return d.xcds * kXcdCus * d.per_cu[kind];
+}
+
+void loop_gate_forget(hipStream_t s) {
+  for (int i = 0; i < kMaxDevices; ++i) loop_gates()[i].forget(s);
 }
 
 void gated_launch_loop(int kind, bool adjoint, const LoopLaunch &l, hipStream_t s) {

@@ -46,6 +46,8 @@ void create_stream(hipStream_t *s) {
 
 void destroy_stream(hipStream_t s) {
   if (!s) return;
+  (void)hipStreamSynchronize(s);
+  loop_gate_forget(s);
   (void)hipStreamDestroy(s);
   --g_live_streams;
 }
