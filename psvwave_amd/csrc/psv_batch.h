@@ -3,7 +3,9 @@
 // models of uneven size).
 #pragma once
 
+#include <map>
 #include <memory>
+#include <utility>
 #include <vector>
 
 #include "psv_model.h"
@@ -80,6 +82,35 @@ class Batch {
   long long zero_max_ = 0;
   void clear_graphs();
   void clear_gradient_tables();
+  // Resident loops (psv_loop.h), the default when every member fits the
+  // device: the loops of a call packed into as few launches as hold them.
+  struct LoopRef {
+    int member, shot;
+    bool forward, snaps;
+  };
+  struct LoopLaunches {
+    int kind = -1;
+    bool forward = true;
+    std::vector<LoopRef> loops;                // in launch order
+    std::vector<std::pair<int, int>> launches; // first loop, blocks
+    std::vector<int> first_block;              // of each launch
+    LoopArgs *args = nullptr;
+    int4 *blocks = nullptr;
+  };
+  bool resident_available();
+  LoopLaunches *loop_launches(int which, int i_shot, int steps);
+  void run_loops(LoopLaunches &p, int steps);
+  void clear_loops();
+  void end_timing();
+  bool resident_ = true;  // until a step variant is chosen
+  int loop_skip_ = 0;     // calls still to run step by step after a refused launch
+  int loop_kind_ = -2;    // -2 not chosen, -1 some member does not fit
+  std::map<int, LoopLaunches> loops_;
+  void *loop_cells_ = nullptr;
+  unsigned loop_tag_ = 1;
+  unsigned *loop_sync_ = nullptr, *loop_poison_ = nullptr;
+  unsigned *loop_status_ = nullptr;  // host memory, one word per launch
+  int loop_words_ = 0;
   void enqueue_gradient_loop(int i_shot, bool forward);
 
   std::vector<std::unique_ptr<Model>> models_;

@@ -57,6 +57,11 @@ Batch::~Batch() {
     if (p) (void)hipFree(p);
   if (zero_lens_) (void)hipFree(zero_lens_);
   clear_gradient_tables();
+  clear_loops();
+  if (loop_cells_) (void)hipFree(loop_cells_);
+  if (loop_sync_) (void)hipFree(loop_sync_);
+  if (loop_poison_) (void)hipFree(loop_poison_);
+  if (loop_status_) (void)hipHostFree(loop_status_);
   for (auto e : ev_)
     if (e) (void)hipEventDestroy(e);
   models_.clear();  // the members run on stream_
@@ -108,6 +113,7 @@ void Batch::set_variant(int variant, int xcd_remap) {
       if (!m->lean_ok())
         throw ValueError("a member of the batch cannot use the lean step variants");
   variant_ = variant;
+  resident_ = false;  // an explicit choice: that kernel, step by step
   xcd_remap_ = xcd_remap ? 1 : 0;
   if (variant != kLeanTz8) persistent_ = false;
   clear_graphs();
@@ -206,9 +212,204 @@ void Batch::enqueue_loop(int i_shot, int nsteps) {
     for (auto &m : models_) m->enqueue_receiver_scan(i_shot, stream_);
 }
 
+// ---- resident loops ----
+
+void Batch::clear_loops() {
+  for (auto &kv : loops_) {
+    if (kv.second.args) (void)hipFree(kv.second.args);
+    if (kv.second.blocks) (void)hipFree(kv.second.blocks);
+  }
+  loops_.clear();
+}
+
+// The kernel of all loops: the smallest tiles with which every loop of
+// forward_all fits one launch, since a step of small tiles is shorter; a
+// batch that needs several launches runs on 28-row tiles, two blocks per
+// compute unit: the blocks of a unit mostly belong to different loops and
+// hide each other's exchange.
+bool Batch::resident_available() {
+  if (!resident_ || graph_mode_ || persistent_) return false;
+  if (loop_skip_ > 0) {
+    --loop_skip_;
+    return false;
+  }
+  if (loop_kind_ == -2) {
+    loop_kind_ = -1;
+    bool able = true;
+    for (auto &m : models_) able = able && m->lean_ok() && m->derived().nx >= 8 && m->derived().nz >= 8;
+    // tiles of all loops and of the largest member
+    auto tiles = [&](int kind, long long *most) {
+      long long sum = 0;
+      *most = 0;
+      for (auto &m : models_) {
+        const long long t =
+            (long long)loop_tiles_x(m->derived().nx) * loop_tiles_z(m->derived().nz, kind);
+        sum += t * n_shots_;
+        *most = std::max(*most, t);
+      }
+      return sum;
+    };
+    auto usable = [&](int kind) {  // the tables of every member
+      for (auto &m : models_)
+        if (m->loop_tile_columns(kind) == 0) return false;
+      return true;
+    };
+    long long most = 0;
+    for (int k = 0; able && k < 3 && loop_kind_ < 0; ++k)
+      if (tiles(k, &most) <= loop_capacity(k) && usable(k)) loop_kind_ = k;
+    for (int k : {2, 3})
+      if (able && loop_kind_ < 0 && tiles(k, &most) > 0 && most <= loop_capacity(k) && usable(k))
+        loop_kind_ = k;
+  }
+  return loop_kind_ >= 0;
+}
+
+// The launches of a call, built on first use.  which: 0 forward_all, 1
+// forward of i_shot, 2 / 3 forward / adjoint of i_shot with the one-shot
+// snapshot stores, 4 the first `steps` steps of forward_all.
+Batch::LoopLaunches *Batch::loop_launches(int which, int i_shot, int steps) {
+  LoopLaunches &p = loops_[which + 8 * i_shot];
+  if (p.kind >= 0 && which != 4) return &p;
+  const int kind = p.kind = loop_kind_;
+  p.forward = which != 3;
+  std::vector<LoopRef> refs;
+  for (int m = 0; m < size(); ++m)
+    for (int s = 0; s < n_shots_; ++s)
+      if (which == 0 || which == 4 || s == i_shot)
+        refs.push_back({m, s, p.forward, which == 2 || which == 3});
+  auto tiles = [&](const LoopRef &r) {
+    return models_[r.member]->loop_tile_columns(kind) *
+           models_[r.member]->loop_tile_rows_of(kind);
+  };
+  // first fit, the largest loops first
+  std::stable_sort(refs.begin(), refs.end(),
+                   [&](const LoopRef &a, const LoopRef &b) { return tiles(a) > tiles(b); });
+  std::vector<std::vector<LoopRef>> bins;
+  std::vector<int> room;
+  for (const LoopRef &r : refs) {
+    size_t b = 0;
+    while (b < bins.size() && room[b] < tiles(r)) ++b;
+    if (b == bins.size()) {
+      bins.push_back({});
+      room.push_back(loop_capacity(kind));
+    }
+    bins[b].push_back(r);
+    room[b] -= tiles(r);
+  }
+  p.loops.clear(), p.launches.clear(), p.first_block.clear();
+  const int cap = loop_capacity(kind);
+  const size_t cell_bytes = loop_cells_bytes(kind, 1);
+  if (!loop_cells_) {
+    hip_check(hipMalloc(&loop_cells_, cell_bytes * cap), "hipMalloc");
+    hip_check(launch_fill((double *)loop_cells_, (long long)(cell_bytes * cap / 8), 0.0, stream_),
+              "clear cells");
+  }
+  std::vector<LoopArgs> args;
+  std::vector<int4> blocks;
+  for (const auto &bin : bins) {
+    const int first = (int)p.loops.size(), block0 = (int)blocks.size();
+    for (size_t i = 0; i < bin.size(); ++i) {
+      const LoopRef &r = bin[i];
+      Model &m = *models_[r.member];
+      LoopArgs a = m.loop_args(kind, r.shot, r.forward);
+      a.cells = (char *)loop_cells_ + cell_bytes * (blocks.size() - block0);
+      a.cells_bytes = (unsigned)(cell_bytes * tiles(r));
+      if (r.snaps) {
+        double *const *store = m.shot_snapshot_store();
+        for (int f = 0; f < 5; ++f) a.snap[f] = store[f];
+      }
+      if (which == 4) a.k1 = steps;
+      const int ntx = m.loop_tile_columns(kind);
+      for (int t = 0; t < tiles(r); ++t)
+        blocks.push_back(make_int4((int)i, t % ntx, t / ntx, 0));
+      args.push_back(a);
+      p.loops.push_back(r);
+    }
+    p.launches.emplace_back(first, (int)blocks.size() - block0);
+    p.first_block.push_back(block0);
+  }
+  auto put = [&](auto *&dst, const auto &v) {
+    hip_check(hipStreamSynchronize(stream_), "sync");
+    if (dst) hip_check(hipFree(dst), "hipFree");
+    dst = nullptr;
+    hip_check(hipMalloc((void **)&dst, v.size() * sizeof(v[0])), "hipMalloc");
+    hip_check(hipMemcpy(dst, v.data(), v.size() * sizeof(v[0]), hipMemcpyHostToDevice), "upload");
+  };
+  put(p.args, args);
+  put(p.blocks, blocks);
+  const int n = (int)p.launches.size();
+  if (n > loop_words_) {
+    if (loop_sync_) hip_check(hipFree(loop_sync_), "hipFree");
+    if (loop_status_) hip_check(hipHostFree(loop_status_), "hipHostFree");
+    loop_sync_ = loop_status_ = nullptr;
+    loop_words_ = 0;
+    hip_check(hipMalloc((void **)&loop_sync_, (size_t)n * 8), "hipMalloc");
+    hip_check(hipHostMalloc((void **)&loop_status_, n * sizeof(unsigned), hipHostMallocDefault),
+              "hipHostMalloc");
+    loop_words_ = n;
+  }
+  if (!loop_poison_) {
+    hip_check(hipMalloc((void **)&loop_poison_, 8), "hipMalloc");
+    hip_check(launch_fill((double *)loop_poison_, 1, 0.0, stream_), "clear poison");
+  }
+  return &p;
+}
+
+// Runs the launches of a call (`steps` time steps each) and waits for them;
+// loops whose launch was refused (psv_loop.h) run step by step.
+void Batch::run_loops(LoopLaunches &p, int steps) {
+  const int n = (int)p.launches.size();
+  for (int i = 0; i < n; ++i) loop_status_[i] = kLoopNotRun;
+  hip_check(launch_fill((double *)loop_sync_, n, 0.0, stream_), "clear loop words");
+  for (int i = 0; i < n; ++i) {
+    if (loop_tag_ + (unsigned)steps < loop_tag_) {  // the tags start over
+      hip_check(launch_fill((double *)loop_cells_,
+                            (long long)(loop_cells_bytes(p.kind, loop_capacity(p.kind)) / 8), 0.0,
+                            stream_),
+                "clear cells");
+      loop_tag_ = 1;
+    }
+    LoopLaunch l;
+    l.loops = p.args + p.launches[i].first;
+    l.blocks = p.blocks + p.first_block[i];
+    l.nblocks = p.launches[i].second;
+    l.tag0 = loop_tag_;
+    l.sync = loop_sync_ + 2 * i;
+    l.poison = loop_poison_;
+    l.status = loop_status_ + i;
+    gated_launch_loop(p.kind, !p.forward, l, stream_);
+    loop_tag_ += (unsigned)steps;
+  }
+  hip_check(hipStreamSynchronize(stream_), "hipStreamSynchronize");
+  bool missing = false;
+  for (int i = 0; i < n; ++i) {
+    if (loop_status_[i] == kLoopStalled)
+      throw RuntimeError("a resident time loop made no progress");
+    missing = missing || loop_status_[i] == kLoopNotRun;
+  }
+  if (!missing) return;
+  loop_skip_ = 64;
+  hip_check(launch_fill((double *)loop_poison_, 1, 0.0, stream_), "clear poison");
+  for (int i = 0; i < n; ++i) {
+    if (loop_status_[i] != kLoopNotRun) continue;
+    const int last = i + 1 < n ? p.launches[i + 1].first : (int)p.loops.size();
+    for (int k = p.launches[i].first; k < last; ++k)
+      models_[p.loops[k].member]->enqueue_store_loop(p.loops[k].shot, p.loops[k].forward,
+                                                     p.loops[k].snaps);
+  }
+  hip_check(hipStreamSynchronize(stream_), "hipStreamSynchronize");
+}
+
 void Batch::forward(int i_shot) {
   if (i_shot < 0 || i_shot >= n_shots_)
     throw ValueError("i_shot is outside [0, n_shots)");
+  if (resident_available()) {
+    LoopLaunches *p = loop_launches(1, i_shot, nt_);
+    hip_check(hipEventRecord(ev_[0], stream_), "hipEventRecord");
+    run_loops(*p, nt_);
+    end_timing();
+    return;
+  }
   hip_check(hipEventRecord(ev_[0], stream_), "hipEventRecord");
   if (graph_mode_) {
     if (graphs_.size() != (size_t)n_shots_) graphs_.assign(n_shots_, nullptr);
@@ -284,7 +485,23 @@ void Batch::enqueue_lockstep_loop(int nsteps) {
   }
 }
 
+// The end of a timed region whose work has been enqueued on stream_.
+void Batch::end_timing() {
+  hip_check(hipEventRecord(ev_[1], stream_), "hipEventRecord");
+  hip_check(hipStreamSynchronize(stream_), "hipStreamSynchronize");
+  float ms = 0.f;
+  hip_check(hipEventElapsedTime(&ms, ev_[0], ev_[1]), "hipEventElapsedTime");
+  loop_ms_ += ms;
+}
+
 void Batch::forward_all() {
+  if (resident_available()) {
+    LoopLaunches *p = loop_launches(0, 0, nt_);
+    hip_check(hipEventRecord(ev_[0], stream_), "hipEventRecord");
+    run_loops(*p, nt_);
+    end_timing();
+    return;
+  }
   if (!lockstep_available()) {
     for (int s = 0; s < n_shots_; ++s) forward(s);
     return;
@@ -352,7 +569,8 @@ void Batch::gradients() {
   if (nt_ % si_ != 0)
     throw ValueError("Snapshot interval and size of accumulator don't match! "
                      "(nt must be a multiple of snapshot_interval)");
-  if (!gfwd_) {
+  const bool resident = resident_available();
+  if (!resident && !gfwd_) {
     std::vector<StepArgs> f, a;
     for (auto &m : models_) {
       double *const *store = m->shot_snapshot_store();
@@ -375,10 +593,16 @@ void Batch::gradients() {
   for (int s = 0; s < n_shots_; ++s) {
     // forward s, its adjoint sources (each member's own stream), adjoint s:
     // the kernels accumulate shot by shot, as in the reference's order
-    enqueue_gradient_loop(s, true);
+    if (resident)
+      run_loops(*loop_launches(2, s, nt_), nt_);
+    else
+      enqueue_gradient_loop(s, true);
     hip_check(hipStreamSynchronize(stream_), "hipStreamSynchronize");
     for (auto &m : models_) m->calculate_l2_adjoint_sources();
-    enqueue_gradient_loop(s, false);
+    if (resident)
+      run_loops(*loop_launches(3, s, nt_), nt_);
+    else
+      enqueue_gradient_loop(s, false);
   }
   hip_check(hipEventRecord(ev_[1], stream_), "hipEventRecord");
   hip_check(hipStreamSynchronize(stream_), "hipStreamSynchronize");
@@ -438,6 +662,22 @@ double Batch::autotune(int steps, int *best, double *ms_per_variant) {
   }
   set_variant(best_v, keep_remap);
   if (best) *best = best_v;
+  // resident loops where they are faster still
+  resident_ = true;
+  if (resident_available()) {
+    const int n = std::min(steps, nt_);
+    LoopLaunches *p = loop_launches(4, 0, n);
+    run_loops(*p, n);  // warm up
+    hip_check(hipEventRecord(ev_[0], stream_), "hipEventRecord");
+    run_loops(*p, n);
+    hip_check(hipEventRecord(ev_[1], stream_), "hipEventRecord");
+    hip_check(hipStreamSynchronize(stream_), "hipStreamSynchronize");
+    float ms = 0.f;
+    hip_check(hipEventElapsedTime(&ms, ev_[0], ev_[1]), "hipEventElapsedTime");
+    resident_ = ms / (n * n_shots_) < best_ms;
+  } else {
+    resident_ = false;
+  }
   return best_ms;
 }
 

@@ -199,3 +199,39 @@ def test_models_in_threads():
         t.join()
     for i, (a, b) in enumerate(zip(got, want)):
         _same(a, b, i)
+
+
+def _batch(cfgs, variant=None):
+    import psvwave_amd
+    b = psvwave_amd.Batch(cfgs)
+    if variant is not None:
+        b.set_variant(variant)
+    rng = np.random.default_rng(4)
+    for m, i in enumerate(b.infos):
+        shape = (i["nx"], i["nz"])
+        vp = 1800.0 + 600.0 * rng.random(shape)
+        b.set_parameter_fields(m, vp, vp * (0.4 + 0.1 * rng.random(shape)),
+                               1500.0 + 300.0 * rng.random(shape))
+        shape = (i["n_shots"], i["nr"], i["nt"])
+        b.set_observed_data(m, rng.standard_normal(shape), rng.standard_normal(shape))
+    return b
+
+
+# one launch of small tiles, one of 28-row tiles, and several launches
+@pytest.mark.parametrize("sizes,shots", [
+    ([(61, 47), (20, 33)], 2), ([(133, 71), (90, 61), (240, 117)], 3),
+    ([(301 + 37 * k, 120 + 31 * (k % 5)) for k in range(12)], 2)])
+def test_batch_equals_steps(sizes, shots):
+    print(f"[resident] batch of {len(sizes)}", flush=True)
+    cfgs = [_cfg(nx, nz, shots=shots, nt=40) for nx, nz in sizes]
+    outs = []
+    for variant in (None, 28):
+        b = _batch(cfgs, variant)
+        b.forward_all()
+        traces = [b.get_synthetic_data(m) for m in range(len(b))]
+        b.forward(shots - 1)
+        again = [b.get_synthetic_data(m) for m in range(len(b))]
+        grads = b.gradients()
+        outs.append([x for t in traces + again for x in t] + [grads] +
+                    [k for m in range(len(b)) for k in b.get_kernels(m)])
+    _same(*outs, sizes[0])
