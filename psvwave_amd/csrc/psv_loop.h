@@ -56,9 +56,10 @@ struct LoopArgs {
   double wcorr;
   // injection targets (one component of one point) by tile * waves + wave:
   // targets inj_off[i] .. inj_off[i + 1], the terms of target t being
-  // inj[inj_first[t]] .. inj[inj_first[t + 1]] in list order
+  // inj[inj_first[t]] .. inj[inj_first[t + 1]] in list order, inj_head[t] the
+  // first of them
   const int *inj_off, *inj_first;
-  const InjEntry *inj;
+  const InjEntry *inj, *inj_head;
   const double *stf, *adj_x, *adj_z;
   // receivers, CSR by tile (null: none recorded)
   const int *rec_off;

@@ -5,18 +5,25 @@
 // this device the state fits on chip: 256 compute units hold 128 MB of
 // registers and 40 MB of LDS.  A resident loop therefore runs all time steps
 // in one launch.  Each block owns one tile for the whole loop; stresses and
-// material factors of its points stay in registers, velocities in LDS, and
-// per step only the velocities on the three-point rim of each tile move, from
-// block to block through memory.  What bounds a step is then FP64 issue
-// (about 125 FP64 instructions per point) plus one exchange latency.
+// material factors of its points stay in registers and LDS, velocities in
+// LDS, and per step only the velocities on the three-point rim of each tile
+// move, from block to block through memory.
 //
-// Tile.  Eight waves; lane l of every wave is column x0 - 2 + l, wave w holds
-// the rows q = w P .. w P + P - 1 of the tile, row q being z0 - 2 + q.  The
-// velocity update of the own points needs stresses two points beyond them:
-// the two outer lanes on either side and the two outer rows at either end
-// compute those ring stresses redundantly from exchanged velocities, so one
-// exchange per step suffices and every lane runs the same code.  Own points:
-// up to 60 columns and 8 P - 4 rows.
+// What bounds a step is FP64 issue (about 111 FP64 instructions per point and
+// 40 others, at 1.8 ns per wave and instruction) plus one exchange, about 2 us
+// from the last store to the first value read.  The exchange is hidden only
+// where two blocks share a compute unit.  us per step: 250 x 150 points 2.9
+// (a launch per step: 7.7), 680 x 380 4.7, 960 x 448 on one block per compute
+// unit 5.8 and two such loops on two 8.1 (107e9 points per second), 1800 x
+// 450 7.8 (27).
+//
+// Tile.  Lane l of every wave is column x0 - 2 + l, wave w holds the rows
+// q = w P .. w P + P - 1 of the tile, row q being z0 - 2 + q.  The velocity
+// update of the own points needs stresses two points beyond them: the two
+// outer lanes on either side and the two outer rows at either end compute
+// those ring stresses redundantly from exchanged velocities, so one exchange
+// per step suffices and every lane runs the same code.  Own points: up to 60
+// columns and waves * P - 4 rows.
 //
 // Exchange.  A velocity on a tile's rim is sent as one 16-byte cell {low word, tag,
 // high word, tag}: each 8-byte half carries its own tag (the step's number),
@@ -70,8 +77,21 @@ __device__ __forceinline__ int fresh(int v) {
   asm volatile("" : "+v"(v));
   return v;
 }
+__device__ __forceinline__ unsigned fresh(unsigned v) {
+  asm volatile("" : "+v"(v));
+  return v;
+}
 __device__ __forceinline__ double fresh(double v) {
   asm volatile("" : "+v"(v));
+  return v;
+}
+__device__ __forceinline__ int fresh_uniform(int v) {  // of a scalar register
+  asm volatile("" : "+s"(v));
+  return v;
+}
+__device__ __forceinline__ int fresh_scalar(int v) {
+  v = __builtin_amdgcn_readfirstlane(v);
+  asm volatile("" : "+s"(v));
   return v;
 }
 __device__ __forceinline__ const ConstArgs *fresh(const ConstArgs *v) {
@@ -79,46 +99,38 @@ __device__ __forceinline__ const ConstArgs *fresh(const ConstArgs *v) {
   return v;
 }
 
-// Divisions x / d by a grid spacing d in [2^-40, 2^40].  All give the
-// correctly rounded quotient; which one a pass may use depends on the values
-// around.  `base` is the difference x was formed from: x itself, or x without
-// its material factor.
-//
-// NormalQuotient: FastDiv's operations (psv_kernels.hip), for x = 0 or
-// 2^-960 <= |x| <= 2^980.
-struct NormalQuotient {
+// Quotients x / d by a grid spacing d in [2^-40, 2^40], correctly rounded.
+// FastDiv's operations (psv_kernels.hip) serve x = 0 and 2^-960 <= |x| <=
+// 2^980.  In lanes `scaled` x was scaled by 2^128 before (exactly) and the
+// last operation, a fused multiply-add that scales its result by 2^-128
+// before its one rounding, undoes it; in the others it is a plain one, at
+// the same rate.
+struct Spacing {
   double d, y, zh, zl;
-  __device__ bool tiny(double) const { return false; }
-  __device__ double operator()(double x, bool) const {
+  __device__ double quotient(double x, unsigned long long scaled) const {
     const double q0 = __builtin_fma(x, zl, x * zh);
     const double r = __builtin_fma(q0, d, -x);
-    return __builtin_fma(-r, y, q0);
+    return __builtin_amdgcn_div_fmas(-r, y, q0, __builtin_amdgcn_inverse_ballot_w64(scaled));
   }
 };
-// SmallQuotient: every |x| <= 2^980, subnormal x and quotients included.
-// Where the difference is below 2^-500, x is scaled by 2^128 first (exactly),
-// and the last operation, a fused multiply-add that in such lanes scales its
-// result by 2^-128 before its one rounding, undoes it (with factors of
-// exponents in [-300, 100], x is below 2^-400 there and above 2^-800 or zero
+// The lanes whose dividends have to be scaled: those where the difference
+// they are formed from is below 2^-500 (with material factors of exponents in
+// [-300, 100], a dividend is below 2^-400 there and above 2^-800 or zero
 // elsewhere).
-struct SmallQuotient {
-  double d, y, zh, zl;
-  __device__ bool tiny(double base) const { return __builtin_fabs(base) < 0x1p-500; }
-  __device__ double operator()(double x, bool t) const {
-    const double xs = __builtin_amdgcn_ldexp(x, fresh(t ? 128 : 0));
-    const double q0 = __builtin_fma(xs, zl, xs * zh);
-    const double r = __builtin_fma(q0, d, -xs);
-    return __builtin_amdgcn_div_fmas(-r, y, q0, t);
-  }
-};
-struct PlainQuotient {
-  double d;
-  __device__ bool tiny(double) const { return false; }
-  __device__ double operator()(double x, bool) const { return x / d; }
-};
+__device__ __forceinline__ unsigned long long small_lanes(double difference) {
+  return __ballot(__builtin_fabs(difference) < 0x1p-500);
+}
+__device__ __forceinline__ int scale_of(unsigned long long lanes) {
+  return fresh(__builtin_amdgcn_inverse_ballot_w64(lanes) ? 128 : 0);
+}
+__device__ __forceinline__ void scale(double &x, int exponent) {
+  x = __builtin_amdgcn_ldexp(x, exponent);
+}
 
-// Which division the next pass over some values needs: kNormal if each is
-// zero or of a binary exponent (frexp) in [elimit, 600]; kSmall if only the
+// How the next pass over some values divides (one code for all three, the
+// wave branches around what a mode adds: separate passes cost registers, and
+// spilled factors, read back behind the other block's polls, made a pass
+// three times as long): kNormal if each is zero or of a binary exponent (frexp) in [elimit, 600]; kSmall if only the
 // lower bound fails, as in the numerical precursor ahead of a wavefront;
 // kIeee otherwise (a plain IEEE division for every value: runs that
 // overflow).  Two roundings of differences can cancel to 2^-109 of the
@@ -139,6 +151,9 @@ struct Range {
   // also for values that may be infinite or no numbers
   __device__ void any_values(double a, double b) {
     values(a, b);
+    finite(a, b);
+  }
+  __device__ void finite(double a, double b) {
     if (!(__builtin_fabs(a) + __builtin_fabs(b) < 0x1p800)) emax = 4096;
   }
   // adds the wave's need to *word (in LDS): one lane's atomic per wave, not
@@ -153,52 +168,55 @@ struct Range {
   }
 };
 
-// Stresses of one point (stress_point's expression trees).  vxx: vx at x-1,
-// x+1, x+2; vxz: vx at z-1, z, z+1, z+2; vzx: vz at x-2, x-1, x+1; vzz: vz
-// at z-2, z-1, z, z+1.  la = lm - 2 mu, dm = dts * mu.
-template <bool FINITE, class D>
-__device__ __forceinline__ void loop_stress(const double (&vxx)[3], double vxm, double vx0,
-                                            double vxp, double vxpp, const double (&vzx)[3],
-                                            double vzmm, double vzm, double vz0, double vzp,
-                                            double lm, double la, double dm, double taper,
-                                            double dts, D divx, D divz, Range &range, double &xx,
-                                            double &zz, double &xz) {
-  const double dvx_x = kC1 * (vxx[1] - vx0) + kC2 * (vxx[0] - vxx[2]);
-  const double dvz_z = kC1 * (vz0 - vzm) + kC2 * (vzmm - vzp);
-  const double dvx_z = kC1 * (vxp - vx0) + kC2 * (vxm - vxpp);
-  const double dvz_x = kC1 * (vz0 - vzx[1]) + kC2 * (vzx[0] - vzx[2]);
-  const bool tx = divx.tiny(dvx_x), tz = divz.tiny(dvz_z);
-  xx = taper * (xx + dts * (divx(lm * dvx_x, tx) + divz(la * dvz_z, tz)));
-  zz = taper * (zz + dts * (divx(la * dvx_x, tx) + divz(lm * dvz_z, tz)));
-  xz = taper * (xz + dm * (divz(dvx_z, divz.tiny(dvx_z)) + divx(dvz_x, divx.tiny(dvz_x))));
-  if (FINITE) {
-    range.values(xx, zz);
-    range.values(xz, xz);
+// The terms of one point's strain rates (stress_point's expression trees), in
+// place: from the differences x_* and z_* of vx and vz along x and z to
+// txx's, tzz's and txz's rates, lambda and mu of txx and tzz included.
+template <bool IEEE>
+__device__ __forceinline__ void stress_rates(double dvx_x, double dvz_z, double dvx_z,
+                                             double dvz_x, double lm, double mu, bool small,
+                                             const Spacing &dx, const Spacing &dz, double &xx_rate,
+                                             double &zz_rate, double &xz_rate) {
+  // one operation instead of two, the same value where 2 mu does not overflow
+  const double la = IEEE ? lm - 2 * mu : __builtin_fma(-2.0, mu, lm);
+  double xx_x = lm * dvx_x, xx_z = la * dvz_z, zz_x = la * dvx_x, zz_z = lm * dvz_z;
+  if (IEEE) {
+    xx_x /= dx.d, xx_z /= dz.d, zz_x /= dx.d, zz_z /= dz.d, dvx_z /= dz.d, dvz_x /= dx.d;
   } else {
-    range.any_values(xx, zz);
-    range.any_values(xz, xz);
+    unsigned long long sx = 0, sz = 0, sxx = 0, sxz = 0;
+    if (small) {
+      sx = small_lanes(dvx_x), sz = small_lanes(dvz_z);
+      sxx = small_lanes(dvx_z), sxz = small_lanes(dvz_x);
+      const int ex = scale_of(sx), ez = scale_of(sz);
+      scale(xx_x, ex), scale(zz_x, ex), scale(xx_z, ez), scale(zz_z, ez);
+      scale(dvx_z, scale_of(sxx)), scale(dvz_x, scale_of(sxz));
+    }
+    xx_x = dx.quotient(xx_x, sx), zz_x = dx.quotient(zz_x, sx);
+    xx_z = dz.quotient(xx_z, sz), zz_z = dz.quotient(zz_z, sz);
+    dvx_z = dz.quotient(dvx_z, sxx), dvz_x = dx.quotient(dvz_x, sxz);
   }
+  xx_rate = xx_x + xx_z, zz_rate = zz_x + zz_z, xz_rate = dvx_z + dvz_x;
 }
 
-// Velocities of one point (velocity_point's expression trees).  xxx: txx at
-// x-2, x-1, x+1; xzx: txz at x-1, x+1, x+2.  bd = b * dts.
-template <bool FINITE, class D>
-__device__ __forceinline__ void loop_velocity(const double (&xxx)[3], double xx0,
-                                              const double (&xzx)[3], double xzmm, double xzm,
-                                              double xz0, double xzp, double zzm, double zz0,
-                                              double zzp, double zzpp, double bd, double taper,
-                                              D divx, D divz, Range &range, double &vx,
-                                              double &vz) {
-  const double dxx_x = kC1 * (xx0 - xxx[1]) + kC2 * (xxx[0] - xxx[2]);
-  const double dxz_z = kC1 * (xz0 - xzm) + kC2 * (xzmm - xzp);
-  const double dxz_x = kC1 * (xzx[1] - xz0) + kC2 * (xzx[0] - xzx[2]);
-  const double dzz_z = kC1 * (zzp - zz0) + kC2 * (zzm - zzpp);
-  vx = taper * (vx + bd * (divx(dxx_x, divx.tiny(dxx_x)) + divz(dxz_z, divz.tiny(dxz_z))));
-  vz = taper * (vz + bd * (divx(dxz_x, divx.tiny(dxz_x)) + divz(dzz_z, divz.tiny(dzz_z))));
-  if (FINITE)
-    range.values(vx, vz);
-  else
-    range.any_values(vx, vz);
+// The stress divergences of one point (velocity_point's expression trees)
+// from the differences of txx and txz along x and z for vx, of txz and tzz
+// for vz.
+template <bool IEEE>
+__device__ __forceinline__ void velocity_rates(double vx_x, double vx_z, double vz_x, double vz_z,
+                                               bool small, const Spacing &dx, const Spacing &dz,
+                                               double &vx_rate, double &vz_rate) {
+  if (IEEE) {
+    vx_x /= dx.d, vx_z /= dz.d, vz_x /= dx.d, vz_z /= dz.d;
+  } else {
+    unsigned long long a = 0, b = 0, c = 0, d = 0;
+    if (small) {
+      a = small_lanes(vx_x), b = small_lanes(vx_z), c = small_lanes(vz_x), d = small_lanes(vz_z);
+      scale(vx_x, scale_of(a)), scale(vx_z, scale_of(b));
+      scale(vz_x, scale_of(c)), scale(vz_z, scale_of(d));
+    }
+    vx_x = dx.quotient(vx_x, a), vx_z = dz.quotient(vx_z, b);
+    vz_x = dx.quotient(vz_x, c), vz_z = dz.quotient(vz_z, d);
+  }
+  vx_rate = vx_x + vx_z, vz_rate = vz_x + vz_z;
 }
 
 // Keeps the scheduler from interleaving the stencils of several rows (whose
@@ -263,12 +281,16 @@ resident_loop(LoopLaunch l) {
   constexpr int NRECV = (66 * (SR + 2) - 60 * (SR - 4) + NT - 1) / NT;
   constexpr int RIM = loop_rim_cells(KIND);
   static_assert(NSEND * NT <= RIM, "a tile's rim fits its cells");
-  __shared__ double s_vx[NV], s_vz[NV];
-  __shared__ double s_tz[SR];  // taper factors of the rows
-  // txz of all rows, txx of the own rows 2 .. SR - 3, and of tzz the rows other
-  // waves read, each wave's rows 0, 1 and P - 1
+  // Velocities; taper factors of the rows; txx of the own rows 2 .. SR - 3,
+  // txz of all rows, and of tzz the rows other waves read, each wave's rows 0,
+  // 1 and P - 1.  In one array in this order, so that a strip's neighbour rows
+  // lie at fixed offsets from its own: those of the first and last wave that
+  // do not exist, which no own point uses, are read from the array beside.
   constexpr int ZR = P < 3 ? P : 3;
-  __shared__ double s_xz[SR * 64], s_xx[(SR - 4) * 64], s_zz[NW * ZR * 64];
+  constexpr int NXX = (SR - 4) * 64, NXZ = SR * 64, NZZ = NW * ZR * 64;
+  __shared__ double s_mem[NV + NXX + NXZ + NZZ + NV + SR];
+  double *const s_vx = s_mem, *const s_xx = s_vx + NV, *const s_xz = s_xx + NXX;
+  double *const s_zz = s_xz + NXZ, *const s_vz = s_zz + NZZ, *const s_tz = s_vz + NV;
   // what the next pass over the velocities (by step parity) and over the
   // stresses needs, kNormal | kSmall | kIeee
   __shared__ int s_vmode[2], s_smode, s_factor;
@@ -287,30 +309,54 @@ resident_loop(LoopLaunch l) {
   __syncthreads();
   if (!s_go) return;
 
-  const int lane = threadIdx.x & 63;
+  // The passes over the rows need nearly all of a wave's 128 registers: what
+  // they do not use is packed, derived again from the thread's number, or
+  // read back from memory where it is used.
+  const int tid = threadIdx.x, lane = tid & 63;
+  auto lane_of = [&]() { return fresh(tid) & 63; };
   const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int nx = A.nx, nz = A.nz, nt = A.nt;
-  const int tile = bt.z * A.ntx + bt.y;
-  const int x0 = (int)((long long)bt.y * nx / A.ntx);
-  const int z0 = (int)((long long)bt.z * nz / A.ntz);
-  const int wt = (int)((long long)(bt.y + 1) * nx / A.ntx) - x0;  // own columns
-  const int ht = (int)((long long)(bt.z + 1) * nz / A.ntz) - z0;  // own rows
+  // first column of tile column i and first row of tile row i (uniform, but
+  // divided in vector registers)
+  auto tile_x0 = [&](int i) {
+    return __builtin_amdgcn_readfirstlane((int)((long long)i * nx / A.ntx));
+  };
+  auto tile_z0 = [&](int i) {
+    return __builtin_amdgcn_readfirstlane((int)((long long)i * nz / A.ntz));
+  };
+  const int tile = __builtin_amdgcn_readfirstlane(bt.z * A.ntx + bt.y);
+  const int x0 = tile_x0(bt.y), wt = tile_x0(bt.y + 1) - x0;  // own columns
+  const int z0 = tile_z0(bt.z), ht = tile_z0(bt.z + 1) - z0;  // own rows
   const int q0 = w * P;         // first row of the strip
   const int zs = z0 - 2 + q0;   // its grid row
   const int x = x0 - 2 + lane;
   const bool own_x = lane >= 2 && lane < 2 + wt;
   // strip rows with a stress / velocity stencil, and own rows
-  auto clampj = [&](int j) { return min(max(j, 0), P); };
-  const int js0 = clampj(2 - zs), js1 = clampj(min(nz - 2 - zs, ht + 4 - q0));
-  const int jo0 = clampj(2 - q0), jo1 = clampj(ht + 2 - q0);
-  const int jv0 = max(js0, jo0), jv1 = min(jo1, clampj(nz - 2 - zs));
+  // the strip's rows with a stress stencil (bit j), with a velocity stencil
+  // (bit 4 + j), its own rows (8 + j) and the rows s_xx has (12 + j)
+  int rows = 0;
+#pragma unroll
+  for (int j = 0; j < P; ++j) {
+    const int q = q0 + j, z = zs + j;
+    const bool stencil = z >= 2 && z < nz - 2, own = q >= 2 && q < ht + 2;
+    rows |= (stencil && q < ht + 4) << j | (stencil && own) << (4 + j) | own << (8 + j) |
+            (q >= 2 && q < SR - 2) << (12 + j);
+  }
+  rows = __builtin_amdgcn_readfirstlane(rows);
+  // (tested anew in each pass: a scalar register, not one per row and test)
+  auto has = [&](int test, int j) { return (fresh_uniform(rows) >> (test + j) & 1) != 0; };
+  enum : int { kStressRow = 0, kVelocityRow = 4, kOwnRow = 8, kXxRow = 12 };
   const bool xs = x >= 2 && x < nx - 2 && lane < wt + 4;
   const bool xv = own_x && xs;
   const double dts = A.dts;
 
   // ---- the tile's constants and initial state ----
-  double lm[P], la[P], dm[P], bd[P];
-  double xx[P], zz[P], xz[P];
+  double lm[P], mu[P], bd[P];
+  // Stresses: tzz and, of the first XK rows, txx stay in registers; txz and the
+  // other rows' txx (of own rows; the ring's is not used) in LDS, where the
+  // velocity pass reads them anyway.
+  constexpr int XK = P == 4 ? 0 : P;
+  double xx[P], zz[P];
   int factor_exp = 0;  // smallest of the material factors; -4096: one is too large
   const double tx = gp(A.taper_x)[min(x, nx + 1)];
   {
@@ -319,22 +365,24 @@ resident_loop(LoopLaunch l) {
     for (int j = 0; j < P; ++j) {
       const int zc = min(zs + j, nz + 1);
       const long long g = A.origin + (long long)zc * A.pitch + xc;
-      const double m = gp(A.mu)[g];
+      mu[j] = gp(A.mu)[g];
       lm[j] = gp(A.lm)[g];
-      la[j] = lm[j] - 2 * m;
-      dm[j] = dts * m;
       bd[j] = gp(A.b)[g] * dts;
-      for (double f : {lm[j], la[j]})
+      for (double f : {lm[j], lm[j] - 2 * mu[j]})
         if (f != 0.0) factor_exp = min(factor_exp, __builtin_amdgcn_frexp_exp(f));
-      for (double f : {lm[j], la[j], m, dm[j], bd[j], dts})
+      for (double f : {lm[j], lm[j] - 2 * mu[j], mu[j], dts * mu[j], bd[j], dts})
         if (!(__builtin_fabs(f) <= 0x1p100)) factor_exp = -4096;
-      xx[j] = zz[j] = xz[j] = 0.0;
+      xx[j] = zz[j] = 0.0;
+      double xz = 0.0;
       if (A.in[0] && x >= 0 && x < nx && zs + j >= 0 && zs + j < nz) {
         const long long s = A.in_origin + (long long)(zs + j) * A.in_pitch + x;
         xx[j] = gp(A.in[2])[s];
         zz[j] = gp(A.in[3])[s];
-        xz[j] = gp(A.in[4])[s];
+        xz = gp(A.in[4])[s];
       }
+      s_xz[(q0 + j) * 64 + lane] = xz;
+      if (has(kXxRow, j)) s_xx[(q0 + j - 2) * 64 + lane] = xx[j];
+      if (j < 2 || j == P - 1) s_zz[(w * ZR + min(j, 2)) * 64 + lane] = zz[j];
     }
   }
   for (int i = threadIdx.x; i < SR; i += NT) s_tz[i] = gp(A.taper_z)[min(z0 - 2 + i, nz + 1)];
@@ -374,11 +422,14 @@ resident_loop(LoopLaunch l) {
     if (r >= ht - 3) return (r - ht + 6) * wt + c;
     return 6 * wt + (c < 3 ? (r - 3) * 3 + c : (ht + r - 9) * 3 + c - wt + 3);
   };
-  int send_l[NSEND], recv_l[NRECV];
+  // LDS indices of the rim cell it sends (low half; kNoCell: none) and of its
+  // receiver (high half), and of the frame cells it receives
+  constexpr unsigned kNoCell = 0xffffu;
+  static_assert(NSEND == 1 && NRECV <= 2 && NV < (int)kNoCell, "cells are packed in halves");
+  unsigned send_rec = kNoCell << 16, recv_pack = 0;
   unsigned recv_g[NRECV];
-#pragma unroll
-  for (int s = 0; s < NSEND; ++s) {
-    const int i = threadIdx.x + s * NT;
+  {
+    const int i = tid;
     int r, c;
     bool on;
     if (wt > 6 && ht > 6) {
@@ -397,7 +448,7 @@ resident_loop(LoopLaunch l) {
       r = i / wt;
       c = i - r * wt;
     }
-    send_l[s] = on ? vidx(r, c) : -1;
+    send_rec |= on ? (unsigned)vidx(r, c) : kNoCell;
   }
 #pragma unroll
   for (int s = 0; s < NRECV; ++s) {
@@ -416,7 +467,7 @@ resident_loop(LoopLaunch l) {
     }
     const int xi = x0 + c, zi = z0 + r;
     on = on && xi >= 0 && xi < nx && zi >= 0 && zi < nz;
-    recv_l[s] = on ? vidx(r, c) : -1;
+    recv_pack |= (on ? (unsigned)vidx(r, c) : kNoCell) << (16 * s);
     recv_g[s] = 0;
     if (on) {  // the adjacent tile that owns the point
       const int ox = bt.y + (c < 0 ? -1 : c >= wt ? 1 : 0);
@@ -430,7 +481,6 @@ resident_loop(LoopLaunch l) {
   }
   const auto cells =
       __builtin_amdgcn_make_buffer_rsrc(A.cells, 0, A.cells_bytes, 0x00020000);
-  const unsigned send_g = (unsigned)(tile * 4 * RIM + (int)threadIdx.x) * 16u;
 
   // ---- this wave's injection targets: target t in lane t ----
   const int tg0 = __builtin_amdgcn_readfirstlane(gp(A.inj_off)[tile * NW + w]);
@@ -447,13 +497,13 @@ resident_loop(LoopLaunch l) {
     return ADJ ? A.dt * b * val / A.dxdz : coef * val * A.dt * b / (comp ? A.d4z : A.d4x);
   };
   // ---- this thread's receiver ----
-  int rec_l = -1, rec_k = 0;
-  double rec_sx = 0.0, rec_sz = 0.0;
+  int rec_k = 0;
+  double rec_sx = 0.0, rec_sz = 0.0;  // (read back where registers are short)
   if (!ADJ && A.rec_off) {
     const int r0 = gp(A.rec_off)[tile], nr = gp(A.rec_off)[tile + 1] - r0;
-    if ((int)threadIdx.x < nr) {
-      rec_l = gp(A.rec)[r0 + threadIdx.x].local;
-      rec_k = gp(A.rec)[r0 + threadIdx.x].src;
+    if (tid < nr) {
+      send_rec = (send_rec & 0xffffu) | (unsigned)gp(A.rec)[r0 + tid].local << 16;
+      rec_k = gp(A.rec)[r0 + tid].src;
     }
   }
   __syncthreads();
@@ -461,63 +511,83 @@ resident_loop(LoopLaunch l) {
   const int tile_exp = __builtin_amdgcn_readfirstlane(s_factor);
   const int floor_mode = tile_exp < -300 ? kIeee : kNormal;
   const int elimit = -849 - tile_exp;
-  // LDS indices of the strip's first velocity and txz row, and of the rows
-  // above and below it (clamped where no stencil uses them), each to be added
+  auto mode_of = [&](int needs) {  // needs: kSmall and kIeee bits
+    return min(max(floor_mode, __builtin_amdgcn_readfirstlane(needs)), (int)kIeee);
+  };
+  // LDS indices of the strip's first velocity and stress row, each to be added
   // to the lane
   const int vrow = (q0 + 2) * kVW + 2, srow = q0 * 64;
-  const int up2 = max(q0 - 2, 0) * 64, up1 = max(q0 - 1, 0) * 64;
-  const int dn1 = min(q0 + P, SR - 1) * 64;
-  auto zrow = [](int q) {
-    q = min(max(q, 0), SR - 1);
-    return (P < 3 ? q : q / P * 3 + (q % P == P - 1 ? 2 : q % P)) * 64;
-  };
-  const int zup = zrow(q0 - 1), zdn0 = zrow(q0 + P), zdn1 = zrow(q0 + P + 1);
-  const bool full_s = js0 == 0 && js1 == P, full_v = jv0 == 0 && jv1 == P;
   unsigned tag = l.tag0;
 
+  // The velocity that the lane's first injection target adds to (2 LDS index +
+  // component; -1: none; bit 30: several terms) and its next term.
+  int inj_at = -1;
+  double inj_value = 0.0;
+  constexpr int kInjMore = 1 << 30;
+  auto inj_fetch = [&](int base, int it) {
+    const ConstArgs &A = *fresh(&A0);
+    const int t = base + lane_of();
+    inj_at = -1;
+    if (t < ntg) {
+      const Global<const InjEntry> *const p = gp(A.inj_head) + tg0 + t;
+      const InjEntry E = {p->local, p->comp, p->src, p->pad, p->coef};
+      const int r = E.local >> 6, c = E.local & 63;
+      inj_at = ((vrow + r * kVW + c) << 1) | E.comp | (E.pad ? kInjMore : 0);
+      inj_value = inj_term(A, E.comp, E.coef,
+                           gp(A.b)[A.origin + (long long)(zs + r) * A.pitch + x0 - 2 + c],
+                           inj_sample(A, E, it));
+    }
+  };
+
   // What a step does with the state at its start: receivers, snapshot store,
-  // correlation.  Called between sending the rims and waiting for the
-  // neighbours' (the state then is the next step's), which hides it.
+  // correlation; and its injection terms.  Called between sending the rims and
+  // the first poll for the neighbours' (the state then is the next step's),
+  // which hides it.
   int phase = (ADJ ? nt - 1 - A0.k0 : A0.k0) % A0.si;  // of the next step's time index
   auto begin_step = [&](int k) {
     const ConstArgs &A = *fresh(&A0);
     const int it = ADJ ? nt - 1 - k : k;
     const bool snap_step = phase == 0;
     phase = ADJ ? (phase == 0 ? A.si : phase) - 1 : (phase + 1 == A.si ? 0 : phase + 1);
-    const int xk = fresh(x), va0 = vrow + fresh(lane);
-    if (rec_l >= 0) {
-      // receiver record at the start of the step (src/fdModel.cpp:576-596)
-      const double ax = A.dt * s_vx[rec_l] / A.dxdz, az = A.dt * s_vz[rec_l] / A.dxdz;
-      rec_sx = k == 0 ? ax : rec_sx + ax;
-      rec_sz = k == 0 ? az : rec_sz + az;
+    const unsigned rec_l = fresh(send_rec) >> 16;
+    if (!ADJ && rec_l != kNoCell) {
+      // receiver record at the start of the step (src/fdModel.cpp:576-596),
+      // which continues the previous step's
       const long long at = (long long)fresh(rec_k) * nt + it;
-      gp(A.rtf_x)[at] = rec_sx;
-      gp(A.rtf_z)[at] = rec_sz;
+      const double ax = A.dt * s_vx[rec_l] / A.dxdz, az = A.dt * s_vz[rec_l] / A.dxdz;
+      double sx = rec_sx, sz = rec_sz;
+      if (P == 4 && k > 0) sx = gp(A.rtf_x)[at - 1], sz = gp(A.rtf_z)[at - 1];
+      sx = k == 0 ? ax : sx + ax;
+      sz = k == 0 ? az : sz + az;
+      gp(A.rtf_x)[at] = sx;
+      gp(A.rtf_z)[at] = sz;
+      if (P < 4) rec_sx = sx, rec_sz = sz;
     }
+    if (ntg > 0) inj_fetch(0, it);
     if (snap_step && A.snap[0] && it / A.si % A.slot_every == 0) {
+      const int ln = lane_of(), va0 = vrow + ln, xk = x0 - 2 + ln;
       const int slot = it / A.si;
       const long long so = (long long)(slot / A.slot_every - A.slot0) * A.slot_stride;
       if (!ADJ) {
         if (own_x)
 #pragma unroll
           for (int j = 0; j < P; ++j)
-            if (j >= jo0 && j < jo1) {
+            if (has(kOwnRow, j)) {
               const long long ci = so + (long long)(zs + j) * nx + xk;
               __builtin_nontemporal_store(s_vx[va0 + j * kVW], gp(A.snap[0]) + ci);
               __builtin_nontemporal_store(s_vz[va0 + j * kVW], gp(A.snap[1]) + ci);
-              __builtin_nontemporal_store(xx[j], gp(A.snap[2]) + ci);
+              __builtin_nontemporal_store(s_xx[srow + ln + (j - 2) * 64], gp(A.snap[2]) + ci);
               __builtin_nontemporal_store(zz[j], gp(A.snap[3]) + ci);
-              __builtin_nontemporal_store(xz[j], gp(A.snap[4]) + ci);
+              __builtin_nontemporal_store(s_xz[srow + ln + j * 64], gp(A.snap[4]) + ci);
             }
       } else {
         const long long ko = A.defer_stride * slot;
-        if (own_x && x >= A.kx0 && x < A.kx1)
+        if (own_x && xk >= A.kx0 && xk < A.kx1)
 #pragma unroll
           for (int j = 0; j < P; ++j) {
             const int z = zs + j;
-            if (j >= jo0 && j < jo1 && z >= A.kz0 && z < A.kz1) {
-              const long long c = (long long)z * nx + x, ci = so + c, ck = ko + c;
-              const long long g = A.origin + (long long)z * A.pitch + xk;
+            if (has(kOwnRow, j) && z >= A.kz0 && z < A.kz1) {
+              const long long c = (long long)z * nx + xk, ci = so + c, ck = ko + c;
               double r = 0.0, la_k = 0.0, m = 0.0, s[5];
 #pragma unroll
               for (int f = 0; f < 5; ++f) s[f] = __builtin_nontemporal_load(gp(A.snap[f]) + ci);
@@ -526,27 +596,28 @@ resident_loop(LoopLaunch l) {
                 la_k = __builtin_nontemporal_load(gp(A.lam_k) + ck);
                 m = __builtin_nontemporal_load(gp(A.mu_k) + ck);
               }
-              correlate_point(A.wcorr, lm[j], gp(A.mu)[g], s_vx[va0 + j * kVW], s_vz[va0 + j * kVW],
-                              xx[j], zz[j], xz[j], s[0], s[1], s[2], s[3], s[4], r, la_k, m);
+              correlate_point(A.wcorr, lm[j], mu[j], s_vx[va0 + j * kVW], s_vz[va0 + j * kVW],
+                              s_xx[srow + ln + (j - 2) * 64], zz[j], s_xz[srow + ln + j * 64], s[0],
+                              s[1], s[2], s[3], s[4], r, la_k, m);
               __builtin_nontemporal_store(r, gp(A.rho_k) + ck);
               __builtin_nontemporal_store(la_k, gp(A.lam_k) + ck);
               __builtin_nontemporal_store(m, gp(A.mu_k) + ck);
             }
+            row_fence();
           }
       }
     }
-
   };
   begin_step(A.k0);
 
   for (int k = A.k0; k < A.k1; ++k, ++tag) {
     const int it = ADJ ? nt - 1 - k : k;
-    const double txk = fresh(tx);
     // ---- stresses ----
-    auto stress_pass = [&](auto full, auto divx, auto divz) {
-      constexpr bool FULL = decltype(full)::value;
-      constexpr bool FINITE = !std::is_same<decltype(divx), PlainQuotient>::value;
-      const int va = vrow + fresh(lane), ta = fresh(q0);
+    const int vmode = mode_of(s_vmode[(k + 1) & 1]);
+    if (xs) {
+      const Spacing dx{A.dx, A.rdx, A.zhx, A.zlx}, dz{A.dz, A.rdz, A.zhz, A.zlz};
+      const int ln = lane_of(), va = vrow + ln, sa = srow + ln, ta = fresh(q0);
+      const int za = fresh_scalar(w) * ZR * 64 + ln;
       Range range;
       // vx rows -1 .. P + 1 and vz rows -2 .. P of the lane's column
       double cx[P + 3], cz[P + 3];
@@ -560,126 +631,110 @@ resident_loop(LoopLaunch l) {
         const int v = va + j * kVW;
         cx[j + 3] = s_vx[v + 2 * kVW];
         cz[j + 3] = s_vz[v + kVW];
-        if (FULL || (j >= js0 && j < js1)) {
-          const double ax[3] = {s_vx[v - 1], s_vx[v + 1], s_vx[v + 2]};
-          const double az[3] = {s_vz[v - 2], s_vz[v - 1], s_vz[v + 1]};
-          loop_stress<FINITE>(ax, cx[j], cx[j + 1], cx[j + 2], cx[j + 3], az, cz[j], cz[j + 1],
-                      cz[j + 2], cz[j + 3], lm[j], la[j], dm[j], min_factor(txk, s_tz[ta + j]),
-                      dts, divx, divz, range, xx[j], zz[j], xz[j]);
+        if (has(kStressRow, j)) {
+          const double dvx_x = kC1 * (s_vx[v + 1] - cx[j + 1]) + kC2 * (s_vx[v - 1] - s_vx[v + 2]);
+          const double dvz_z = kC1 * (cz[j + 2] - cz[j + 1]) + kC2 * (cz[j] - cz[j + 3]);
+          const double dvx_z = kC1 * (cx[j + 2] - cx[j + 1]) + kC2 * (cx[j] - cx[j + 3]);
+          const double dvz_x = kC1 * (cz[j + 2] - s_vz[v - 1]) + kC2 * (s_vz[v - 2] - s_vz[v + 1]);
+          // read while the rates are computed, not before: the neighbours'
+          // registers are free by now
+          if (P == 4) row_fence();
+          double tz;
+          if (P < 4) tz = s_tz[ta + j];
+          double xz = s_xz[sa + j * 64];
+          if (j >= XK) xx[j] = has(kXxRow, j) ? s_xx[sa + (j - 2) * 64] : 0.0;
+          mu[j] = fresh(mu[j]);  // 2 mu, dts mu: computed here, not kept (and spilled)
+          double xx_rate, zz_rate, xz_rate;
+          if (__builtin_expect(vmode == kIeee, 0))
+            stress_rates<true>(dvx_x, dvz_z, dvx_z, dvz_x, lm[j], mu[j], false, dx, dz, xx_rate,
+                               zz_rate, xz_rate);
+          else
+            stress_rates<false>(dvx_x, dvz_z, dvx_z, dvz_x, lm[j], mu[j], vmode == kSmall, dx, dz,
+                                xx_rate, zz_rate, xz_rate);
+          if (P == 4) tz = s_tz[ta + j];
+          const double taper = min_factor(tx, tz);
+          xx[j] = taper * (xx[j] + dts * xx_rate);
+          zz[j] = taper * (zz[j] + dts * zz_rate);
+          xz = taper * (xz + dts * mu[j] * xz_rate);
+          range.values(xx[j], zz[j]);
+          range.values(xz, xz);
+          if (vmode == kIeee) {
+            asm volatile("");  // a branch, no selects for the other modes to run
+            range.finite(xx[j], zz[j]);
+            range.finite(xz, xz);
+          }
+          s_xz[sa + j * 64] = xz;
+          if (has(kXxRow, j)) s_xx[sa + (j - 2) * 64] = xx[j];
+          if (j < 2 || j == P - 1) s_zz[za + min(j, 2) * 64] = zz[j];
         }
         row_fence();
       }
       range.report(&s_smode, elimit);
-    };
-    const int vmode = max(floor_mode, __builtin_amdgcn_readfirstlane(s_vmode[(k + 1) & 1]));
-    if (xs) {
-      if (vmode == kNormal) {
-        const NormalQuotient dx{A.dx, A.rdx, A.zhx, A.zlx}, dz{A.dz, A.rdz, A.zhz, A.zlz};
-        if (full_s)
-          stress_pass(std::true_type{}, dx, dz);
-        else
-          stress_pass(std::false_type{}, dx, dz);
-      } else if (vmode == kSmall) {
-        const SmallQuotient dx{A.dx, A.rdx, A.zhx, A.zlx}, dz{A.dz, A.rdz, A.zhz, A.zlz};
-        if (full_s)
-          stress_pass(std::true_type{}, dx, dz);
-        else
-          stress_pass(std::false_type{}, dx, dz);
-      } else {
-        stress_pass(std::false_type{}, PlainQuotient{A.dx}, PlainQuotient{A.dz});
-      }
-    }
-    {
-    const int sa0 = srow + fresh(lane);
-#pragma unroll
-    for (int j = 0; j < P; ++j) {
-      if (q0 + j >= 2 && q0 + j < SR - 2) s_xx[sa0 + (j - 2) * 64] = xx[j];
-      s_xz[sa0 + j * 64] = xz[j];
-    }
-#pragma unroll
-    for (int j = 0; j < ZR; ++j) s_zz[w * ZR * 64 - srow + sa0 + j * 64] = zz[j < 2 ? j : P - 1];
     }
     __syncthreads();
 
     // ---- velocities ----
-    // the injection operands of the wave's first 64 targets, in flight during
-    // the pass
-    int inj_at = 0, inj_more = 0;
-    double inj_coef = 0.0, inj_bv = 0.0, inj_val = 0.0;
-    auto inj_fetch = [&](int base) {
-      const ConstArgs &A = *fresh(&A0);
-      const int t = base + fresh(lane);
-      if (t < ntg) {
-        const int e = gp(A.inj_first)[tg0 + t];
-        const InjEntry E = inj_entry(A, e);
-        // LDS index of the point's velocity, and the component
-        inj_at = ((vrow + (E.local >> 6) * kVW + (E.local & 63)) << 1) | E.comp;
-        inj_more = E.pad;
-        inj_coef = E.coef;
-        inj_bv = gp(A.b)[A.origin + (long long)(zs + (E.local >> 6)) * A.pitch + x0 - 2 +
-                     (E.local & 63)];
-        inj_val = inj_sample(A, E, it);
-      }
-    };
-    inj_fetch(0);
     if (threadIdx.x == 0) s_vmode[(k + 1) & 1] = 0;  // read by all before the barrier
-    auto velocity_pass = [&](auto full, auto divx, auto divz) {
-      constexpr bool FULL = decltype(full)::value;
-      constexpr bool FINITE = !std::is_same<decltype(divx), PlainQuotient>::value;
-      const int ln = fresh(lane), va = vrow + ln, sa = srow + ln, ta = fresh(q0);
+    const int smode = mode_of(s_smode);
+    if (xv) {
+      const Spacing dx{A.dx, A.rdx, A.zhx, A.zlx}, dz{A.dz, A.rdz, A.zhz, A.zlz};
+      const int ln = lane_of(), va = vrow + ln, sa = srow + ln, ta = fresh(q0);
+      const int za = fresh_scalar(w) * ZR * 64 + ln;
       Range range;
-      const double xzu2 = s_xz[up2 + ln], xzu1 = s_xz[up1 + ln], xzd = s_xz[dn1 + ln];
-      const double zzu = s_zz[zup + ln], zzd0 = s_zz[zdn0 + ln], zzd1 = s_zz[zdn1 + ln];
-      auto XZ = [&](int j) { return j == -2 ? xzu2 : j == -1 ? xzu1 : j == P ? xzd : xz[j]; };
-      auto ZZ = [&](int j) { return j == -1 ? zzu : j == P ? zzd0 : j == P + 1 ? zzd1 : zz[j]; };
+      // txz rows -2 .. P and tzz rows -1 .. P + 1 of the lane's column
+      double xz[P + 3] = {s_xz[sa - 128], s_xz[sa - 64], s_xz[sa]};
+      double cz[P + 3] = {s_zz[za - 64], zz[0], P > 1 ? zz[P > 1 ? 1 : 0] : s_zz[za + ZR * 64]};
 #pragma unroll
       for (int j = 0; j < P; ++j) {
-        if (FULL || (j >= jv0 && j < jv1)) {
+        xz[j + 3] = s_xz[sa + (j + 1) * 64];
+        cz[j + 3] = j + 2 < P ? zz[j + 2 < P ? j + 2 : 0] : s_zz[za + (ZR + j + 2 - P) * 64];
+        if (has(kVelocityRow, j)) {
           const int s = sa + j * 64, x2 = s - 2 * 64;
-          double vx = s_vx[va + j * kVW], vz = s_vz[va + j * kVW];
-          const double ax[3] = {s_xx[x2 - 2], s_xx[x2 - 1], s_xx[x2 + 1]};
-          const double az[3] = {s_xz[s - 1], s_xz[s + 1], s_xz[s + 2]};
-          loop_velocity<FINITE>(ax, xx[j], az, XZ(j - 2), XZ(j - 1), XZ(j), XZ(j + 1), ZZ(j - 1), ZZ(j),
-                        ZZ(j + 1), ZZ(j + 2), bd[j], min_factor(txk, s_tz[ta + j]), divx, divz,
-                        range, vx, vz);
+          const double xx0 = j < XK ? xx[j] : s_xx[x2];
+          const double vx_x = kC1 * (xx0 - s_xx[x2 - 1]) + kC2 * (s_xx[x2 - 2] - s_xx[x2 + 1]);
+          const double vx_z = kC1 * (xz[j + 2] - xz[j + 1]) + kC2 * (xz[j] - xz[j + 3]);
+          const double vz_x = kC1 * (s_xz[s + 1] - xz[j + 2]) + kC2 * (s_xz[s - 1] - s_xz[s + 2]);
+          const double vz_z = kC1 * (cz[j + 2] - cz[j + 1]) + kC2 * (cz[j] - cz[j + 3]);
+          if (P == 4) row_fence();
+          const double tz = s_tz[ta + j], vx0 = s_vx[va + j * kVW], vz0 = s_vz[va + j * kVW];
+          double vx_rate, vz_rate;
+          if (__builtin_expect(smode == kIeee, 0))
+            velocity_rates<true>(vx_x, vx_z, vz_x, vz_z, false, dx, dz, vx_rate, vz_rate);
+          else
+            velocity_rates<false>(vx_x, vx_z, vz_x, vz_z, smode == kSmall, dx, dz, vx_rate,
+                                  vz_rate);
+          const double taper = min_factor(tx, tz);
+          const double vx = taper * (vx0 + bd[j] * vx_rate);
+          const double vz = taper * (vz0 + bd[j] * vz_rate);
+          range.values(vx, vz);
+          if (smode == kIeee) {
+            asm volatile("");
+            range.finite(vx, vz);
+          }
           s_vx[va + j * kVW] = vx;
           s_vz[va + j * kVW] = vz;
         }
         row_fence();
       }
       range.report(&s_vmode[k & 1], elimit);
-    };
-    const int smode = max(floor_mode, __builtin_amdgcn_readfirstlane(s_smode));
-    if (xv) {
-      if (smode == kNormal) {
-        const NormalQuotient dx{A.dx, A.rdx, A.zhx, A.zlx}, dz{A.dz, A.rdz, A.zhz, A.zlz};
-        if (full_v)
-          velocity_pass(std::true_type{}, dx, dz);
-        else
-          velocity_pass(std::false_type{}, dx, dz);
-      } else if (smode == kSmall) {
-        const SmallQuotient dx{A.dx, A.rdx, A.zhx, A.zlx}, dz{A.dz, A.rdz, A.zhz, A.zlz};
-        if (full_v)
-          velocity_pass(std::true_type{}, dx, dz);
-        else
-          velocity_pass(std::false_type{}, dx, dz);
-      } else {
-        velocity_pass(std::false_type{}, PlainQuotient{A.dx}, PlainQuotient{A.dz});
-      }
     }
     // injection: lane t adds the terms of target t in list order
     for (int base = 0; base < ntg; base += 64) {
       const ConstArgs &A = *fresh(&A0);
-      if (base) inj_fetch(base);
-      if (base + lane < ntg) {
-        double *const v = (inj_at & 1 ? s_vz : s_vx) + (inj_at >> 1);
-        double a = *v + inj_term(A, inj_at & 1, inj_coef, inj_bv, inj_val);
-        if (inj_more) {  // several terms at one point
-          int e = gp(A.inj_first)[tg0 + base + lane];
-          const int e1 = gp(A.inj_first)[tg0 + base + lane + 1];
+      if (base) inj_fetch(base, it);
+      if (inj_at >= 0) {
+        const int vi = (inj_at & ~kInjMore) >> 1;
+        double *const v = (inj_at & 1 ? s_vz : s_vx) + vi;
+        double a = *v + inj_value;
+        if (inj_at & kInjMore) {  // several terms at one point
+          const int t = tg0 + base + lane_of();
+          int e = gp(A.inj_first)[t];
+          const int e1 = gp(A.inj_first)[t + 1];
+          const int r = vi / kVW - 2, c = vi % kVW - 2;
+          const double bv = gp(A.b)[A.origin + (long long)(z0 - 2 + r) * A.pitch + x0 - 2 + c];
           for (++e; e < e1; ++e) {
             const InjEntry F = inj_entry(A, e);
-            a += inj_term(A, F.comp, F.coef, inj_bv, inj_sample(A, F, it));
+            a += inj_term(A, F.comp, F.coef, bv, inj_sample(A, F, it));
           }
         }
         *v = a;
@@ -694,35 +749,41 @@ resident_loop(LoopLaunch l) {
     if (threadIdx.x == 0) s_smode = 0;  // read by all before the barrier
     if (k + 1 < A.k1) {
       const unsigned set = (k & 1) ? 2u * RIM * 16u : 0u;
-#pragma unroll
-      for (int s = 0; s < NSEND; ++s)
-        if (send_l[s] >= 0) {
-          const int at = fresh(send_l[s]);
-          const double a = s_vx[at], b = s_vz[at];
-          const u32x4 ca = {(unsigned)__double2loint(a), tag, (unsigned)__double2hiint(a), tag};
-          const u32x4 cb = {(unsigned)__double2loint(b), tag, (unsigned)__double2hiint(b), tag};
-          __builtin_amdgcn_raw_buffer_store_b128(ca, cells, (int)(send_g + set + s * NT * 16), 0,
-                                                 kDeviceScope);
-          __builtin_amdgcn_raw_buffer_store_b128(cb, cells, (int)(send_g + set + (RIM + s * NT) * 16), 0,
-                                                 kDeviceScope);
-        }
-      begin_step(k + 1);
+      const unsigned send_l = fresh(send_rec) & 0xffffu;
+      if (send_l != kNoCell) {
+        const double a = s_vx[send_l], b = s_vz[send_l];
+        const u32x4 ca = {(unsigned)__double2loint(a), tag, (unsigned)__double2hiint(a), tag};
+        const u32x4 cb = {(unsigned)__double2loint(b), tag, (unsigned)__double2hiint(b), tag};
+        const int to = fresh(tid) * 16, base = (int)(tile * 4u * RIM * 16u + set);
+        __builtin_amdgcn_raw_buffer_store_b128(ca, cells, to, base, kDeviceScope);
+        __builtin_amdgcn_raw_buffer_store_b128(cb, cells, to, base + RIM * 16, kDeviceScope);
+      }
       u32x4 ra[NRECV], rb[NRECV];
+      unsigned recv_l[NRECV];
+#pragma unroll
+      for (int s = 0; s < NRECV; ++s) recv_l[s] = fresh(recv_pack) >> (16 * s) & 0xffffu;
+      auto poll = [&]() {
+#pragma unroll
+        for (int s = 0; s < NRECV; ++s)
+          if (recv_l[s] != kNoCell) {
+            ra[s] = __builtin_amdgcn_raw_buffer_load_b128(cells, (int)recv_g[s], (int)set,
+                                                          kDeviceScope);
+            rb[s] = __builtin_amdgcn_raw_buffer_load_b128(cells, (int)recv_g[s],
+                                                          (int)(set + RIM * 16u), kDeviceScope);
+          }
+        asm volatile("" ::: "memory");
+      };
+      begin_step(k + 1);
+      // polls share the fabric with the cells they wait for: asking at once
+      // and without pause cost 960 x 448 points 6.8 us per step, these pauses
+      // (of 64 cycles each) make it 6.0, longer ones no less
+      __builtin_amdgcn_s_sleep(P == 4 ? 8 : 4);
+      poll();
       for (unsigned spin = 0;;) {
         bool ready = true;
 #pragma unroll
         for (int s = 0; s < NRECV; ++s)
-          if (recv_l[s] >= 0) {
-            ra[s] = __builtin_amdgcn_raw_buffer_load_b128(cells, (int)(set + recv_g[s]), 0,
-                                                          kDeviceScope);
-            rb[s] = __builtin_amdgcn_raw_buffer_load_b128(cells, (int)(set + recv_g[s] + RIM * 16u),
-                                                          0,
-                                                          kDeviceScope);
-          }
-        asm volatile("" ::: "memory");
-#pragma unroll
-        for (int s = 0; s < NRECV; ++s)
-          if (recv_l[s] >= 0)
+          if (recv_l[s] != kNoCell)
             ready = ready && ra[s].y == tag && ra[s].w == tag && rb[s].y == tag && rb[s].w == tag;
         if (ready) break;
         // all blocks run, so a neighbour answers within microseconds; a wait
@@ -731,12 +792,14 @@ resident_loop(LoopLaunch l) {
           s_stall = 1;
           break;
         }
+        __builtin_amdgcn_s_sleep(2);
+        poll();
       }
       Range range;
 #pragma unroll
       for (int s = 0; s < NRECV; ++s)
-        if (recv_l[s] >= 0) {
-          const int at = fresh(recv_l[s]);
+        if (recv_l[s] != kNoCell) {
+          const unsigned at = recv_l[s];
           const double a = __hiloint2double((int)ra[s].z, (int)ra[s].x);
           const double b = __hiloint2double((int)rb[s].z, (int)rb[s].x);
           s_vx[at] = a;
@@ -754,13 +817,13 @@ resident_loop(LoopLaunch l) {
     } else if (A.out[0] && own_x) {
 #pragma unroll
       for (int j = 0; j < P; ++j)
-        if (j >= jo0 && j < jo1) {
-          const long long g = A.origin + (long long)(zs + j) * A.pitch + x;
+        if (has(kOwnRow, j)) {
+          const long long g = A.origin + (long long)(zs + j) * A.pitch + x0 - 2 + lane;
           gp(A.out[0])[g] = s_vx[vrow + lane + j * kVW];
           gp(A.out[1])[g] = s_vz[vrow + lane + j * kVW];
-          gp(A.out[2])[g] = xx[j];
+          gp(A.out[2])[g] = s_xx[srow + lane + (j - 2) * 64];
           gp(A.out[3])[g] = zz[j];
-          gp(A.out[4])[g] = xz[j];
+          gp(A.out[4])[g] = s_xz[srow + lane + j * 64];
         }
     }
   }

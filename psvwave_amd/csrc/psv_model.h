@@ -300,7 +300,8 @@ class Model {
     int4 *blocks = nullptr;
     int *fwd_off = nullptr, *fwd_first = nullptr, *adj_off = nullptr, *adj_first = nullptr;
     int *rec_off = nullptr;
-    InjEntry *fwd = nullptr, *adj = nullptr, *rec = nullptr;
+    InjEntry *fwd = nullptr, *fwd_head = nullptr, *adj = nullptr, *adj_head = nullptr;
+    InjEntry *rec = nullptr;
     int tiles() const { return ntx * ntz; }
   };
   struct LoopJob {

@@ -803,20 +803,16 @@ void Model::release(void *p, size_t bytes) {
 
 // The kernel for `loops` loops side by side: the smallest tiles with which
 // the device holds them all (-1: none).  Small tiles shorten a step, since
-// each wave advances fewer rows.  A single loop on more than one 28-row tile
-// per compute unit runs on 60-row tiles instead where they fit: two blocks
-// of one loop wait for their neighbours at the same time, so the second
-// hides nothing and only adds rim (1800 x 450: 9.3 against 10.1 us per step).
+// each wave advances fewer rows (680 x 380 points: 4.7 us per step on 12-row
+// tiles, 5.7 on 28-row and 7.6 on 60-row ones); two blocks of 28 rows on a
+// compute unit beat one of 60 rows, which waits for its neighbours with the
+// unit idle (1800 x 450: 7.8 against 8.0 us).
 int Model::loop_kind(int loops) {
-  auto fits = [&](int k, int per_cu) {
-    const long long cap = loop_capacity(k);
-    const long long room = cap == 2 * loop_capacity(kNumLoopKinds - 1) ? cap * per_cu / 2 : cap;
-    return ensure_loop_tables(k) && (long long)loops * loop_tables_[k].tiles() <= room;
-  };
   if (d_.nx < 8 || d_.nz < 8) return -1;
   for (int k = 0; k < kNumLoopKinds; ++k)
-    if (fits(k, k == 2 && loops == 1 ? 1 : 2)) return k;
-  return fits(2, 2) ? 2 : -1;
+    if (ensure_loop_tables(k) && (long long)loops * loop_tables_[k].tiles() <= loop_capacity(k))
+      return k;
+  return -1;
 }
 
 // Loops per launch when `limit` may run together: as many as the device
@@ -902,8 +898,14 @@ bool Model::ensure_loop_tables(int kind) {
   std::vector<int> foff, ffirst, aoff, afirst;
   std::vector<InjEntry> fent, aent;
   for (int s = 0; s < cfg_.n_shots; ++s) bucket(forward_terms(s), foff, ffirst, fent);
-  ffirst.push_back((int)fent.size());
   bucket(adjoint_terms(), aoff, afirst, aent);
+  auto heads = [](const std::vector<int> &first, const std::vector<InjEntry> &terms) {
+    std::vector<InjEntry> head;
+    for (int f : first) head.push_back(terms[f]);
+    return head;
+  };
+  const std::vector<InjEntry> fhead = heads(ffirst, fent), ahead = heads(afirst, aent);
+  ffirst.push_back((int)fent.size());
   afirst.push_back((int)aent.size());
   std::vector<int4> blocks;
   const int loops = std::min(std::max(cfg_.n_shots, 1), loop_capacity(kind) / ntiles);
@@ -924,9 +926,11 @@ bool Model::ensure_loop_tables(int kind) {
   put(t.fwd_off, foff);
   put(t.fwd_first, ffirst);
   put(t.fwd, fent);
+  put(t.fwd_head, fhead);
   put(t.adj_off, aoff);
   put(t.adj_first, afirst);
   put(t.adj, aent);
+  put(t.adj_head, ahead);
   put(t.rec_off, roff);
   put(t.rec, rent);
   t.state = 1;
@@ -958,12 +962,14 @@ LoopArgs Model::loop_args(int kind, int i_shot, bool forward) const {
     a.inj_off = t.fwd_off + (size_t)i_shot * (t.tiles() * kLoopKinds[kind].waves + 1);
     a.inj_first = t.fwd_first;
     a.inj = t.fwd;
+    a.inj_head = t.fwd_head;
     a.rec_off = t.rec_off;
     a.rec = t.rec;
   } else {
     a.inj_off = t.adj_off;
     a.inj_first = t.adj_first;
     a.inj = t.adj;
+    a.inj_head = t.adj_head;
   }
   a.stf = b.stf, a.adj_x = b.adj_x, a.adj_z = b.adj_z;
   a.rtf_x = b.rtf_x, a.rtf_z = b.rtf_z;
