@@ -905,8 +905,13 @@ class LoopGate {
     retire(old_);
     retire(before_);
     retire(now_);
-    int sum = need;
-    for (const Entry &e : now_) sum += e.need;
+    // launches of one stream follow each other: each stream counts once, with
+    // its largest
+    std::map<hipStream_t, int> most;
+    for (const Entry &e : now_) most[e.stream] = std::max(most[e.stream], e.need);
+    most[s] = std::max(most[s], need);
+    int sum = 0;
+    for (const auto &m : most) sum += m.second;
     if (sum > 2 * kXcdCus && !now_.empty()) {
       // the launches of now_ themselves wait for those of before_
       old_.insert(old_.end(), before_.begin(), before_.end());

@@ -247,8 +247,11 @@ class Model {
                     std::vector<std::pair<hipEvent_t, hipEvent_t>> *pairs,
                     bool dump);
   void enqueue_checkpointed_adjoint(
-      StepArgs &aa, int i_shot,
-      std::vector<std::pair<hipEvent_t, hipEvent_t>> *pairs);
+      StepArgs &aa, int i_shot, std::vector<std::pair<hipEvent_t, hipEvent_t>> *pairs, int first,
+      int parity);
+  int checkpoint_segments() const;
+  void ensure_segments();
+  void run_checkpointed_resident(int i_shot);
   bool stored_slot(int i_shot, int it, double **dst) const;
   int stored_snapshots() const;
   int ckpt_every_ = 1;
@@ -327,6 +330,7 @@ class Model {
   static constexpr int kLoopSkip = 64;
   void ensure_loop_words();
   bool resident_path(bool dump);
+  void ensure_loop_room(int n, size_t cells, unsigned steps);
   bool ensure_loop_tables(int kind);
   int loop_kind(int loops);
   int loop_group(int limit);

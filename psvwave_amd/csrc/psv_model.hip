@@ -1017,7 +1017,28 @@ void Model::ensure_loop_words() {
                           hipHostMallocDefault),
             "hipHostMalloc");
   std::memset(loop_status_, 0, kLoopStatusWords * sizeof(unsigned));
-  loop_sync_ = (unsigned *)dalloc(1);
+  loop_sync_ = (unsigned *)dalloc(2);  // two words for each stream's launches
+}
+
+// Arguments and exchange cells of n loops, `cells` bytes of cells each, for
+// launches of `steps` steps in all.
+void Model::ensure_loop_room(int n, size_t cells, unsigned steps) {
+  ensure_loop_words();
+  if (loop_args_n_ < n) {
+    release(loop_args_, loop_args_n_ * sizeof(LoopArgs));
+    loop_args_ = (LoopArgs *)dalloc(n * sizeof(LoopArgs) / 8);
+    loop_args_n_ = n;
+  }
+  if (loop_cells_bytes_ < cells * n) {  // new cells are zero: no tag matches
+    release(loop_cells_, loop_cells_bytes_);
+    loop_cells_ = dalloc(cells * n / 8);
+    loop_cells_bytes_ = cells * n;
+    loop_tag_ = 1;
+  } else if (loop_tag_ + steps < loop_tag_) {  // the tags start over
+    hip_check(launch_fill((double *)loop_cells_, (long long)(loop_cells_bytes_ / 8), 0.0, stream_),
+              "clear cells");
+    loop_tag_ = 1;
+  }
 }
 
 void Model::refuse_next_loops() {
@@ -1038,21 +1059,7 @@ void Model::flush_loops() {
   const int kind = loop_kind(n);
   const LoopTables &t = loop_tables_[kind];
   const size_t cells = loop_cells_bytes(kind, t.tiles());
-  ensure_loop_words();
-  if (loop_args_n_ < n) {
-    release(loop_args_, loop_args_n_ * sizeof(LoopArgs));
-    loop_args_ = (LoopArgs *)dalloc(n * sizeof(LoopArgs) / 8);
-    loop_args_n_ = n;
-  }
-  if (loop_cells_bytes_ < cells * n) {  // new cells are zero: no tag matches
-    release(loop_cells_, loop_cells_bytes_);
-    loop_cells_ = dalloc(cells * n / 8);
-    loop_cells_bytes_ = cells * n;
-  } else if (loop_tag_ + (unsigned)cfg_.nt < loop_tag_) {  // the tags start over
-    hip_check(launch_fill((double *)loop_cells_, (long long)(loop_cells_bytes_ / 8), 0.0, stream_),
-              "clear cells");
-    loop_tag_ = 1;
-  }
+  ensure_loop_room(n, cells, (unsigned)cfg_.nt);
   for (int i = 0; i < n; ++i) {
     LoopJob &j = loop_jobs_[first + i];
     j.word = first;
@@ -1184,25 +1191,15 @@ void Model::run_resident(int kind, int i_shot, bool store) {
   settle();
 }
 
-// Adjoint with checkpointing: segments of ckpt_every_ snapshot intervals
-// are processed last to first.  For each, the forward state is restored
-// from the segment's checkpoint into a second buffer pair, the segment's
-// snapshots are recomputed into one of two small buffers (on the second
-// stream, one segment ahead of the adjoint), and the adjoint steps of the
-// segment correlate with them.  The recomputed forward runs the same
-// kernels on the same state, so the kernels equal those of full storage
-// bit for bit.
-void Model::enqueue_checkpointed_adjoint(
-    StepArgs &aa, int i_shot,
-    std::vector<std::pair<hipEvent_t, hipEvent_t>> *pairs) {
-  const int nt = cfg_.nt, si = cfg_.snapshot_interval, k = ckpt_every_;
-  if (!state2_[0][0]) {
-    for (int p = 0; p < 2; ++p)
-      for (int f = 0; f < 5; ++f) state2_[p][f] = dalloc(npad_);
-    // all-zero CSR offsets for the finest tiling (64 x 8 tiles)
-    const long long max_tiles = (long long)ntx_ * ((d_.nz + 7) / 8);
-    scratch_off_ = (int *)dalloc((size_t)(max_tiles + 2) / 2 + 1);
-  }
+int Model::checkpoint_segments() const {
+  const int L = ckpt_every_ * cfg_.snapshot_interval;
+  return (cfg_.nt + L - 1) / L;
+}
+
+// What both ways of a checkpointed adjoint use: segment buffers, the second
+// stream and events.
+void Model::ensure_segments() {
+  const int k = ckpt_every_;
   if (seg_k_ < k) {  // two segment buffers of k snapshot slots
     for (int f = 0; f < 5; ++f) {
       if (seg_[f]) {
@@ -1221,13 +1218,38 @@ void Model::enqueue_checkpointed_adjoint(
     hip_check(hipEventCreateWithFlags(&e, hipEventDisableTiming), "hipEventCreate");
     ckpt_events_.push_back(e);
   }
+}
+
+// Adjoint with checkpointing: segments of ckpt_every_ snapshot intervals
+// are processed last to first.  For each, the forward state is restored
+// from the segment's checkpoint into a second buffer pair, the segment's
+// snapshots are recomputed into one of two small buffers (on the second
+// stream, one segment ahead of the adjoint), and the adjoint steps of the
+// segment correlate with them.  The recomputed forward runs the same
+// kernels on the same state, so the kernels equal those of full storage
+// bit for bit.
+// Segments `first` to 0 are processed; the state before them is zero, or
+// where later segments have been processed in state_[parity].
+void Model::enqueue_checkpointed_adjoint(
+    StepArgs &aa, int i_shot, std::vector<std::pair<hipEvent_t, hipEvent_t>> *pairs, int first,
+    int parity) {
+  const int nt = cfg_.nt, si = cfg_.snapshot_interval, k = ckpt_every_;
+  if (!state2_[0][0]) {
+    for (int p = 0; p < 2; ++p)
+      for (int f = 0; f < 5; ++f) state2_[p][f] = dalloc(npad_);
+    // all-zero CSR offsets for the finest tiling (64 x 8 tiles)
+    const long long max_tiles = (long long)ntx_ * ((d_.nz + 7) / 8);
+    scratch_off_ = (int *)dalloc((size_t)(max_tiles + 2) / 2 + 1);
+  }
+  ensure_segments();
   hipEvent_t ev_start = ckpt_events_[0], ev_join = ckpt_events_[1];
   hipEvent_t ev_ready[2] = {ckpt_events_[2], ckpt_events_[3]};  // segment recomputed
   hipEvent_t ev_done[2] = {ckpt_events_[4], ckpt_events_[5]};   // segment correlated
   const bool inplace = step_is_inplace(variant_);
-  for (int p = 0; p < (inplace ? 1 : 2); ++p)
-    for (int f = 0; f < 5; ++f)
-      hip_check(launch_fill(state_[p][f], npad_, 0.0, stream_), "zero state");
+  if (first == checkpoint_segments() - 1)
+    for (int p = 0; p < (inplace ? 1 : 2); ++p)
+      for (int f = 0; f < 5; ++f)
+        hip_check(launch_fill(state_[p][f], npad_, 0.0, stream_), "zero state");
   hip_check(hipEventRecord(ev_start, stream_), "hipEventRecord");
   hip_check(hipStreamWaitEvent(lane_stream_, ev_start, 0), "hipStreamWaitEvent");
   StepArgs fa = base_args();
@@ -1245,16 +1267,14 @@ void Model::enqueue_checkpointed_adjoint(
   // adjoint steps stay in order on stream_, so the kernels are those of one
   // stream bit for bit.
   const int L = k * si;
-  const int nseg = (nt + L - 1) / L;
-  int parity = 0;
-  for (int c = nseg - 1; c >= 0; --c) {
+  for (int c = first; c >= 0; --c) {
     const int t0 = c * L, t1 = std::min(t0 + L, nt), b = c & 1;
     SlotFn seg = [this, c, k, si, b](int it, double **dst) {
       long long off = ((long long)b * k + (it / si - c * k)) * ngrid_;
       for (int f = 0; f < 5; ++f) dst[f] = seg_[f] + off;
       return true;
     };
-    if (c + 2 < nseg)  // buffer b was read by the adjoint of segment c + 2
+    if (c + 2 <= first)  // buffer b was read by the adjoint of segment c + 2
       hip_check(hipStreamWaitEvent(lane_stream_, ev_done[b], 0), "hipStreamWaitEvent");
     double *ck[5];
     stored_slot(i_shot, t0, ck);
@@ -1271,6 +1291,103 @@ void Model::enqueue_checkpointed_adjoint(
   }
   hip_check(hipEventRecord(ev_join, lane_stream_), "hipEventRecord");
   hip_check(hipStreamWaitEvent(stream_, ev_join, 0), "hipStreamWaitEvent");
+}
+
+// The same on resident loops: a launch per segment and direction, the
+// recomputation of segment c - 1 beside the adjoint of segment c.  With the
+// tiles with which the device holds both at once the pair costs less than one
+// after the other on smaller tiles (a gradient of four shots on 680 x 380
+// points, 4000 steps, snapshots every 10 and a checkpoint every 80: 194
+// against 227 ms; by steps 279); where it holds only one, the gate keeps them
+// apart.  The
+// state of the adjoint passes from launch to launch through state_, in turn
+// from one buffer to the other (a block may end its segment before another
+// has read its part).  After a launch that did not take place none of the
+// later ones does anything, and the remaining segments run step by step.
+void Model::run_checkpointed_resident(int i_shot) {
+  const int nt = cfg_.nt, si = cfg_.snapshot_interval, every = ckpt_every_, L = every * si;
+  const int kind = loop_kind(2) >= 0 ? loop_kind(2) : loop_kind(1);
+  const LoopTables &t = loop_tables_[kind];
+  const size_t cells = loop_cells_bytes(kind, t.tiles());
+  ensure_segments();
+  ensure_loop_room(2, cells, 2u * (unsigned)nt);
+  hipEvent_t ev_start = ckpt_events_[0], ev_join = ckpt_events_[1];
+  hipEvent_t ev_ready[2] = {ckpt_events_[2], ckpt_events_[3]};
+  hipEvent_t ev_done[2] = {ckpt_events_[4], ckpt_events_[5]};
+  // loop 0: the adjoint, on stream_; loop 1: the recomputation, on lane_stream_
+  auto launch = [&](LoopArgs &a, int c, bool fwd, int word) {
+    hipStream_t s = fwd ? lane_stream_ : stream_;
+    const int b = c & 1;
+    for (int f = 0; f < 5; ++f) a.snap[f] = seg_[f] + (long long)b * every * ngrid_;
+    a.slot0 = c * every;
+    a.cells = (char *)loop_cells_ + (fwd ? cells : 0);
+    a.cells_bytes = (unsigned)cells;
+    unsigned *sync_words = loop_sync_ + (fwd ? 2 : 0);
+    hip_check(launch_loop_prepare(loop_args_ + fwd, a, sync_words, s), "prepare loop");
+    LoopLaunch l;
+    l.loops = loop_args_ + fwd;
+    l.blocks = t.blocks;
+    l.nblocks = t.tiles();
+    l.tag0 = loop_tag_;
+    l.sync = sync_words;
+    l.poison = loop_poison_;
+    l.status = loop_status_ + word;
+    gated_launch_loop(kind, !fwd, l, s);
+    loop_tag_ += (unsigned)(a.k1 - a.k0);
+    launches_ += a.k1 - a.k0;
+  };
+  hip_check(hipEventRecord(ev_start, stream_), "hipEventRecord");
+  hip_check(hipStreamWaitEvent(lane_stream_, ev_start, 0), "hipStreamWaitEvent");
+  const int nseg = checkpoint_segments();
+  int parity = 0;
+  for (int c1 = nseg - 1; c1 >= 0;) {
+    const int n = std::min(c1 + 1, kLoopStatusWords / 2);
+    for (int c = c1; c > c1 - n; --c) {
+      const int t0 = c * L, t1 = std::min(t0 + L, nt), b = c & 1, word = 2 * (c1 - c);
+      if (c + 2 <= nseg - 1)  // buffer b was read by the adjoint of segment c + 2
+        hip_check(hipStreamWaitEvent(lane_stream_, ev_done[b], 0), "hipStreamWaitEvent");
+      LoopArgs f = loop_args(kind, i_shot, true);
+      f.rec_off = nullptr;  // the recomputation records no receivers
+      double *ck[5];
+      stored_slot(i_shot, t0, ck);
+      for (int i = 0; i < 5; ++i) f.in[i] = ck[i];
+      f.in_pitch = d_.nx;
+      f.k0 = t0, f.k1 = t1;
+      launch(f, c, true, word);
+      hip_check(hipEventRecord(ev_ready[b], lane_stream_), "hipEventRecord");
+      hip_check(hipStreamWaitEvent(stream_, ev_ready[b], 0), "hipStreamWaitEvent");
+      LoopArgs a = loop_args(kind, i_shot, false);
+      const int p = (parity + c1 - c) & 1;
+      for (int i = 0; i < 5; ++i) {
+        a.in[i] = c < nseg - 1 ? state_[p][i] : nullptr;
+        a.out[i] = state_[1 - p][i];
+      }
+      a.in_pitch = pitch_, a.in_origin = origin_;
+      a.k0 = nt - t1, a.k1 = nt - t0;
+      launch(a, c, false, word + 1);
+      hip_check(hipEventRecord(ev_done[b], stream_), "hipEventRecord");
+    }
+    hip_check(hipEventRecord(ev_join, lane_stream_), "hipEventRecord");
+    hip_check(hipStreamWaitEvent(stream_, ev_join, 0), "hipStreamWaitEvent");
+    sync();
+    const std::vector<unsigned> ran(loop_status_, loop_status_ + 2 * n);
+    std::memset(loop_status_, 0, 2 * n * sizeof(unsigned));
+    int done = 0;
+    for (int i = 0; i < 2 * n; ++i)
+      if (ran[i] == kLoopStalled) throw RuntimeError("a resident time loop made no progress");
+    while (done < n && ran[2 * done] == kLoopRan && ran[2 * done + 1] == kLoopRan) ++done;
+    c1 -= done;
+    parity = (parity + done) & 1;
+    if (done < n) {
+      loop_skip_ = kLoopSkip;
+      hip_check(launch_fill((double *)loop_poison_, 1, 0.0, stream_), "clear poison");
+      StepArgs a = adjoint_args(i_shot);
+      enqueue_checkpointed_adjoint(a, i_shot, nullptr, c1, parity);
+      sync();
+      return;
+    }
+  }
+  loop_skip_ = 0;
 }
 
 // The time loop.  Plain mode launches step by step; graph mode replays a
@@ -1558,12 +1675,18 @@ void Model::adjoint(int i_shot, bool verbose) {
   settle();
   StepArgs a = adjoint_args(i_shot);
   auto t0 = std::chrono::steady_clock::now();
-  if (ckpt_every_ > 1 && timing_stride_ < 0) {
-    timed_loop([&] { enqueue_checkpointed_adjoint(a, i_shot, nullptr); });
+  const int last = checkpoint_segments() - 1;
+  if (ckpt_every_ > 1 && resident_path(false)) {
+    if (timing_stride_ < 0)
+      timed_loop([&] { run_checkpointed_resident(i_shot); });
+    else
+      run_checkpointed_resident(i_shot);
+  } else if (ckpt_every_ > 1 && timing_stride_ < 0) {
+    timed_loop([&] { enqueue_checkpointed_adjoint(a, i_shot, nullptr, last, 0); });
   } else if (ckpt_every_ > 1) {
     std::vector<std::pair<hipEvent_t, hipEvent_t>> pairs;
     event_cursor_ = 0;
-    enqueue_checkpointed_adjoint(a, i_shot, &pairs);
+    enqueue_checkpointed_adjoint(a, i_shot, &pairs, last, 0);
     sync();
     for (auto &p : pairs) {
       float ms = 0.f;

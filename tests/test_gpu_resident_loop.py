@@ -180,6 +180,43 @@ def test_refused_launch_runs_by_steps(every):
     _same(got[:n], _gradient(cfg, 27)[:n], "refused")
 
 
+@pytest.mark.parametrize("nx, nz, nt, si, every, refused", [
+    (131, 77, 60, 5, 5, False),     # 25 + 25 + 10 steps
+    (131, 77, 61, 1, 2, False),     # a last segment of one step
+    (90, 61, 60, 5, 12, False),     # one segment
+    (90, 61, 40, 10, 2, True),
+    (1200, 450, 24, 4, 3, False),   # too large for both directions at once
+])
+def test_checkpointed_segments(nx, nz, nt, si, every, refused):
+    """Segments of a checkpointed adjoint as resident loops that take the
+    state over, against full storage by steps."""
+    import psvwave_amd
+    from psvwave_amd import _lib
+    lib = _lib.load()
+    lib.psv_refuse_resident_loops.argtypes = [C.c_void_p]
+    cfg = _cfg(nx, nz, nt=nt, si=si, shots=2)
+    print(f"[resident] checkpoints {nx}x{nz} {nt} {si} {every}", flush=True)
+    outs = []
+    for variant in (None, 27):
+        m = psvwave_amd.fdModel(cfg)
+        if variant is not None:
+            m.set_step_variant(variant)
+        else:
+            m.set_checkpointing(every)
+        m.set_parameter_fields(*_fields(m, 5))
+        for s in range(2):
+            m.forward_simulate(s)
+        m.calculate_l2_misfit()
+        m.calculate_l2_adjoint_sources()
+        m.reset_kernels()
+        for s in range(2):
+            if refused and variant is None:
+                _lib.check(lib.psv_refuse_resident_loops(m._h))
+            m.adjoint_simulate(s)
+        outs.append([*m.get_synthetic_data(), *m.get_lame_kernels()])
+    _same(*outs, "checkpoints")
+
+
 def test_models_in_threads():
     """Loops of several models from several threads at once: the launches of
     all of them share the device."""
