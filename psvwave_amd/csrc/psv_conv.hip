@@ -84,18 +84,29 @@ __device__ inline void conv_store(const ConvGemm &a, long long pix, int co, floa
     a.out16[o] = to_bf16(v);
 }
 
+// Blocks go to the device's 8 dies (XCDs) in turn, each with an L2 of its own.
+// A kernel numbers its blocks so that those which read the same data follow
+// each other, and this number gives them to one die (3 x 3 layers of a
+// training step 1.43 -> 1.36 ms): launched with a multiple of 8 blocks, those
+// beyond the last exit.
+__device__ inline int xcd_block() { return (blockIdx.x & 7) * (gridDim.x >> 3) + (blockIdx.x >> 3); }
+unsigned xcd_grid(long long blocks) { return (unsigned)((blocks + 7) / 8 * 8); }
+
 // One wavefront computes a (32 WM) x (32 WN) tile of out with
 // v_mfma_f32_32x32x16_bf16: per step of 16 along K each lane loads 16 bytes
-// per 32-row slice of A and of B, and issues WM x WN matrix instructions.
+// per 32-row slice of A and of B, and issues WM x WN matrix instructions.  A
+// small image is bound by the latency of those loads: 2 x 2 scatter of 24 x 40
+// pixels, 128 -> 64 channels: 37 us in 64 x 64 tiles of 15 blocks, 9.5 us in
+// 32 x 32 tiles of 60.
 template <int WM, int WN>
 __global__ void __launch_bounds__(256) conv_mfma_kernel(ConvGemm a) {
   const int lane = threadIdx.x & 63, half = lane >> 5, l32 = lane & 31;
   const int M = a.rows * a.W, N = a.mode == kScatter ? 4 * a.cout : a.cout;
   const int ntaps = a.mode == kGather2x2 ? 4 : a.ks * a.ks, K = ntaps * a.cin;
   const int ntm = (M + 32 * WM - 1) / (32 * WM), ntn = (N + 32 * WN - 1) / (32 * WN);
-  const int tile = blockIdx.x * 4 + (threadIdx.x >> 6);
+  const int tile = xcd_block() * 4 + (threadIdx.x >> 6);
   if (tile >= ntm * ntn) return;  // whole wavefronts exit together
-  const int tm = tile % ntm, tn = tile / ntm;
+  const int tn = tile % ntn, tm = tile / ntn;
   int yg[WM], xx[WM], yi[WM];
   bool mok[WM];
 #pragma unroll
@@ -127,20 +138,20 @@ __global__ void __launch_bounds__(256) conv_mfma_kernel(ConvGemm a) {
 #pragma unroll
       for (int r = 0; r < 16; ++r) acc[i][j][r] = 0.f;
   const bf16x8 zero = {};
-  for (int k0 = 0; k0 < K; k0 += 16) {
+  // A step's loads are issued kAhead steps before its matrix instructions:
+  // far ahead in the small tiles, which few wavefronts run; the large ones
+  // need their registers for wavefronts that hide the latency instead (with
+  // 4 steps 128 x 32 tiles took 480 us a training step, with one 378)
+  constexpr int kAhead = WM * WN == 1 ? 4 : 1;
+  bf16x8 av[kAhead][WM], bv[kAhead][WN];
+  auto load = [&](int s, int k0) {
     const bool kok = tap < ntaps;
-    bf16x8 av[WM], bv[WN];
 #pragma unroll
     for (int i = 0; i < WM; ++i)
-      av[i] = kok && src[i] >= 0 ? *(const bf16x8 *)(a.in + src[i] + ci) : zero;
+      av[s][i] = kok && src[i] >= 0 ? *(const bf16x8 *)(a.in + src[i] + ci) : zero;
 #pragma unroll
     for (int j = 0; j < WN; ++j)
-      bv[j] = kok && nok[j] ? *(const bf16x8 *)(bp[j] + k0) : zero;
-#pragma unroll
-    for (int i = 0; i < WM; ++i)
-#pragma unroll
-      for (int j = 0; j < WN; ++j)
-        acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(av[i], bv[j], acc[i][j], 0, 0, 0);
+      bv[s][j] = kok && nok[j] ? *(const bf16x8 *)(bp[j] + k0) : zero;
     ci += 16;
     if (ci >= a.cin) {
       do {
@@ -151,6 +162,22 @@ __global__ void __launch_bounds__(256) conv_mfma_kernel(ConvGemm a) {
 #pragma unroll
         for (int i = 0; i < WM; ++i)
           src[i] = mok[i] ? conv_src(a, tap, yg[i], xx[i], yi[i]) : -1;
+      }
+    }
+  };
+#pragma unroll
+  for (int s = 0; s < kAhead; ++s) load(s, 16 * s);  // past K: zeros
+  for (int k0 = 0; k0 < K; k0 += 16 * kAhead) {
+#pragma unroll
+    for (int s = 0; s < kAhead; ++s) {
+      if (k0 + 16 * s < K) {
+#pragma unroll
+        for (int i = 0; i < WM; ++i)
+#pragma unroll
+          for (int j = 0; j < WN; ++j)
+            acc[i][j] =
+                __builtin_amdgcn_mfma_f32_32x32x16_bf16(av[s][i], bv[s][j], acc[i][j], 0, 0, 0);
+        load(s, k0 + 16 * (s + kAhead));
       }
     }
   }
@@ -179,71 +206,88 @@ __global__ void __launch_bounds__(256) conv_mfma_kernel(ConvGemm a) {
 
 // 3 x 3 convolution (mode 0, cin a multiple of 16, H a multiple of 4) with
 // the operands staged in LDS.  A block computes 4 output rows x 32 columns
-// x (32 WN) channels; each wavefront one row.  Per 16 input channels the
+// x 32 channels; each wavefront one row.  Per 16 input channels the
 // block loads the input tile with its halo (6 x 34 pixels, zero outside the
 // image) and the weights of all 9 taps for its channels into LDS; the 9
 // taps then read their A fragments from the same tile shifted by (dy, dx),
 // so every input value is fetched from L2 once per block instead of 9 times.
+// What bounds a small image is the chain of load latencies, a large one the
+// LDS traffic: a chunk's loads are all issued together, during the matrix
+// instructions of the chunk before (3 x 3 layers of one 316 x 188 image: 12 to
+// 31 us each before, 10 to 15 so).  32 channels a block, not 64: twice the
+// blocks and half the registers (all 26 layers of a training step on 16 images
+// 1.39 ms against 1.49, inference on one 224 us against 296).
 constexpr int kC3Rows = 4, kC3Cols = 32, kC3TileW = kC3Cols + 2, kC3TileP = (kC3Rows + 2) * kC3TileW;
-template <int WN>
+constexpr int kC3Chan = 32;
 __global__ void __launch_bounds__(256) conv3_lds_kernel(ConvGemm a) {
   __shared__ __attribute__((aligned(16))) uint16_t s_in[kC3TileP * 16];
-  __shared__ __attribute__((aligned(16))) uint16_t s_w[9 * 32 * WN * 16];
+  __shared__ __attribute__((aligned(16))) uint16_t s_w[9 * kC3Chan * 16];
   const int t = threadIdx.x, wave = t >> 6, lane = t & 63, half = lane >> 5, l32 = lane & 31;
-  const int N = a.cout, NB = 32 * WN, K = 9 * a.cin;
-  const int ntn = (N + NB - 1) / NB, ncol = (a.W + kC3Cols - 1) / kC3Cols;
-  const int nt = blockIdx.x % ntn, rest = blockIdx.x / ntn;
+  const int N = a.cout, K = 9 * a.cin;
+  const int ntn = (N + kC3Chan - 1) / kC3Chan, ncol = (a.W + kC3Cols - 1) / kC3Cols;
+  const int block = xcd_block();
+  if (block >= a.rows / kC3Rows * ncol * ntn) return;
+  const int nt = block % ntn, rest = block / ntn;
   const int ct = rest % ncol, band = rest / ncol;
-  const int y0 = band * kC3Rows, x0 = ct * kC3Cols, n0 = nt * NB;
+  const int y0 = band * kC3Rows, x0 = ct * kC3Cols, n0 = nt * kC3Chan;
   const int yi0 = y0 % a.H;  // image row of the band's first row (bands never straddle images)
-  f32x16 acc[WN];
+  f32x16 acc;
 #pragma unroll
-  for (int j = 0; j < WN; ++j)
+  for (int r = 0; r < 16; ++r) acc[r] = 0.f;
+  // this thread's 16-byte pieces of a chunk: source (null: zero) and place
+  constexpr int NI = (kC3TileP * 2 + 255) / 256, NW = (9 * kC3Chan * 2 + 255) / 256;
+  const uint16_t *src_in[NI], *src_w[NW];
 #pragma unroll
-    for (int r = 0; r < 16; ++r) acc[j][r] = 0.f;
+  for (int q = 0; q < NI; ++q) {
+    const int item = t + 256 * q, p = item >> 1, r = p / kC3TileW, c = p - r * kC3TileW;
+    const int yl = yi0 - 1 + r, x = x0 - 1 + c;
+    const bool ok = item < kC3TileP * 2 && yl >= 0 && yl < a.H && x >= 0 && x < a.W;
+    src_in[q] = ok ? a.in + ((long long)(y0 - 1 + r) * a.W + x) * a.in_stride + 8 * (item & 1)
+                   : nullptr;
+  }
+#pragma unroll
+  for (int q = 0; q < NW; ++q) {
+    const int item = t + 256 * q, tn = item >> 1, tap = tn / kC3Chan, n = tn - tap * kC3Chan;
+    const bool ok = item < 9 * kC3Chan * 2 && n0 + n < N;
+    src_w[q] = ok ? a.w + (long long)(n0 + n) * K + tap * a.cin + 8 * (item & 1) : nullptr;
+  }
   const u32x4 zero = {0u, 0u, 0u, 0u};
+  u32x4 vi[NI], vw[NW];
+  auto load = [&](int c0) {
+#pragma unroll
+    for (int q = 0; q < NI; ++q) vi[q] = src_in[q] ? *(const u32x4 *)(src_in[q] + c0) : zero;
+#pragma unroll
+    for (int q = 0; q < NW; ++q) vw[q] = src_w[q] ? *(const u32x4 *)(src_w[q] + c0) : zero;
+  };
+  load(0);
   for (int c0 = 0; c0 < a.cin; c0 += 16) {
     __syncthreads();  // the previous chunk's fragments have been read
-    for (int item = t; item < kC3TileP * 2; item += 256) {
-      const int p = item >> 1, h = item & 1, r = p / kC3TileW, c = p - r * kC3TileW;
-      const int yl = yi0 - 1 + r, x = x0 - 1 + c;
-      u32x4 v = zero;
-      if (yl >= 0 && yl < a.H && x >= 0 && x < a.W)
-        v = *(const u32x4 *)(a.in + ((long long)(y0 - 1 + r) * a.W + x) * a.in_stride + c0 +
-                             8 * h);
-      *(u32x4 *)(s_in + p * 16 + 8 * h) = v;
-    }
-    for (int item = t; item < 9 * NB * 2; item += 256) {
-      const int h = item & 1, tn = item >> 1, tap = tn / NB, n = tn - tap * NB;
-      u32x4 v = zero;
-      if (n0 + n < N)
-        v = *(const u32x4 *)(a.w + (long long)(n0 + n) * K + tap * a.cin + c0 + 8 * h);
-      *(u32x4 *)(s_w + tn * 16 + 8 * h) = v;
-    }
+#pragma unroll
+    for (int q = 0; q < NI; ++q)
+      if (256 * (q + 1) <= kC3TileP * 2 || t + 256 * q < kC3TileP * 2)
+        *(u32x4 *)(s_in + (t + 256 * q) * 8) = vi[q];
+#pragma unroll
+    for (int q = 0; q < NW; ++q)
+      if (256 * (q + 1) <= 9 * kC3Chan * 2 || t + 256 * q < 9 * kC3Chan * 2)
+        *(u32x4 *)(s_w + (t + 256 * q) * 8) = vw[q];
     __syncthreads();
+    if (c0 + 16 < a.cin) load(c0 + 16);
 #pragma unroll
     for (int tap = 0; tap < 9; ++tap) {
       const int dy = tap / 3, dx = tap % 3;
       const bf16x8 av =
           *(const bf16x8 *)(s_in + ((wave + dy) * kC3TileW + l32 + dx) * 16 + 8 * half);
-#pragma unroll
-      for (int j = 0; j < WN; ++j) {
-        const bf16x8 bv = *(const bf16x8 *)(s_w + (tap * NB + 32 * j + l32) * 16 + 8 * half);
-        acc[j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(av, bv, acc[j], 0, 0, 0);
-      }
+      const bf16x8 bv = *(const bf16x8 *)(s_w + (tap * kC3Chan + l32) * 16 + 8 * half);
+      acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(av, bv, acc, 0, 0, 0);
     }
   }
-  const int y = y0 + wave;
+  const int y = y0 + wave, n = n0 + l32;
+  if (n >= N) return;
+  const float b = a.bias ? a.bias[n] : 0.f;
 #pragma unroll
-  for (int j = 0; j < WN; ++j) {
-    const int n = n0 + 32 * j + l32;
-    if (n >= N) continue;
-    const float b = a.bias ? a.bias[n] : 0.f;
-#pragma unroll
-    for (int r = 0; r < 16; ++r) {
-      const int x = x0 + acc_row(r, half);
-      if (x < a.W) conv_store(a, (long long)y * a.W + x, n, acc[j][r] + b);
-    }
+  for (int r = 0; r < 16; ++r) {
+    const int x = x0 + acc_row(r, half);
+    if (x < a.W) conv_store(a, (long long)y * a.W + x, n, acc[r] + b);
   }
 }
 
@@ -253,13 +297,27 @@ __global__ void __launch_bounds__(256) conv3_lds_kernel(ConvGemm a) {
 // fine pixel (2y + q / 2, 2x + q % 2)); R: the layer input gathered as the
 // forward convolution gathers it (j = tap * rc + c, zero outside the image).
 // One wavefront computes a 64 x 64 tile of out.  Per step of 16 pixels each
-// lane loads 16 bytes (8 consecutive channels of one pixel) from two
-// 8-column chunks of L and of R, and writes them transposed into this
-// wavefront's part of LDS ([column][pixel]); the MFMA fragments
-// (8 consecutive pixels of one column) are then single 16-byte LDS reads.
-constexpr int kWgRow = 24;  // LDS row pitch in bf16 (16 pixels + 8 pad): 16-byte aligned rows
+// lane loads 16 bytes (8 consecutive channels) of four consecutive pixels, one
+// half of the lanes of L and the other of R, transposes them in registers and
+// writes them, four pixels of a channel at a time, into this wavefront's part
+// of LDS ([column][pixel]); the MFMA fragments (8 consecutive pixels of one
+// column) are then two 8-byte LDS reads.  The LDS traffic bounds it: rows of
+// 20 values and 16 between L and R put the lanes of every access on different
+// banks.  The next step's loads are in flight meanwhile.  Where rows hold a
+// multiple of 4 pixels (ROW4) a lane's four lie in one row and need one test
+// and one address.  18 layers of a training step on 16 images: 1.70 ms with a
+// pixel per lane, written to LDS value by value; 1.38 so without ROW4, 1.04
+// with it.
+constexpr int kWgRow = 20;                   // LDS row pitch in bf16: 16 pixels + 4
+constexpr int kWgPart = 64 * kWgRow + 16;    // of L, with the shift of R's banks
+typedef unsigned int u32x2 __attribute__((ext_vector_type(2)));
+__device__ inline bf16x8 wgrad_fragment(const uint16_t *p) {
+  const u32x2 lo = *(const u32x2 *)p, hi = *(const u32x2 *)(p + 4);
+  return __builtin_bit_cast(bf16x8, u32x4{lo.x, lo.y, hi.x, hi.y});
+}
+template <bool ROW4>
 __global__ void __launch_bounds__(256) wgrad_mfma_kernel(Wgrad a) {
-  __shared__ __attribute__((aligned(16))) uint16_t lds[4][2][64 * kWgRow];
+  __shared__ __attribute__((aligned(16))) uint16_t lds[4][2 * kWgPart];
   const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, half = lane >> 5, l32 = lane & 31;
   const int nti = (a.I + 63) / 64, ntj = (a.J + 63) / 64;
   const int tile = blockIdx.x * 4 + wave;
@@ -269,24 +327,24 @@ __global__ void __launch_bounds__(256) wgrad_mfma_kernel(Wgrad a) {
   const long long P = (long long)a.rows * a.W;
   const long long p_begin = (long long)s * a.chunk;
   const long long p_end = p_begin + a.chunk < P ? p_begin + a.chunk : P;
-  uint16_t *la = lds[wave][0], *lb = lds[wave][1];
-  // loading role: pixel slot ps of each step, column chunks 2 cg and 2 cg + 1
-  const int ps = lane >> 2, cg = lane & 3;
-  int lq[2], lcol[2], dy[2], dx[2], rcol[2];
-  bool lok[2], rok[2];
-#pragma unroll
-  for (int c = 0; c < 2; ++c) {
-    const int i = i0 + 8 * (2 * cg + c), j = j0 + 8 * (2 * cg + c);
-    lok[c] = i < a.I;
-    lq[c] = a.l_s2d ? i / a.lc : 0;
-    lcol[c] = a.l_s2d ? i - lq[c] * a.lc : i;
-    rok[c] = j < a.J;
-    const int tap = j / a.rc, pad = a.ks / 2;
-    rcol[c] = j - tap * a.rc;
-    dy[c] = tap / a.ks - pad;
-    dx[c] = tap % a.ks - pad;
-  }
-  long long p = p_begin + ps;
+  const uint16_t *const la = lds[wave], *const lb = la + kWgPart;
+  // loading role: pixels 4 g .. 4 g + 3 of each step and columns 8 c .. 8 c + 7
+  // of L (half 0) or R (half 1)
+  const int g = (lane >> 3) & 3, c8 = 8 * (lane & 7);
+  const bool fine = half == 0 && a.l_s2d;  // reads fine pixels
+  const int col = half ? j0 + c8 : i0 + c8;
+  const bool cok = col < (half ? a.J : a.I);
+  const int tap = half ? col / a.rc : 0, pad = a.ks / 2;
+  const int q = fine ? col / a.lc : 0;
+  const int dy = half ? tap / a.ks - pad : 0, dx = half ? tap % a.ks - pad : 0;
+  const int stride = half ? a.r_stride : a.l_stride;
+  // element of pixel p: base + p * stride (fine pixels: see load)
+  const uint16_t *const base =
+      half ? a.r + ((long long)dy * a.W + dx) * stride + (col - tap * a.rc)
+           : a.l + (fine ? ((long long)(q >> 1) * (2 * a.W) + (q & 1)) * stride + (col - q * a.lc)
+                         : col);
+  uint16_t *const to = lds[wave] + half * kWgPart + c8 * kWgRow + 4 * g;
+  long long p = p_begin + 4 * g;
   int yg = (int)(p / a.W), x = (int)(p - (long long)yg * a.W), yi = yg % a.H;
   f32x16 acc[2][2];
 #pragma unroll
@@ -298,48 +356,66 @@ __global__ void __launch_bounds__(256) wgrad_mfma_kernel(Wgrad a) {
   const bool bias_tile = a.bias_out && tj == 0;  // also sums L over the pixels
   float lsum = 0.f;
   const u32x4 zero = {0u, 0u, 0u, 0u};
-  for (long long p0 = p_begin; p0 < p_end; p0 += 16, p += 16) {
-    const bool pok = p < p_end;
-    u32x4 lv[2], rv[2];  // 8 bf16 each, element t in the (t & 1) half of word t / 2
+  u32x4 v[4];  // 8 bf16 of a pixel each, element t in the (t & 1) half of word t / 2
+  const uint16_t *next = base + p * stride;  // of pixel p (not of fine pixels)
+  auto load = [&]() {
+    int xe = x, ye = yi, row = yg;
+    if (ROW4) {  // four pixels of one row
+      const bool ok = cok && p < p_end && yi + dy >= 0 && yi + dy < a.H;
+      const uint16_t *from = next;
+      long long each = stride;
+      if (fine) from = base + (2 * p + 2LL * yg * a.W) * stride, each = 2 * stride;
 #pragma unroll
-    for (int c = 0; c < 2; ++c) {
-      lv[c] = zero;
-      if (pok && lok[c]) {
-        long long li;
-        if (a.l_s2d)
-          li = ((long long)(2 * yg + (lq[c] >> 1)) * (2 * a.W) + 2 * x + (lq[c] & 1)) *
-                   a.l_stride + lcol[c];
-        else
-          li = p * a.l_stride + lcol[c];
-        lv[c] = *(const u32x4 *)(a.l + li);
+      for (int e = 0; e < 4; ++e) {
+        v[e] = zero;
+        if (ok && (e > 0 || x + dx >= 0) && (e < 3 || x + 3 + dx < a.W))
+          v[e] = *(const u32x4 *)(from + e * each);
       }
-      rv[c] = zero;
-      const int yy = yi + dy[c], xx = x + dx[c];
-      if (pok && rok[c] && yy >= 0 && yy < a.H && xx >= 0 && xx < a.W)
-        rv[c] = *(const u32x4 *)(a.r + ((long long)(yg + dy[c]) * a.W + xx) * a.r_stride +
-                                 rcol[c]);
+      next += 16LL * stride;
     }
-    // transpose into LDS: column 8 (2 cg + c) + t, pixel ps
 #pragma unroll
-    for (int c = 0; c < 2; ++c)
-#pragma unroll
-      for (int t = 0; t < 8; ++t) {
-        const int row = 8 * (2 * cg + c) + t;
-        la[row * kWgRow + ps] = (uint16_t)(lv[c][t >> 1] >> (16 * (t & 1)));
-        lb[row * kWgRow + ps] = (uint16_t)(rv[c][t >> 1] >> (16 * (t & 1)));
+    for (int e = 0; !ROW4 && e < 4; ++e) {
+      v[e] = zero;
+      const int yy = ye + dy, xx = xe + dx;
+      if (cok && p + e < p_end && yy >= 0 && yy < a.H && xx >= 0 && xx < a.W)
+        v[e] = *(const u32x4 *)(base + (fine ? 2 * (p + e) + 2LL * row * a.W : p + e) * stride);
+      if (++xe == a.W) {
+        xe = 0;
+        ++row;
+        if (++ye == a.H) ye = 0;
       }
+    }
+    p += 16;
+    x += 16;
+    while (x >= a.W) {
+      x -= a.W;
+      ++yg;
+      if (++yi == a.H) yi = 0;
+    }
+  };
+  load();
+  for (long long p0 = p_begin; p0 < p_end; p0 += 16) {
+    // channel t of the four pixels
+#pragma unroll
+    for (int t = 0; t < 8; ++t) {
+      const unsigned sel = t & 1 ? 0x07060302u : 0x05040100u;  // high or low halves
+      const u32x2 w = {__builtin_amdgcn_perm(v[1][t >> 1], v[0][t >> 1], sel),
+                       __builtin_amdgcn_perm(v[3][t >> 1], v[2][t >> 1], sel)};
+      *(u32x2 *)(to + t * kWgRow) = w;
+    }
+    load();
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
     __builtin_amdgcn_wave_barrier();
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
     bf16x8 af[2], bf[2];
 #pragma unroll
     for (int u = 0; u < 2; ++u) {
-      af[u] = *(const bf16x8 *)(la + (32 * u + l32) * kWgRow + 8 * half);
-      bf[u] = *(const bf16x8 *)(lb + (32 * u + l32) * kWgRow + 8 * half);
+      af[u] = wgrad_fragment(la + (32 * u + l32) * kWgRow + 8 * half);
+      bf[u] = wgrad_fragment(lb + (32 * u + l32) * kWgRow + 8 * half);
     }
     if (bias_tile) {
-      const bf16x8 r0 = *(const bf16x8 *)(la + lane * kWgRow);
-      const bf16x8 r1 = *(const bf16x8 *)(la + lane * kWgRow + 8);
+      const bf16x8 r0 = wgrad_fragment(la + lane * kWgRow);
+      const bf16x8 r1 = wgrad_fragment(la + lane * kWgRow + 8);
       float t0 = 0.f;
 #pragma unroll
       for (int t = 0; t < 8; ++t) t0 += (float)r0[t];
@@ -355,12 +431,6 @@ __global__ void __launch_bounds__(256) wgrad_mfma_kernel(Wgrad a) {
 #pragma unroll
       for (int v = 0; v < 2; ++v)
         acc[u][v] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(af[u], bf[v], acc[u][v], 0, 0, 0);
-    x += 16;
-    while (x >= a.W) {
-      x -= a.W;
-      ++yg;
-      if (++yi == a.H) yi = 0;
-    }
   }
   if (bias_tile && i0 + lane < a.I) a.bias_out[(long long)s * a.I + i0 + lane] = lsum;
   float *out = a.out + (long long)s * a.I * a.J;
@@ -498,23 +568,28 @@ hipError_t launch_conv_gemm(const ConvGemm &a, hipStream_t s) {
   if (((uintptr_t)a.in | (uintptr_t)a.w) & 15) return hipErrorInvalidValue;  // 16-byte loads
   if (a.mode == kConv && a.ks == 3 && a.cin % 16 == 0 && a.H % kC3Rows == 0) {
     const long long blocks = (long long)(a.rows / kC3Rows) * ((a.W + kC3Cols - 1) / kC3Cols);
-    if (a.cout > 32) {
-      hipLaunchKernelGGL(HIP_KERNEL_NAME(conv3_lds_kernel<2>),
-                         dim3((unsigned)(blocks * ((a.cout + 63) / 64))), dim3(256), 0, s, a);
-    } else {
-      hipLaunchKernelGGL(HIP_KERNEL_NAME(conv3_lds_kernel<1>),
-                         dim3((unsigned)(blocks * ((a.cout + 31) / 32))), dim3(256), 0, s, a);
-    }
+    hipLaunchKernelGGL(conv3_lds_kernel,
+                       dim3(xcd_grid(blocks * ((a.cout + kC3Chan - 1) / kC3Chan))), dim3(256), 0,
+                       s, a);
     return hipGetLastError();
   }
   const long long M = (long long)a.rows * a.W, N = a.mode == kScatter ? 4LL * a.cout : a.cout;
-  if (N > 32) {  // 64 x 64 per wavefront
-    const long long tiles = ((M + 63) / 64) * ((N + 63) / 64);
-    hipLaunchKernelGGL(HIP_KERNEL_NAME(conv_mfma_kernel<2, 2>), dim3(blocks_of(tiles, 4)),
+  // 64 x 64 or 128 x 32 per wavefront, which reuses each operand; 32 x 32
+  // where that leaves vector units (four a compute unit) without a wavefront
+  // (2 x 2 scatter of 24 x 40 pixels x 16 images, 128 -> 64 channels: 44 us in
+  // 64 x 64 tiles, 20 in 32 x 32; inference on one 316 x 188 image 324 against
+  // 224 us)
+  const bool wide = N > 32;
+  const long long tiles = wide ? ((M + 63) / 64) * ((N + 63) / 64) : (M + 127) / 128;
+  if (tiles < 1024) {
+    const long long small = ((M + 31) / 32) * ((N + 31) / 32);
+    hipLaunchKernelGGL(HIP_KERNEL_NAME(conv_mfma_kernel<1, 1>), dim3(xcd_grid((small + 3) / 4)),
                        dim3(256), 0, s, a);
-  } else {  // 128 x 32
-    const long long tiles = ((M + 127) / 128) * ((N + 31) / 32);
-    hipLaunchKernelGGL(HIP_KERNEL_NAME(conv_mfma_kernel<4, 1>), dim3(blocks_of(tiles, 4)),
+  } else if (wide) {
+    hipLaunchKernelGGL(HIP_KERNEL_NAME(conv_mfma_kernel<2, 2>), dim3(xcd_grid((tiles + 3) / 4)),
+                       dim3(256), 0, s, a);
+  } else {
+    hipLaunchKernelGGL(HIP_KERNEL_NAME(conv_mfma_kernel<4, 1>), dim3(xcd_grid((tiles + 3) / 4)),
                        dim3(256), 0, s, a);
   }
   return hipGetLastError();
@@ -557,7 +632,12 @@ hipError_t launch_wgrad(Wgrad a, float *dw, float *db, float *workspace,
   a.out = split ? workspace : dw;
   a.bias_out = db ? (split ? workspace + (long long)a.nsplit * n : db) : nullptr;
   const long long tiles = (long long)((a.I + 63) / 64) * ((a.J + 63) / 64) * a.nsplit;
-  hipLaunchKernelGGL(wgrad_mfma_kernel, dim3(blocks_of(tiles, 4)), dim3(256), 0, s, a);
+  if (a.W % 4 == 0)
+    hipLaunchKernelGGL(HIP_KERNEL_NAME(wgrad_mfma_kernel<true>), dim3(blocks_of(tiles, 4)),
+                       dim3(256), 0, s, a);
+  else
+    hipLaunchKernelGGL(HIP_KERNEL_NAME(wgrad_mfma_kernel<false>), dim3(blocks_of(tiles, 4)),
+                       dim3(256), 0, s, a);
   if (split) {
     launch_reduce_splits(workspace, dw, n, a.nsplit, s);
     if (db) launch_reduce_splits(a.bias_out, db, a.I, a.nsplit, s);
