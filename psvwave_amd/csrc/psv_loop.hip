@@ -899,20 +899,26 @@ class LoopGate {
   void launch(int kind, bool adjoint, const LoopLaunch &l, hipStream_t s,
               const LoopDevice &device) {
     std::lock_guard<std::mutex> lock(m_);
-    // in halves of a compute unit of one XCD; blocks go to the XCDs in turn
-    const int need = (l.nblocks + device.xcds - 1) / device.xcds *
-                     (device.per_cu[kind] == 2 ? 1 : 2);
+    // blocks on one XCD (they go to the XCDs in turn), and whether two share a
+    // compute unit
+    const int blocks = (l.nblocks + device.xcds - 1) / device.xcds;
+    const bool half = device.per_cu[kind] == 2;
     retire(old_);
     retire(before_);
     retire(now_);
     // launches of one stream follow each other: each stream counts once, with
-    // its largest
+    // its largest.  Beside blocks that need a whole compute unit every block
+    // counts as one, since those that could share a unit may have one each.
     std::map<hipStream_t, int> most;
-    for (const Entry &e : now_) most[e.stream] = std::max(most[e.stream], e.need);
-    most[s] = std::max(most[s], need);
+    bool halves = half;
+    for (const Entry &e : now_) {
+      most[e.stream] = std::max(most[e.stream], e.blocks);
+      halves = halves && e.half;
+    }
+    most[s] = std::max(most[s], blocks);
     int sum = 0;
     for (const auto &m : most) sum += m.second;
-    if (sum > 2 * kXcdCus && !now_.empty()) {
+    if (sum > (halves ? 2 : 1) * kXcdCus && !now_.empty()) {
       // the launches of now_ themselves wait for those of before_
       old_.insert(old_.end(), before_.begin(), before_.end());
       before_.swap(now_);
@@ -930,7 +936,7 @@ class LoopGate {
     }
     const hipError_t le = launch_loop(kind, adjoint, l, s);
     const hipError_t re = hipEventRecord(end, s);
-    now_.push_back({end, s, need});
+    now_.push_back({end, s, blocks, half});
     check(le, "resident time loop");
     check(re, "hipEventRecord");
   }
@@ -957,7 +963,8 @@ class LoopGate {
   struct Entry {
     hipEvent_t end;
     hipStream_t stream;
-    int need;
+    int blocks;
+    bool half;
   };
   static void check(hipError_t e, const char *what) {
     if (e != hipSuccess) throw RuntimeError(std::string(what) + ": " + hipGetErrorString(e));
