@@ -81,3 +81,75 @@ def test_weight_gradient_tiles(batch, h, w, cin, cout, ks, fine):
     sums = db.cpu().double()
     sums = sums.view(4, cout).sum(0) if fine else sums
     assert torch.equal(sums, dy.sum(dim=(0, 2, 3)))
+
+
+# 8 channels to a store where everything is aligned for it, one value else: the
+# same bits, in each mode, with ragged rows, columns and channels, and with the
+# pre-activation, the activation and the stored derivative
+@pytest.mark.parametrize("h,w,cin,cout,ks,mode", [
+    (8, 33, 32, 40, 3, 0), (4, 1, 16, 8, 3, 0), (5, 37, 16, 24, 3, 0), (365, 360, 8, 24, 3, 0),
+    (9, 7, 8, 72, 1, 0), (257, 255, 24, 40, 1, 0), (9, 5, 40, 8, 1, 1), (130, 128, 16, 24, 1, 1),
+    (6, 5, 16, 40, 1, 2)])
+@pytest.mark.parametrize("f32,fused", [(0, False), (1, False), (0, True)])
+def test_convolution_stores(h, w, cin, cout, ks, mode, f32, fused):
+    import torch
+    from psvwave_amd import _lib
+    lib = _lib.load()
+    print(f"[stores] {h}x{w} {cin}->{cout} ks {ks} mode {mode} f32 {f32} {fused}", flush=True)
+    g = torch.Generator().manual_seed(h * w + cout)
+    taps, up = (ks * ks, 1) if mode < 2 else (4, 2)
+    x = torch.randn(1, up * h, up * w, cin, generator=g).to("cuda", torch.bfloat16)
+    rows = 4 * cout if mode == 1 else cout
+    wt = torch.randn(rows, taps * cin, generator=g).to("cuda", torch.bfloat16)
+    b = torch.randn(cout, generator=g).cuda()
+    oh, ow = (2 * h, 2 * w) if mode == 1 else (h, w)
+    z = torch.randn(oh, ow, cout, generator=g).to("cuda", torch.bfloat16)
+    results = []
+    for off in (8, 4):  # in 16-byte accesses; value by value
+        stride = cout + 16
+        out = torch.full((oh, ow, stride), 7.0, device="cuda",
+                         dtype=torch.float32 if f32 else torch.bfloat16)
+        pre = torch.zeros(oh, ow, cout, device="cuda", dtype=torch.bfloat16)
+        _lib.check(lib.psv_conv_bf16(
+            x.data_ptr(), cin, wt.data_ptr(), b.data_ptr(), out.data_ptr(), f32, stride, off,
+            pre.data_ptr() if fused and mode == 0 else 0, z.data_ptr() if fused else 0, cout, 1, h,
+            w, cin, cout, ks, mode, int(fused), torch.cuda.current_stream().cuda_stream))
+        assert (out[..., :off] == 7).all() and (out[..., off + cout:] == 7).all()
+        results.append((out[..., off:off + cout].float().cpu(), pre.float().cpu()))
+    assert torch.equal(results[0][0], results[1][0])
+    assert torch.equal(results[0][1], results[1][1])
+
+
+@pytest.mark.parametrize("h,w,c", [(2, 2, 8), (6, 10, 24), (34, 62, 40), (2, 130, 64)])
+def test_pooling_in_wide_accesses(h, w, c):
+    import torch
+    from psvwave_amd import _lib
+    lib = _lib.load()
+    print(f"[pool] {h}x{w}x{c}", flush=True)
+    g = torch.Generator().manual_seed(h * w + c)
+    stream = torch.cuda.current_stream().cuda_stream
+    a = _ints(g, h, w, c).to("cuda", torch.bfloat16)  # with ties
+    room = torch.zeros(h * w * c + 8, device="cuda", dtype=torch.bfloat16)
+    shifted = room[4:4 + h * w * c].view(h, w, c)  # 8 bytes off: value by value
+    shifted.copy_(a)
+    pooled = []
+    for t in (a, shifted):
+        out = torch.zeros(h // 2, w // 2, c, device="cuda", dtype=torch.bfloat16)
+        _lib.check(lib.psv_maxpool2_bf16(t.data_ptr(), out.data_ptr(), h, w, c, stream))
+        pooled.append(out.cpu())
+    ref = torch.nn.functional.max_pool2d(a.float().cpu().permute(2, 0, 1)[None], 2)[0]
+    assert torch.equal(pooled[0].float().permute(2, 0, 1), ref)
+    assert torch.equal(pooled[0], pooled[1])
+    z = torch.randn(h, w, c, generator=g).to("cuda", torch.bfloat16)
+    d = torch.randn(h // 2, w // 2, c, generator=g).cuda()
+    skip = torch.randn(h, w, 2 * c, generator=g).to("cuda", torch.bfloat16)
+    for dpool, dskip in ((d, skip), (d, None), (None, skip)):
+        grads = []
+        for t in (a, shifted):
+            out = torch.zeros(h, w, c, device="cuda", dtype=torch.bfloat16)
+            _lib.check(lib.psv_maxpool2_backward_bf16(
+                t.data_ptr(), z.data_ptr(), 0 if dpool is None else dpool.data_ptr(),
+                0 if dskip is None else dskip.data_ptr(), 2 * c, c, out.data_ptr(), 1, h, w, c,
+                stream))
+            grads.append(out.float().cpu())
+        assert torch.equal(grads[0], grads[1])
