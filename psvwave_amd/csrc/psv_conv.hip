@@ -319,12 +319,20 @@ __global__ void __launch_bounds__(256) conv_mfma_kernel(ConvGemm a) {
 // 31 us each before, 10 to 15 so).  32 channels a block, not 64: twice the
 // blocks and half the registers (all 26 layers of a training step on 16 images
 // 1.39 ms against 1.49, inference on one 224 us against 296).
-constexpr int kC3Rows = 4, kC3Cols = 32, kC3TileW = kC3Cols + 2, kC3TileP = (kC3Rows + 2) * kC3TileW;
-constexpr int kC3Chan = 32;
-template <bool STORE8>
+// With R = 2 rows a wavefront a value read from LDS serves two products more
+// often (21 fragments for 18 instead of 36) and a block loads half the weights
+// per row: 928 -> 893 us for the 26 layers of a training step, together with
+// the operands' places free of bank conflicts.  What is left is vector issue,
+// three quarters of the time: the activation, its derivative and the stores.
+constexpr int kC3Cols = 32, kC3TileW = kC3Cols + 2, kC3Chan = 32;
+template <bool STORE8, int R>
 __global__ void __launch_bounds__(256) conv3_lds_kernel(ConvGemm a) {
   // the input tile and the weights, then the tiles of the four wavefronts
-  constexpr int kIn = kC3TileP * 16, kBytes = 2 * (kIn + 9 * kC3Chan * 16);
+  constexpr int kC3Rows = 4 * R, kC3TileP = (kC3Rows + 2) * kC3TileW;
+  // (each of channels 0 .. 7 of all pixels, then 8 .. 15, so that neighbouring
+  // lanes read and write neighbouring 16 bytes)
+  constexpr int kInHalf = kC3TileP * 8, kWHalf = 9 * kC3Chan * 8 + 32;
+  constexpr int kIn = 2 * kInHalf, kBytes = 2 * (kIn + 2 * kWHalf);
   constexpr int kTurnBytes = STORE8 ? 4 * 4 * 32 * kTurnPitch : 0;
   __shared__ __attribute__((aligned(16))) char s_mem[kBytes > kTurnBytes ? kBytes : kTurnBytes];
   uint16_t *const s_in = (uint16_t *)s_mem, *const s_w = s_in + kIn;
@@ -337,9 +345,11 @@ __global__ void __launch_bounds__(256) conv3_lds_kernel(ConvGemm a) {
   const int ct = rest % ncol, band = rest / ncol;
   const int y0 = band * kC3Rows, x0 = ct * kC3Cols, n0 = nt * kC3Chan;
   const int yi0 = y0 % a.H;  // image row of the band's first row (bands never straddle images)
-  f32x16 acc;
+  f32x16 acc[R];
 #pragma unroll
-  for (int r = 0; r < 16; ++r) acc[r] = 0.f;
+  for (int j = 0; j < R; ++j)
+#pragma unroll
+    for (int r = 0; r < 16; ++r) acc[j][r] = 0.f;
   // this thread's 16-byte pieces of a chunk: source (null: zero) and place
   constexpr int NI = (kC3TileP * 2 + 255) / 256, NW = (9 * kC3Chan * 2 + 255) / 256;
   const uint16_t *src_in[NI], *src_w[NW];
@@ -371,39 +381,52 @@ __global__ void __launch_bounds__(256) conv3_lds_kernel(ConvGemm a) {
 #pragma unroll
     for (int q = 0; q < NI; ++q)
       if (256 * (q + 1) <= kC3TileP * 2 || t + 256 * q < kC3TileP * 2)
-        *(u32x4 *)(s_in + (t + 256 * q) * 8) = vi[q];
+        *(u32x4 *)(s_in + (t & 1) * kInHalf + ((t + 256 * q) >> 1) * 8) = vi[q];
 #pragma unroll
     for (int q = 0; q < NW; ++q)
       if (256 * (q + 1) <= 9 * kC3Chan * 2 || t + 256 * q < 9 * kC3Chan * 2)
-        *(u32x4 *)(s_w + (t + 256 * q) * 8) = vw[q];
+        *(u32x4 *)(s_w + (t & 1) * kWHalf + ((t + 256 * q) >> 1) * 8) = vw[q];
     __syncthreads();
     if (c0 + 16 < a.cin) load(c0 + 16);
+    bf16x8 av[R + 2][3];
 #pragma unroll
-    for (int tap = 0; tap < 9; ++tap) {
-      const int dy = tap / 3, dx = tap % 3;
-      const bf16x8 av =
-          *(const bf16x8 *)(s_in + ((wave + dy) * kC3TileW + l32 + dx) * 16 + 8 * half);
-      const bf16x8 bv = *(const bf16x8 *)(s_w + (tap * kC3Chan + l32) * 16 + 8 * half);
-      acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(av, bv, acc, 0, 0, 0);
+    for (int dy = 0; dy < 3; ++dy) {
+#pragma unroll
+      for (int j = dy == 0 ? 0 : R + dy - 1; j < R + dy; ++j)
+#pragma unroll
+        for (int dx = 0; dx < 3; ++dx)
+          av[j][dx] = *(const bf16x8 *)(s_in + half * kInHalf + ((wave * R + j) * kC3TileW + l32 + dx) * 8);
+#pragma unroll
+      for (int dx = 0; dx < 3; ++dx) {
+        const bf16x8 bv =
+            *(const bf16x8 *)(s_w + half * kWHalf + ((3 * dy + dx) * kC3Chan + l32) * 8);
+#pragma unroll
+        for (int j = 0; j < R; ++j)
+          acc[j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(av[j + dy][dx], bv, acc[j], 0, 0, 0);
+      }
     }
   }
-  const int y = y0 + wave, n = n0 + l32;
+  const int y = y0 + wave * R, n = n0 + l32;
   if (STORE8) {
     __syncthreads();  // the operands have been read
-    turn_tile((float *)s_mem + wave * 32 * kTurnPitch, acc, a.bias && n < N ? a.bias[n] : 0.f, lane,
-              [&](int row, int c, float *v) {
-                if (x0 + row < a.W && n0 + c < N)
-                  conv_store8(a, (long long)y * a.W + x0 + row, n0 + c, v);
-              });
+#pragma unroll
+    for (int j = 0; j < R; ++j)
+      turn_tile((float *)s_mem + wave * 32 * kTurnPitch, acc[j], a.bias && n < N ? a.bias[n] : 0.f,
+                lane, [&](int row, int c, float *v) {
+                  if (x0 + row < a.W && n0 + c < N)
+                    conv_store8(a, (long long)(y + j) * a.W + x0 + row, n0 + c, v);
+                });
     return;
   }
   if (n >= N) return;
   const float b = a.bias ? a.bias[n] : 0.f;
 #pragma unroll
-  for (int r = 0; r < 16; ++r) {
-    const int x = x0 + acc_row(r, half);
-    if (x < a.W) conv_store(a, (long long)y * a.W + x, n, acc[r] + b);
-  }
+  for (int j = 0; j < R; ++j)
+#pragma unroll
+    for (int r = 0; r < 16; ++r) {
+      const int x = x0 + acc_row(r, half);
+      if (x < a.W) conv_store(a, (long long)(y + j) * a.W + x, n, acc[j][r] + b);
+    }
 }
 
 // Weight gradient: out[s][i][j] = sum over pixels p of split s of
@@ -411,61 +434,77 @@ __global__ void __launch_bounds__(256) conv3_lds_kernel(ConvGemm a) {
 // (l_s2d = 0: L[p][i] = l[p * l_stride + i]; l_s2d = 1: i = q * lc + c reads
 // fine pixel (2y + q / 2, 2x + q % 2)); R: the layer input gathered as the
 // forward convolution gathers it (j = tap * rc + c, zero outside the image).
-// One wavefront computes a 64 x 64 tile of out.  Per step of 16 pixels each
-// lane loads 16 bytes (8 consecutive channels) of four consecutive pixels, one
-// half of the lanes of L and the other of R, transposes them in registers and
+// A block computes a tile of out, 64 x 64 or 32 x 96, each of its wavefronts
+// a quarter of the split's pixels, added up in LDS in the end (a fourth of the
+// partial sums to write and read again).  Per step of 16 pixels each
+// lane loads 16 bytes (8 consecutive channels) of four consecutive pixels, of
+// one of the tile's 16 groups of 8 columns of L or R, transposes them in registers and
 // writes them, four pixels of a channel at a time, into this wavefront's part
 // of LDS ([column][pixel]); the MFMA fragments (8 consecutive pixels of one
-// column) are then two 8-byte LDS reads.  The LDS traffic bounds it: rows of
-// 20 values and 16 between L and R put the lanes of every access on different
-// banks.  The next step's loads are in flight meanwhile.  Where rows hold a
-// multiple of 4 pixels (ROW4) a lane's four lie in one row and need one test
-// and one address.  18 layers of a training step on 16 images: 1.70 ms with a
-// pixel per lane, written to LDS value by value; 1.38 so without ROW4, 1.04
-// with it.
+// column) are then two 8-byte LDS reads, all free of bank conflicts.  The next
+// step's loads are in flight meanwhile.  Where rows hold a multiple of 4 pixels
+// (ROW4) a lane's four lie in one row and need one test and one address.
+// 18 layers of a training step on 16 images: 1.70 ms with a pixel per lane,
+// written to LDS value by value; 1.38 so without ROW4, 1.04 with it; 0.86 with
+// the flat tile and conflict-free writes (before, LDS was busy 83 % of the time,
+// most of it with conflicts), and 0.33 -> 0.20 ms for the partial sums' addition.
 constexpr int kWgRow = 20;                   // LDS row pitch in bf16: 16 pixels + 4
-constexpr int kWgPart = 64 * kWgRow + 16;    // of L, with the shift of R's banks
 typedef unsigned int u32x2 __attribute__((ext_vector_type(2)));
+// LDS place of a column: in every other 16 columns the two halves of 8 change
+// places, so that the 16 lanes whose writes go together (4 groups of 8 columns
+// by 4 of pixels) reach all banks; reads of 16 columns do in any case.
+__device__ inline int wgrad_row(int col) { return (col ^ ((col >> 2) & 4)) * kWgRow; }
 __device__ inline bf16x8 wgrad_fragment(const uint16_t *p) {
   const u32x2 lo = *(const u32x2 *)p, hi = *(const u32x2 *)(p + 4);
   return __builtin_bit_cast(bf16x8, u32x4{lo.x, lo.y, hi.x, hi.y});
 }
-template <bool ROW4>
-__global__ void __launch_bounds__(256) wgrad_mfma_kernel(Wgrad a) {
-  __shared__ __attribute__((aligned(16))) uint16_t lds[4][2 * kWgPart];
+template <bool ROW4, int U, int V>
+__global__ void __launch_bounds__(256, U == 2 ? 3 : 4) wgrad_mfma_kernel(Wgrad a) {
+  static_assert(4 * (U + V) == 16, "a lane for every group of columns and pixels");
+  constexpr int kPart = 32 * U * kWgRow, kWave = kPart + 32 * V * kWgRow;
+  __shared__ __attribute__((aligned(16))) uint16_t lds[4 * kWave];
+  __shared__ float s_bias[4][32 * U];
+  static_assert(sizeof(lds) >= 3 * 64 * 16 * sizeof(float), "a 32 x 32 tile of three wavefronts");
   const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, half = lane >> 5, l32 = lane & 31;
-  const int nti = (a.I + 63) / 64, ntj = (a.J + 63) / 64;
-  const int tile = blockIdx.x * 4 + wave;
-  if (tile >= nti * ntj * a.nsplit) return;  // whole wavefronts exit together
+  const int nti = (a.I + 32 * U - 1) / (32 * U), ntj = (a.J + 32 * V - 1) / (32 * V);
+  // the tiles of a split, which read the same pixels, on one die
+  const int tile = xcd_block();
+  if (tile >= nti * ntj * a.nsplit) return;
   const int ti = tile % nti, tj = (tile / nti) % ntj, s = tile / (nti * ntj);
-  const int i0 = ti * 64, j0 = tj * 64;
+  const int i0 = ti * 32 * U, j0 = tj * 32 * V;
   const long long P = (long long)a.rows * a.W;
-  const long long p_begin = (long long)s * a.chunk;
-  const long long p_end = p_begin + a.chunk < P ? p_begin + a.chunk : P;
-  const uint16_t *const la = lds[wave], *const lb = la + kWgPart;
+  const long long p_begin = (long long)s * a.chunk + wave * (a.chunk / 4);
+  const long long p_stop = p_begin + a.chunk / 4;
+  const long long p_end = p_stop < P ? p_stop : P;
+  uint16_t *const mine = lds + wave * kWave;
+  const uint16_t *const la = mine, *const lb = la + kPart;
   // loading role: pixels 4 g .. 4 g + 3 of each step and columns 8 c .. 8 c + 7
-  // of L (half 0) or R (half 1)
-  const int g = (lane >> 3) & 3, c8 = 8 * (lane & 7);
-  const bool fine = half == 0 && a.l_s2d;  // reads fine pixels
-  const int col = half ? j0 + c8 : i0 + c8;
-  const bool cok = col < (half ? a.J : a.I);
-  const int tap = half ? col / a.rc : 0, pad = a.ks / 2;
+  // of L or R
+  const bool of_r = lane >= 16 * U;
+  const int li = of_r ? lane - 16 * U : lane;
+  const int g = (li >> 2) & 3, c8 = 8 * ((li & 3) + 4 * (li >> 4));
+  const bool fine = !of_r && a.l_s2d;  // reads fine pixels
+  const int col = of_r ? j0 + c8 : i0 + c8;
+  const bool cok = col < (of_r ? a.J : a.I);
+  const int tap = of_r ? col / a.rc : 0, pad = a.ks / 2;
   const int q = fine ? col / a.lc : 0;
-  const int dy = half ? tap / a.ks - pad : 0, dx = half ? tap % a.ks - pad : 0;
-  const int stride = half ? a.r_stride : a.l_stride;
+  const int dy = of_r ? tap / a.ks - pad : 0, dx = of_r ? tap % a.ks - pad : 0;
+  const int stride = of_r ? a.r_stride : a.l_stride;
   // element of pixel p: base + p * stride (fine pixels: see load)
   const uint16_t *const base =
-      half ? a.r + ((long long)dy * a.W + dx) * stride + (col - tap * a.rc)
+      of_r ? a.r + ((long long)dy * a.W + dx) * stride + (col - tap * a.rc)
            : a.l + (fine ? ((long long)(q >> 1) * (2 * a.W) + (q & 1)) * stride + (col - q * a.lc)
                          : col);
-  uint16_t *const to = lds[wave] + half * kWgPart + c8 * kWgRow + 4 * g;
+  // its columns 0 .. 3 and 4 .. 7 of the 8
+  uint16_t *const at = mine + (of_r ? kPart : 0) + 4 * g;
+  uint16_t *const to[2] = {at + wgrad_row(c8), at + wgrad_row(c8 + 4)};
   long long p = p_begin + 4 * g;
   int yg = (int)(p / a.W), x = (int)(p - (long long)yg * a.W), yi = yg % a.H;
-  f32x16 acc[2][2];
+  f32x16 acc[U][V];
 #pragma unroll
-  for (int u = 0; u < 2; ++u)
+  for (int u = 0; u < U; ++u)
 #pragma unroll
-    for (int v = 0; v < 2; ++v)
+    for (int v = 0; v < V; ++v)
 #pragma unroll
       for (int r = 0; r < 16; ++r) acc[u][v][r] = 0.f;
   const bool bias_tile = a.bias_out && tj == 0;  // also sums L over the pixels
@@ -516,21 +555,20 @@ __global__ void __launch_bounds__(256) wgrad_mfma_kernel(Wgrad a) {
       const unsigned sel = t & 1 ? 0x07060302u : 0x05040100u;  // high or low halves
       const u32x2 w = {__builtin_amdgcn_perm(v[1][t >> 1], v[0][t >> 1], sel),
                        __builtin_amdgcn_perm(v[3][t >> 1], v[2][t >> 1], sel)};
-      *(u32x2 *)(to + t * kWgRow) = w;
+      *(u32x2 *)(to[t >> 2] + (t & 3) * kWgRow) = w;
     }
     load();
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
     __builtin_amdgcn_wave_barrier();
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-    bf16x8 af[2], bf[2];
+    bf16x8 af[U], bf[V];
 #pragma unroll
-    for (int u = 0; u < 2; ++u) {
-      af[u] = wgrad_fragment(la + (32 * u + l32) * kWgRow + 8 * half);
-      bf[u] = wgrad_fragment(lb + (32 * u + l32) * kWgRow + 8 * half);
-    }
+    for (int u = 0; u < U; ++u) af[u] = wgrad_fragment(la + wgrad_row(32 * u + l32) + 8 * half);
+#pragma unroll
+    for (int u = 0; u < V; ++u) bf[u] = wgrad_fragment(lb + wgrad_row(32 * u + l32) + 8 * half);
     if (bias_tile) {
-      const bf16x8 r0 = wgrad_fragment(la + lane * kWgRow);
-      const bf16x8 r1 = wgrad_fragment(la + lane * kWgRow + 8);
+      const bf16x8 r0 = wgrad_fragment(la + wgrad_row(lane & (32 * U - 1)));
+      const bf16x8 r1 = wgrad_fragment(la + wgrad_row(lane & (32 * U - 1)) + 8);
       float t0 = 0.f;
 #pragma unroll
       for (int t = 0; t < 8; ++t) t0 += (float)r0[t];
@@ -542,25 +580,46 @@ __global__ void __launch_bounds__(256) wgrad_mfma_kernel(Wgrad a) {
     __builtin_amdgcn_wave_barrier();  // the next step overwrites this wavefront's LDS rows
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 #pragma unroll
-    for (int u = 0; u < 2; ++u)
+    for (int u = 0; u < U; ++u)
 #pragma unroll
-      for (int v = 0; v < 2; ++v)
+      for (int v = 0; v < V; ++v)
         acc[u][v] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(af[u], bf[v], acc[u][v], 0, 0, 0);
   }
-  if (bias_tile && i0 + lane < a.I) a.bias_out[(long long)s * a.I + i0 + lane] = lsum;
+  // the four wavefronts' sums, added in their order: each 32 x 32 part by one
+  // of them, the others' values through LDS
+  if (bias_tile && lane < 32 * U) s_bias[wave][lane] = lsum;
   float *out = a.out + (long long)s * a.I * a.J;
+  float *const part = (float *)lds;
 #pragma unroll
-  for (int v = 0; v < 2; ++v) {
-    const int j = j0 + 32 * v + l32;
-    if (j >= a.J) continue;
+  for (int u = 0; u < U; ++u)
 #pragma unroll
-    for (int u = 0; u < 2; ++u)
+    for (int v = 0; v < V; ++v) {
+      const int owner = (u * V + v) & 3;
+      __syncthreads();  // the operands, or the part before, have been read
+      if (wave != owner) {
+        float *const to = part + ((wave - owner - 1) & 3) * 1024 + lane;
+#pragma unroll
+        for (int r = 0; r < 16; ++r) to[64 * r] = acc[u][v][r];
+      }
+      __syncthreads();
+      if (wave != owner) continue;
+      const int j = j0 + 32 * v + l32;
 #pragma unroll
       for (int r = 0; r < 16; ++r) {
+        float sum = 0.f;
+#pragma unroll
+        for (int w = 0; w < 4; ++w) {
+          const float x =
+              w == owner ? acc[u][v][r] : part[((w - owner - 1) & 3) * 1024 + 64 * r + lane];
+          sum = w == 0 ? x : sum + x;
+        }
         const int ii = i0 + 32 * u + acc_row(r, half);
-        if (ii < a.I) out[(long long)ii * a.J + j] = acc[u][v][r];
+        if (ii < a.I && j < a.J) out[(long long)ii * a.J + j] = sum;
       }
-  }
+    }
+  if (bias_tile && wave == 0 && lane < 32 * U && i0 + lane < a.I)
+    a.bias_out[(long long)s * a.I + i0 + lane] =
+        ((s_bias[0][lane] + s_bias[1][lane]) + s_bias[2][lane]) + s_bias[3][lane];
 }
 
 // out[e] = sum over s < nsplit of part[s * n + e]: `so` split lanes per
@@ -748,6 +807,8 @@ __global__ void __launch_bounds__(256)
   }
 }
 
+constexpr long long kC3TwoRows = 1024;  // blocks of two rows a wavefront
+
 unsigned blocks_of(long long n, int per) { return (unsigned)((n + per - 1) / per); }
 
 }  // namespace
@@ -760,11 +821,20 @@ hipError_t launch_conv_gemm(const ConvGemm &a, hipStream_t s) {
     return hipErrorInvalidValue;
   if (((uintptr_t)a.in | (uintptr_t)a.w) & 15) return hipErrorInvalidValue;  // 16-byte loads
   const bool store8 = conv_stores8(a);
-  if (a.mode == kConv && a.ks == 3 && a.cin % 16 == 0 && a.H % kC3Rows == 0) {
-    const long long blocks = (long long)(a.rows / kC3Rows) * ((a.W + kC3Cols - 1) / kC3Cols);
-    hipLaunchKernelGGL(store8 ? conv3_lds_kernel<true> : conv3_lds_kernel<false>,
-                       dim3(xcd_grid(blocks * ((a.cout + kC3Chan - 1) / kC3Chan))), dim3(256), 0,
-                       s, a);
+  if (a.mode == kConv && a.ks == 3 && a.cin % 16 == 0 && a.H % 4 == 0) {
+    // two rows a wavefront where bands of 8 rows lie within an image and their
+    // blocks still fill the device, four to a compute unit (with 16 images of
+    // 316 x 188 the two finer levels; the coarser ones keep twice the blocks)
+    const long long blocks = (long long)(a.rows / 4) * ((a.W + kC3Cols - 1) / kC3Cols) *
+                             ((a.cout + kC3Chan - 1) / kC3Chan);
+    const bool two = a.H % 8 == 0 && blocks >= 2 * kC3TwoRows;
+    auto launch = [&](auto kernel, auto kernel8, long long n) {
+      hipLaunchKernelGGL(store8 ? kernel8 : kernel, dim3(xcd_grid(n)), dim3(256), 0, s, a);
+    };
+    if (two)
+      launch(conv3_lds_kernel<false, 2>, conv3_lds_kernel<true, 2>, blocks / 2);
+    else
+      launch(conv3_lds_kernel<false, 1>, conv3_lds_kernel<true, 1>, blocks);
     return hipGetLastError();
   }
   const long long M = (long long)a.rows * a.W, N = a.mode == kScatter ? 4LL * a.cout : a.cout;
@@ -796,20 +866,34 @@ static void launch_reduce_splits(const float *part, float *out, long long n, int
                      part, out, n, nsplit, so);
 }
 
-static long long wgrad_plan(Wgrad &a, long long workspace_floats) {
+// Tile and splits.  A step costs a block the same in either tile, so the one
+// that covers out in fewer is taken: 32 x 96 for up to 32 channels (32 x 288
+// in 3 tiles instead of 5, half of which would be empty), mostly 64 x 64 else.
+// As many blocks as the device's 256 compute units hold at once (four, three of
+// the square tile, which needs more registers: with four of it, spilling, its
+// layers took 36 and 110 us where they now take 28 and 97), of at least 512
+// pixels a wavefront.
+struct WgradPlan {
+  bool flat;  // 32 x 96
+  long long tiles;
+};
+static WgradPlan wgrad_plan(Wgrad &a, long long workspace_floats) {
   const long long P = (long long)a.rows * a.W;
-  const long long tiles = (long long)((a.I + 63) / 64) * ((a.J + 63) / 64);
-  long long ns = (2048 + tiles - 1) / tiles;
-  const long long max_ns = (P + 511) / 512;
+  const long long square = (long long)((a.I + 63) / 64) * ((a.J + 63) / 64);
+  const long long flat = (long long)((a.I + 31) / 32) * ((a.J + 95) / 96);
+  const long long tiles = flat <= square ? flat : square;
+  const long long blocks = flat <= square ? 1024 : 768;
+  long long ns = (blocks + tiles - 1) / tiles;
+  const long long max_ns = (P + 2047) / 2048;
   if (ns > max_ns) ns = max_ns;
   const long long fit = workspace_floats / ((long long)a.I * a.J + a.I);
   if (ns > fit) ns = fit;
   if (ns < 1) ns = 1;
   long long chunk = (P + ns - 1) / ns;
-  chunk = (chunk + 15) / 16 * 16;
+  chunk = (chunk + 63) / 64 * 64;
   a.nsplit = (int)((P + chunk - 1) / chunk);
   a.chunk = chunk;
-  return a.nsplit;
+  return {flat <= square, tiles * a.nsplit};
 }
 
 hipError_t launch_wgrad(Wgrad a, float *dw, float *db, float *workspace,
@@ -819,18 +903,18 @@ hipError_t launch_wgrad(Wgrad a, float *dw, float *db, float *workspace,
       a.l_stride % 8 || a.r_stride % 8 || (((uintptr_t)a.l | (uintptr_t)a.r) & 15) ||
       (a.l_s2d && (a.lc <= 0 || a.lc % 8 || a.I != 4 * a.lc)))
     return hipErrorInvalidValue;
-  wgrad_plan(a, workspace ? workspace_floats : 0);
+  const WgradPlan plan = wgrad_plan(a, workspace ? workspace_floats : 0);
   const long long n = (long long)a.I * a.J;
   const bool split = a.nsplit > 1;
   a.out = split ? workspace : dw;
   a.bias_out = db ? (split ? workspace + (long long)a.nsplit * n : db) : nullptr;
-  const long long tiles = (long long)((a.I + 63) / 64) * ((a.J + 63) / 64) * a.nsplit;
+  auto launch = [&](auto square, auto flat) {
+    hipLaunchKernelGGL(plan.flat ? flat : square, dim3(xcd_grid(plan.tiles)), dim3(256), 0, s, a);
+  };
   if (a.W % 4 == 0)
-    hipLaunchKernelGGL(HIP_KERNEL_NAME(wgrad_mfma_kernel<true>), dim3(blocks_of(tiles, 4)),
-                       dim3(256), 0, s, a);
+    launch(wgrad_mfma_kernel<true, 2, 2>, wgrad_mfma_kernel<true, 1, 3>);
   else
-    hipLaunchKernelGGL(HIP_KERNEL_NAME(wgrad_mfma_kernel<false>), dim3(blocks_of(tiles, 4)),
-                       dim3(256), 0, s, a);
+    launch(wgrad_mfma_kernel<false, 2, 2>, wgrad_mfma_kernel<false, 1, 3>);
   if (split) {
     launch_reduce_splits(workspace, dw, n, a.nsplit, s);
     if (db) launch_reduce_splits(a.bias_out, db, a.I, a.nsplit, s);

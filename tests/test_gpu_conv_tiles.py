@@ -13,12 +13,13 @@ def _ints(g, *shape):
 
 # 32 x 32 tiles below 1024 wide tiles, 64 x 64 (cout > 32) and 128 x 32 from
 # there on; 3 x 3 from LDS where cin % 16 == 0 and h % 4 == 0, with ragged
-# columns and channels; K below, at and beyond the four steps loaded ahead
+# columns and channels, one and two rows a wavefront; K below, at and beyond the four steps loaded ahead
 @pytest.mark.parametrize("h,w,cin,cout,ks,transposed", [
     (9, 7, 8, 33, 1, False), (33, 31, 64, 32, 1, False), (33, 31, 72, 40, 1, False),
     (256, 255, 24, 33, 1, False), (256, 129, 24, 40, 1, False),
     (365, 360, 8, 20, 3, False), (363, 360, 8, 32, 3, False),
     (4, 1, 16, 1, 3, False), (8, 33, 32, 33, 3, False), (64, 95, 48, 65, 3, False),
+    (256, 999, 16, 40, 3, False), (260, 999, 16, 40, 3, False),
     (128, 130, 16, 17, 1, True), (9, 5, 40, 9, 1, True)])
 def test_convolution_tiles(h, w, cin, cout, ks, transposed):
     import torch
@@ -46,10 +47,11 @@ def test_convolution_tiles(h, w, cin, cout, ks, transposed):
 
 
 # rows of a multiple of four pixels (one of them: both edges in a group) and
-# others, channels below and beyond a 64-column tile, a ragged last split, the
+# others, channels below and beyond the tiles, ragged last splits, the
 # output gradient at fine pixels
 @pytest.mark.parametrize("batch,h,w,cin,cout,ks,fine", [
     (2, 3, 4, 8, 8, 3, False), (1, 5, 12, 16, 72, 3, False), (3, 17, 20, 72, 8, 1, False),
+    (3, 41, 52, 64, 64, 3, False), (1, 70, 61, 64, 64, 3, False), (3, 41, 52, 16, 32, 3, False),
     (2, 40, 36, 8, 16, 3, False), (1, 31, 37, 8, 16, 3, False), (1, 7, 2, 8, 8, 3, False),
     (2, 6, 8, 16, 24, 1, True), (1, 9, 5, 16, 24, 1, True)])
 def test_weight_gradient_tiles(batch, h, w, cin, cout, ks, fine):
