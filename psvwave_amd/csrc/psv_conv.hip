@@ -624,31 +624,40 @@ __global__ void __launch_bounds__(256, U == 2 ? 3 : 4) wgrad_mfma_kernel(Wgrad a
 
 // out[e] = sum over s < nsplit of part[s * n + e]: `so` split lanes per
 // output (a power of two dividing 256), each summing every so-th split, then
-// a tree over the lanes -- a fixed order for a given (n, nsplit).
-__global__ void __launch_bounds__(256) reduce_splits_kernel(const float *__restrict__ part,
-                                                            float *out, long long n,
+// a tree over the lanes -- a fixed order for a given (n, nsplit).  Two such
+// sums of as many splits in one launch, since the second is mostly too small
+// to pay for its own: the blocks beyond the first's belong to it.
+struct SplitSum {
+  const float *part;
+  float *out;
+  long long n;
+};
+__global__ void __launch_bounds__(256) reduce_splits_kernel(SplitSum first, SplitSum second,
                                                             int nsplit, int so) {
   __shared__ float red[256];
   const int eo = 256 / so, el = threadIdx.x % eo, sl = threadIdx.x / eo;
-  const long long e = (long long)blockIdx.x * eo + el;
-  float v0 = 0.f, v1 = 0.f, v2 = 0.f, v3 = 0.f;
+  const long long blocks = (first.n + eo - 1) / eo;
+  const bool of_second = blockIdx.x >= blocks;
+  const float *const part = of_second ? second.part : first.part;
+  const long long n = of_second ? second.n : first.n;
+  const long long e = (blockIdx.x - (of_second ? blocks : 0)) * eo + el;
+  float v[8] = {};
   if (e < n) {
     int sp = sl;
-    for (; sp + 3 * so < nsplit; sp += 4 * so) {
-      v0 += part[(long long)sp * n + e];
-      v1 += part[(long long)(sp + so) * n + e];
-      v2 += part[(long long)(sp + 2 * so) * n + e];
-      v3 += part[(long long)(sp + 3 * so) * n + e];
-    }
-    for (; sp < nsplit; sp += so) v0 += part[(long long)sp * n + e];
+    for (; sp + 7 * so < nsplit; sp += 8 * so)
+#pragma unroll
+      for (int k = 0; k < 8; ++k) v[k] += part[(long long)(sp + k * so) * n + e];
+#pragma unroll
+    for (int k = 0; k < 7; ++k)
+      if (sp + k * so < nsplit) v[k] += part[(long long)(sp + k * so) * n + e];
   }
-  red[threadIdx.x] = (v0 + v1) + (v2 + v3);
+  red[threadIdx.x] = ((v[0] + v[1]) + (v[2] + v[3])) + ((v[4] + v[5]) + (v[6] + v[7]));
   __syncthreads();
   for (int w = so / 2; w >= 1; w /= 2) {
     if (sl < w) red[sl * eo + el] += red[(sl + w) * eo + el];
     __syncthreads();
   }
-  if (sl == 0 && e < n) out[e] = red[el];
+  if (sl == 0 && e < n) (of_second ? second.out : first.out)[e] = red[el];
 }
 
 // part[s][c] = sum of src[p * stride + off + c] over the pixels of split s;
@@ -858,12 +867,15 @@ hipError_t launch_conv_gemm(const ConvGemm &a, hipStream_t s) {
   return hipGetLastError();
 }
 
-static void launch_reduce_splits(const float *part, float *out, long long n, int nsplit,
-                          hipStream_t s) {
+// Split lanes: up to 16 as the splits need, so that 16 neighbouring outputs are
+// read together (with 4, as 344 splits had them, 9216 sums took 17 us); more
+// where the outputs are too few to fill the device.
+static void launch_reduce_splits(const SplitSum &a, const SplitSum &b, int nsplit, hipStream_t s) {
   int so = 1;
-  while (so < 256 && (long long)so * 8 < nsplit) so *= 2;
-  hipLaunchKernelGGL(reduce_splits_kernel, dim3(blocks_of(n, 256 / so)), dim3(256), 0, s,
-                     part, out, n, nsplit, so);
+  while (so < 256 && (long long)so * 8 < nsplit && (so < 16 || a.n * so < 65536)) so *= 2;
+  const int eo = 256 / so;
+  hipLaunchKernelGGL(reduce_splits_kernel, dim3(blocks_of(a.n, eo) + blocks_of(b.n, eo)), dim3(256),
+                     0, s, a, b, nsplit, so);
 }
 
 // Tile and splits.  A step costs a block the same in either tile, so the one
@@ -915,10 +927,8 @@ hipError_t launch_wgrad(Wgrad a, float *dw, float *db, float *workspace,
     launch(wgrad_mfma_kernel<true, 2, 2>, wgrad_mfma_kernel<true, 1, 3>);
   else
     launch(wgrad_mfma_kernel<false, 2, 2>, wgrad_mfma_kernel<false, 1, 3>);
-  if (split) {
-    launch_reduce_splits(workspace, dw, n, a.nsplit, s);
-    if (db) launch_reduce_splits(a.bias_out, db, a.I, a.nsplit, s);
-  }
+  if (split)
+    launch_reduce_splits({workspace, dw, n}, {a.bias_out, db, db ? a.I : 0}, a.nsplit, s);
   return hipGetLastError();
 }
 
@@ -934,7 +944,7 @@ hipError_t launch_channel_sum(const uint16_t *src, int stride, int off, int c, l
   ns = (P + chunk - 1) / chunk;
   hipLaunchKernelGGL(channel_sum_kernel, dim3(blocks_of(c, 64), (unsigned)ns), dim3(256), 0,
                      s, src, stride, off, c, P, chunk, ns > 1 ? workspace : out);
-  if (ns > 1) launch_reduce_splits(workspace, out, (long long)c, (int)ns, s);
+  if (ns > 1) launch_reduce_splits({workspace, out, c}, {}, (int)ns, s);
   return hipGetLastError();
 }
 
