@@ -398,6 +398,17 @@ int psv_conv_wgrad_bf16(const void *dy, int dy_stride, int dy_gather2x2, int dy_
                         const void *x, int x_stride, int x_channels, int ks, int batch, int h,
                         int w, float *dw, float *db, float *workspace,
                         int64_t workspace_floats, void *stream);
+/* Weight and gradient layouts: item i writes dims[0] x .. x dims[3] values,
+ * contiguous in dst, value (i0, .., i3) being src[offset + sum of ik *
+ * strides[k]], or zero from i3 = valid on.  dst is fp32, or with to_bf16
+ * bfloat16; all items go in a launch or a few. */
+typedef struct {
+  void *dst;
+  const float *src;
+  int64_t offset;
+  int dims[4], strides[4], valid, reserved;
+} psv_rearrangement;
+int psv_rearrange(const psv_rearrangement *items, int n, int to_bf16, void *stream);
 /* out[c] = sum over pixels of src[p * stride + offset + c] (bias gradients),
  * fixed-order fp32 sums. */
 int psv_channel_sum_bf16(const void *src, int stride, int offset, int channels,

@@ -50,6 +50,13 @@ class Info(C.Structure):
             "scalar_vp", "scalar_vs", "misfit")]
 
 
+class Rearrangement(C.Structure):
+    """psv_rearrangement: one strided copy of psv_rearrange."""
+    _fields_ = [("dst", C.c_void_p), ("src", C.c_void_p), ("offset", C.c_int64),
+                ("dims", C.c_int * 4), ("strides", C.c_int * 4), ("valid", C.c_int),
+                ("reserved", C.c_int)]
+
+
 _P = C.c_void_p
 _D = C.POINTER(C.c_double)
 _I = C.POINTER(C.c_int)
@@ -145,6 +152,7 @@ _SIGNATURES = {
                             C.c_void_p, C.c_void_p, C.c_void_p, C.c_int64, C.c_void_p],
     "psv_channel_sum_bf16": [C.c_void_p, _i, _i, _i, C.c_int64, C.c_void_p, C.c_void_p,
                              C.c_int64, C.c_void_p],
+    "psv_rearrange": [C.POINTER(Rearrangement), _i, _i, C.c_void_p],
     "psv_maxpool2_backward_bf16": [C.c_void_p, C.c_void_p, C.c_void_p, C.c_void_p, _i, _i,
                                    C.c_void_p, _i, _i, _i, _i, C.c_void_p],
 }

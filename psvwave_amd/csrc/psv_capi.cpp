@@ -8,6 +8,7 @@
 #include <new>
 #include <stdexcept>
 #include <string>
+#include <vector>
 
 #include "psv_batch.h"
 #include "psv_model.h"
@@ -951,6 +952,25 @@ int psv_channel_sum_bf16(const void *src, int stride, int offset, int channels,
                                            (hipStream_t)stream);
     if (e != hipSuccess)
       throw psv::RuntimeError(std::string("channel_sum: ") + hipGetErrorString(e));
+  });
+}
+
+int psv_rearrange(const psv_rearrangement *items, int n, int to_bf16, void *stream) {
+  static_assert(sizeof(psv_rearrangement) == sizeof(psv::Rearrangement), "the same struct");
+  return guard([&] {
+    if (n < 0) throw psv::ValueError("negative number of rearrangements");
+    if (n == 0) return;
+    need(items, "items");
+    std::vector<psv::Rearrangement> list(n);
+    std::memcpy(list.data(), items, n * sizeof(psv::Rearrangement));
+    for (const psv::Rearrangement &m : list) {
+      need(m.dst, "dst");
+      need(m.src, "src");
+    }
+    hipError_t e = psv::launch_rearrange(list.data(), n, to_bf16 != 0, (hipStream_t)stream);
+    if (e == hipErrorInvalidValue)
+      throw psv::ValueError("a rearrangement needs positive sizes, below 2^31 values in all");
+    if (e != hipSuccess) throw psv::RuntimeError(std::string("rearrange: ") + hipGetErrorString(e));
   });
 }
 

@@ -306,6 +306,16 @@ struct Wgrad {
 };
 hipError_t launch_wgrad(Wgrad a, float *dw, float *db, float *workspace,
                         long long workspace_floats, hipStream_t s);
+// dst[e] = src[offset + sum of the indices of e along dims times strides], zero
+// from index `valid` of the last dimension on; the same struct as the C
+// interface's.
+struct Rearrangement {
+  void *dst;
+  const float *src;
+  long long offset;
+  int dims[4], strides[4], valid, reserved;
+};
+hipError_t launch_rearrange(const Rearrangement *items, int n, bool to_bf16, hipStream_t s);
 hipError_t launch_channel_sum(const uint16_t *src, int stride, int off, int c, long long P,
                               float *out, float *workspace, long long workspace_floats,
                               hipStream_t s);

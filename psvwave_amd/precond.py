@@ -435,6 +435,34 @@ def learned_direction_ensemble(unets, g, fields, mirror=True):
     return [sum(d[k] for d in ds) / len(ds) for k in range(len(fields))]
 
 
+def _rearrange(items):
+    """Strided copies (dst, src, offset, dims, strides, valid): value (i0, .., i3)
+    of dst, contiguous and of shape dims, is src's element offset + sum of
+    ik strides[k], or zero for i3 >= valid.  All of dst have one type, fp32 or
+    bfloat16; on the GPU they go in a launch or two (psv_rearrange)."""
+    import torch
+    if not items:
+        return
+    if items[0][0].is_cuda:
+        from . import _lib
+        table = (_lib.Rearrangement * len(items))()
+        for t, (dst, src, offset, dims, strides, valid) in zip(table, items):
+            t.dst, t.src, t.offset, t.valid = dst.data_ptr(), src.data_ptr(), offset, valid
+            t.dims[:], t.strides[:] = dims, strides
+        _lib.check(_lib.load().psv_rearrange(
+            table, len(items), int(items[0][0].dtype == torch.bfloat16),
+            torch.cuda.current_stream().cuda_stream))
+        return
+    for dst, src, offset, dims, strides, valid in items:
+        index = torch.tensor(offset)
+        for d, stride in zip(dims, strides):
+            index = index.unsqueeze(-1) + torch.arange(d) * stride
+        values = src.reshape(-1)[index[..., :valid]]
+        full = torch.zeros(dims)
+        full[..., :valid] = values
+        dst.copy_(full.view(dst.shape))
+
+
 class HipUNetTrainer:
     """Training of a ``UNet`` with this library's bfloat16 MFMA kernels:
     forward convolutions keep their bfloat16 pre-activations, the backward
@@ -462,38 +490,49 @@ class HipUNetTrainer:
     def _pad8(c):
         return -(-c // 8) * 8
 
-    def _conv_layout(self, conv):
+    def _conv_layout(self, conv, items=None):
         """Forward [co][(ky ks + kx) cin8 + ci] and input-gradient
-        [ci][(ky ks + kx) co8 + co] (flipped taps) weights, bfloat16."""
-        import torch
-        w = conv.weight.detach()
+        [ci][(ky ks + kx) co8 + co] (flipped taps) weights, bfloat16; with
+        `items` their copies are left to the caller."""
+        w = conv.weight.detach().float().contiguous()
         co, ci, k, _ = w.shape
-        c8, o8 = self._pad8(ci), self._pad8(co)
-        f = torch.zeros(co, k, k, c8, device=self.device)
-        f[..., :ci] = w.permute(0, 2, 3, 1)
-        d = torch.zeros(ci, k, k, o8, device=self.device)
-        d[..., :co] = w.flip(2, 3).permute(1, 2, 3, 0)
-        return dict(kind="conv", mod=conv, ci=ci, c8=c8, co=co, o8=o8, k=k,
-                    wf=f.reshape(co, -1).to(torch.bfloat16).contiguous(),
-                    wd=d.reshape(ci, -1).to(torch.bfloat16).contiguous(),
+        c8, o8, kk = self._pad8(ci), self._pad8(co), k * k
+        wf, wd = self._empty(co, kk * c8), self._empty(ci, kk * o8)
+        mine = [(wf, w, 0, (co, k, k, c8), (ci * kk, k, 1, kk), ci),
+                (wd, w, kk - 1, (ci, k, k, o8), (kk, -k, -1, ci * kk), co)]
+        if items is None:
+            _rearrange(mine)
+        else:
+            items += mine
+        return dict(kind="conv", mod=conv, ci=ci, c8=c8, co=co, o8=o8, k=k, wf=wf, wd=wd,
                     b=conv.bias.detach().float().contiguous())
 
-    def _convt_layout(self, ct):
-        import torch
-        w = ct.weight.detach()  # (ci, co, 2, 2)
+    def _convt_layout(self, ct, items=None):
+        w = ct.weight.detach().float().contiguous()  # (ci, co, 2, 2)
         ci, co = w.shape[:2]
-        return dict(kind="convt", mod=ct, ci=ci, co=co,
-                    wf=w.permute(2, 3, 1, 0).reshape(4 * co, ci).to(torch.bfloat16).contiguous(),
-                    wd=w.permute(0, 2, 3, 1).reshape(ci, 4 * co).to(torch.bfloat16).contiguous(),
+        wf, wd = self._empty(4 * co, ci), self._empty(ci, 4 * co)
+        mine = [(wf, w, 0, (2, 2, co, ci), (2, 1, 4, 4 * co), ci),
+                (wd, w, 0, (ci, 2, 2, co), (4 * co, 2, 1, 4), co)]
+        if items is None:
+            _rearrange(mine)
+        else:
+            items += mine
+        return dict(kind="convt", mod=ct, ci=ci, co=co, wf=wf, wd=wd,
                     b=ct.bias.detach().float().contiguous())
 
     def _layouts(self):
-        n = self.net
-        return dict(enc=[(self._conv_layout(b[0]), self._conv_layout(b[2])) for b in n.enc],
-                    mid=(self._conv_layout(n.mid[0]), self._conv_layout(n.mid[2])),
-                    up=[self._convt_layout(u) for u in n.up],
-                    dec=[(self._conv_layout(b[0]), self._conv_layout(b[2])) for b in n.dec],
-                    out=self._conv_layout(n.out))
+        n, items = self.net, []
+
+        def conv(m):
+            return self._conv_layout(m, items)
+
+        L = dict(enc=[(conv(b[0]), conv(b[2])) for b in n.enc],
+                 mid=(conv(n.mid[0]), conv(n.mid[2])),
+                 up=[self._convt_layout(u, items) for u in n.up],
+                 dec=[(conv(b[0]), conv(b[2])) for b in n.dec],
+                 out=conv(n.out))
+        _rearrange(items)
+        return L
 
     # ---- kernel calls ---------------------------------------------------
     def _stream(self):
@@ -643,16 +682,20 @@ class HipUNetTrainer:
     @staticmethod
     def _to_param_grads(L, grads):
         """Kernel-layout gradients -> (module, dW shaped like the weight, db)."""
-        out = []
+        import torch
+        out, items = [], []
         for mod, (dw, db) in grads.items():
             wsh = mod.weight.shape
+            g = torch.empty(wsh, device=dw.device)
             if isinstance(mod, type(L["up"][0]["mod"])):
                 ci, co = wsh[:2]
-                g = dw.view(2, 2, co, ci).permute(3, 2, 0, 1)
+                items.append((g, dw, 0, (ci, co, 2, 2), (1, ci, 2 * co * ci, co * ci), 2))
             else:
                 co, ci, k, _ = wsh
-                g = dw.view(co, k, k, -1)[..., :ci].permute(0, 3, 1, 2)
-            out.append((mod, g.contiguous(), db))
+                c8 = dw.numel() // (co * k * k)
+                items.append((g, dw, 0, (co, ci, k, k), (k * k * c8, 1, k * c8, c8), k))
+            out.append((mod, g, db))
+        _rearrange(items)
         return out
 
     def prepare(self, x):

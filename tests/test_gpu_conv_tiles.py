@@ -155,3 +155,28 @@ def test_pooling_in_wide_accesses(h, w, c):
                 stream))
             grads.append(out.float().cpu())
         assert torch.equal(grads[0], grads[1])
+
+
+# more items than a launch holds, one value to several blocks, flipped taps,
+# padded and cut channels
+@pytest.mark.parametrize("half", [False, True])
+def test_rearrangements(half):
+    import torch
+    from psvwave_amd.precond import _rearrange
+    shapes = [(1, 1, 1, 1), (3, 3, 3, 8), (128, 3, 3, 40), (7, 2, 2, 512), (5, 1, 1, 9)] * 8
+    results = []
+    for device in ("cpu", "cuda"):
+        items = []
+        for n, (a, b, c, d) in enumerate(shapes):
+            valid = d if n % 3 else max(1, d - 3)
+            src = torch.arange(a * b * c * valid, dtype=torch.float32).mul_(0.37).add_(n)
+            dst = torch.full((a, b * c * d), float("nan"), device=device,
+                             dtype=torch.bfloat16 if half else torch.float32)
+            flip = -1 if n % 2 else 1  # the two inner dimensions in either order
+            items.append((dst, src.to(device), (b * c - 1) if flip < 0 else 0, (a, b, c, d),
+                          (b * c, flip * c, flip, a * b * c), valid))
+        print(f"[rearrange] {device} {half}", flush=True)
+        _rearrange(items)
+        results.append([item[0].float().cpu() for item in items])
+    for x, y in zip(*results):
+        assert torch.equal(x, y)
