@@ -8,7 +8,12 @@ storage, L2 misfit, adjoint sources, kernel reset, adjoint of all 8 shots
 with kernel correlation, kernel mapping -- 7.776e10 point-updates.
 
 Prints one JSON line.  ``value`` is point-updates per second of the whole
-step with all inputs resident in HBM.  ``roofline`` prices the step kernel
+step with all inputs resident in HBM.  The library runs each time loop as one
+resident launch, which moves only snapshots and kernel terms; ``roofline``
+then prices that kernel at its FP64 instructions against the device's FP64
+issue rate (one wave instruction in 4 cycles and vector unit), with the bytes
+it moves beside it.  With --variant, the time loops run step by step:
+``roofline`` prices the step kernel
 (the dominant kernel) at its algorithmic bytes per launch over its average
 duration when it runs alone (HIP start/end events of every launch of one
 shot's forward + adjoint on one stream, after the timed region);
@@ -63,8 +68,9 @@ def _args():
     p.add_argument("--gpus", type=int, default=1)
     p.add_argument("--steps", type=int, default=2)
     p.add_argument("--warmup", type=int, default=1)
-    p.add_argument("--variant", type=int, default=27,
-                   help="step kernel: 0 fused 64x8, 1 fused 64x16, 2 split; "
+    p.add_argument("--variant", type=int, default=None,
+                   help="run the time loops step by step on this step kernel "
+                        "instead of the library's resident loops: 0 fused 64x8, 1 fused 64x16, 2 split; "
                         "3-5 the same with reciprocal-multiply division; "
                         "6, 7 two steps per launch (64x8, 64x16); 8-13 lean "
                         "one-step kernels with 64 x 16, 8, 12, 20, 24, 32 "
@@ -77,8 +83,8 @@ def _args():
                         "with halo columns and ring "
                         "operands by DMA, 6 waves per SIMD; 25 the same "
                         "without the halo columns; 26 lean 64x16 with ring "
-                        "operands by DMA, 4 waves per SIMD; 27 (the library "
-                        "default), 28 variants 24, 26 with loads capped to "
+                        "operands by DMA, 4 waves per SIMD; 27 (the library's "
+                        "own where it runs by steps), 28 variants 24, 26 with loads capped to "
                         "the grid")
     p.add_argument("--no-xcd-remap", action="store_true")
     p.add_argument("--sequential", action="store_true",
@@ -251,6 +257,34 @@ def kernel_alone_us(model):
     return ms / max(timed, 1) * 1e3
 
 
+def resident_roofline(gpts, bytes_per_step, points):
+    """What bounds the resident loops at `gpts` 1e9 point updates per second:
+    the FP64 instructions of a point update against the device's issue rate,
+    and the bytes still moved (snapshots and kernel terms, an average per time
+    step) against its memory."""
+    instr = 111  # FP64 instructions of a point update, from the kernel's listing
+    peak = 256 * 4 * 16 * 2.4  # 256 compute units, 4 units of 16 lanes, GHz: 1e9 lanes / s
+    step_us = points / gpts * 1e-3
+    gbs = bytes_per_step / step_us * 1e-3
+    return {
+        "bound": "fp64 issue and the exchange between tiles",
+        "kernel": "resident_loop",
+        "achieved": round(instr * gpts, 1),
+        "peak": round(peak, 1),
+        "unit": "1e9 FP64 lane instructions/s",
+        "frac": round(instr * gpts / peak, 4),
+        "instructions_per_point_update": instr,
+        "us_per_time_step": round(step_us, 3),
+        "timing": "wall clock of the timed steps over the time steps of every shot",
+        "hbm": {"achieved": round(gbs, 1), "peak": HBM_PEAK_GBS, "unit": "GB/s",
+                "frac": round(gbs / HBM_PEAK_GBS, 4),
+                "bytes_per_time_step": bytes_per_step,
+                "by_steps_GBs": round((bytes_per_step + 104.0 * points) / step_us * 1e-3, 1),
+                "note": "by_steps: the bytes that a launch per step would have to move in "
+                        "the same time"},
+    }
+
+
 def monte_carlo(a):
     """Forward-only throughput of the Monte-Carlo batch: 512 Gaussian
     random-field models of uneven size (87M grid points in total), 2 shots,
@@ -305,11 +339,12 @@ def monte_carlo(a):
     # Algorithmic bytes per point-update: state read + written (80 B) and
     # the materials lm, mu, b (24 B) -- read once per time step for both
     # shots when forward_all runs them in lockstep (92 B per update).
-    lock = batch.lockstep()
+    resident = batch.resident()
+    lock = not resident and batch.lockstep()
     bytes_per_update = 92.0 if lock else 104.0
     achieved = bytes_per_update * upd / loop_s_per_step / 1e9
     launch_bytes = bytes_per_update * points * (2 if lock else 1)
-    return {
+    out = {
         "metric": METRIC + " (Monte-Carlo forward batch)",
         "value": round(value, 3), "unit": "Gpt-updates/s", "n_gpus": 1,
         "steps": a.steps, "warmup": a.warmup,
@@ -321,6 +356,7 @@ def monte_carlo(a):
         "config": {"workload": "Monte-Carlo forward batch", "models": len(cfgs),
                    "grid_points": points, "nt": nt, "shots": 2, "receivers": 32,
                    "point_updates_per_step": upd, "variant": best,
+                   "resident_loops": resident,
                    "autotune_ms_per_step": tuned, "hip_graph": a.graph,
                    "persistent": a.persistent,
                    "shots_in_lockstep": lock,
@@ -338,6 +374,10 @@ def monte_carlo(a):
                      "stream_ceiling": stream_ceiling(launch_bytes, achieved)},
         "misfit_mean": float(np.mean(mis)),
     }
+    if resident:
+        # the synthetic traces are all that is left to write
+        out["roofline"] = resident_roofline(value, 16.0 * 32 * len(cfgs), points)
+    return out
 
 
 def gradient_check(a):
@@ -657,7 +697,10 @@ def main():
 
     cfg = layered_faulted_config(nt=a.nt, n_shots=a.shots)
     model = psvwave_amd.fdModel(cfg)
-    model.set_step_variant(a.variant, not a.no_xcd_remap)
+    resident = a.variant is None and not a.graph and a.timing_stride <= 0
+    if not resident:
+        a.variant = 27 if a.variant is None else a.variant
+        model.set_step_variant(a.variant, not a.no_xcd_remap)
     if a.graph:
         model.set_graph_mode(True)
     true = layered_faulted_model(cfg, faulted=False)
@@ -690,7 +733,8 @@ def main():
         _progress(f"warmup step {k + 1}/{a.warmup}")
     # the per-shot calls run asynchronously only without step timing, so
     # the call-by-call driver is timed by the wall clock alone
-    events = not a.sequential or a.graph or a.timing_stride > 0
+    # (resident loops too: events around each would keep shots apart)
+    events = not resident and (not a.sequential or a.graph or a.timing_stride > 0)
     model.set_timing(a.timing_stride if events else 0)
     model.reset_step_timing()
     t0 = time.perf_counter()
@@ -704,7 +748,7 @@ def main():
         launches = timed = 2 * model.n_shots * model.nt * a.steps
         kern_ms = secs * 1e3
     model.set_timing(0)
-    alone_us = kernel_alone_us(model)
+    alone_us = 0.0 if resident else kernel_alone_us(model)
 
     nx, nz, nt = model.nx, model.nz, model.nt
     points_per_step = 2.0 * model.n_shots * nx * nz * nt
@@ -717,7 +761,7 @@ def main():
     launches_per_kernel = {2: 2, 5: 2, 6: 0.5, 7: 0.5, 14: 0.5}.get(a.variant, 1)
     avg_launch_s = kern_ms / 1e3 / max(timed, 1)
     device_achieved = bytes_per_launch / avg_launch_s / 1e9
-    achieved = bytes_per_launch / (alone_us * 1e-6) / 1e9
+    achieved = 0.0 if resident else bytes_per_launch / (alone_us * 1e-6) / 1e9
     kernel_name = {0: "step_fused<8,ieee>", 1: "step_fused<16,ieee>",
                    2: "step_split_stress<8,ieee>+step_split_velocity<8,ieee>",
                    3: "step_fused<8,recip>", 4: "step_fused<16,recip>",
@@ -734,7 +778,7 @@ def main():
                    26: "step_lean<16,ring DMA>",
                    27: "step_lean<8,halo+ring DMA,capped>",
                    28: "step_lean<16,ring DMA,capped>",
-                   }[a.variant]
+                   }.get(a.variant, "resident_loop")
     out = {
         "metric": METRIC,
         "value": round(value, 3),
@@ -759,7 +803,10 @@ def main():
             "step_kernel": kernel_name,
             "xcd_remap": not a.no_xcd_remap,
             "hip_graph": a.graph,
-            "driver": ("call by call, one stream" if a.graph or a.timing_stride > 0 else
+            "driver": (("call by call" if a.sequential else "run_model") +
+                       ": each time loop one resident launch, the state on "
+                       "chip" if resident else
+                       "call by call, one stream" if a.graph or a.timing_stride > 0 else
                        "call by call (forward_simulate per shot, misfit, adjoint "
                        "sources, adjoint_simulate per shot): asynchronous calls, "
                        "forwards two at a time, adjoints in pairs with deferred "
@@ -809,9 +856,13 @@ def main():
             },
         },
     }
+    if resident:
+        out["roofline"] = resident_roofline(
+            value, bytes_per_launch - 104.0 * nx * nz, nx * nz)
     if copy:
         out["roofline"]["copy_calibration"] = copy
-    out["roofline"]["stream_ceiling"] = stream_ceiling(bytes_per_launch, achieved)
+    if not resident:
+        out["roofline"]["stream_ceiling"] = stream_ceiling(bytes_per_launch, achieved)
     if not a.no_cpu_baseline:
         out["cpu_baseline"] = cpu_baseline(a.cpu_baseline_nt)
     print(json.dumps(out), flush=True)

@@ -310,6 +310,10 @@ int psv_batch_forward_all(psv_batch *b);
  * current variant and modes (allocating the extra state sets if needed),
  * else 0. */
 int psv_batch_lockstep(psv_batch *b, int *on);
+/* *on = 1 when the batch's time loops run as resident launches (the default
+ * where every member fits the device; psv_batch_autotune may decide against
+ * it), else 0: step by step. */
+int psv_batch_resident(psv_batch *b, int *on);
 /* L2 misfit of every model (n values), as calculate_l2_misfit. */
 int psv_batch_misfits(psv_batch *b, double *out);
 /* Step kernel for all members: 0, 1, 6, 7, 8-13 or 18-28 (see

@@ -92,6 +92,13 @@ class Batch:
         _lib.check(self._lib.psv_batch_lockstep(self._h, C.byref(on)))
         return bool(on.value)
 
+    def resident(self):
+        """Whether the time loops run as resident launches, the state on
+        chip, rather than step by step."""
+        on = C.c_int()
+        _lib.check(self._lib.psv_batch_resident(self._h, C.byref(on)))
+        return bool(on.value)
+
     def misfits(self):
         """L2 misfit of every member (calculate_l2_misfit of each)."""
         out = np.empty(len(self))

@@ -759,6 +759,13 @@ int psv_batch_lockstep(psv_batch *b, int *on) {
   });
 }
 
+int psv_batch_resident(psv_batch *b, int *on) {
+  return guard([&] {
+    need(on, "on");
+    *on = B(b).runs_resident() ? 1 : 0;
+  });
+}
+
 int psv_batch_misfits(psv_batch *b, double *out) {
   return guard([&] {
     need(out, "out");
