@@ -98,6 +98,7 @@ class Batch {
     LoopArgs *args = nullptr;
     int4 *blocks = nullptr;
   };
+  int choose_loop_kind(int shots);
   bool resident_available();
   LoopLaunches *loop_launches(int which, int i_shot, int steps);
   void run_loops(LoopLaunches &p, int steps);
@@ -108,6 +109,7 @@ class Batch {
   int loop_kind_ = -2;    // -2 not chosen, -1 some member does not fit
   std::map<int, LoopLaunches> loops_;
   void *loop_cells_ = nullptr;
+  size_t loop_cells_bytes_ = 0;
   unsigned loop_tag_ = 1;
   unsigned *loop_sync_ = nullptr, *loop_poison_ = nullptr;
   unsigned *loop_status_ = nullptr;  // host memory, one word per launch

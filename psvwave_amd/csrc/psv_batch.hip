@@ -222,45 +222,45 @@ void Batch::clear_loops() {
   loops_.clear();
 }
 
-// The kernel of all loops: the smallest tiles with which every loop of
-// forward_all fits one launch, since a step of small tiles is shorter; a
-// batch that needs several launches runs on 28-row tiles, two blocks per
-// compute unit: the blocks of a unit mostly belong to different loops and
-// hide each other's exchange.
+// The kernel for launches of `shots` loops of every member: the first that
+// holds them all (kLoopFits), or where several launches are needed 28-row tiles,
+// two blocks per compute unit: the blocks of a unit mostly belong to different
+// loops and hide each other's exchange.  -1: some member fits no kernel.
+int Batch::choose_loop_kind(int shots) {
+  for (auto &m : models_)
+    if (!m->lean_ok() || m->derived().nx < 8 || m->derived().nz < 8) return -1;
+  // tiles of all loops and of the largest member
+  auto tiles = [&](int kind, long long *most) {
+    long long sum = 0;
+    *most = 0;
+    for (auto &m : models_) {
+      const long long t =
+          (long long)loop_tiles_x(m->derived().nx) * loop_tiles_z(m->derived().nz, kind);
+      sum += t * shots;
+      *most = std::max(*most, t);
+    }
+    return sum;
+  };
+  auto usable = [&](int kind) {  // the tables of every member
+    for (auto &m : models_)
+      if (m->loop_tile_columns(kind) == 0) return false;
+    return true;
+  };
+  long long most = 0;
+  for (const LoopFit &f : kLoopFits)
+    if (tiles(f.kind, &most) <= loop_capacity(f.kind, f.per_unit) && usable(f.kind)) return f.kind;
+  for (int k : {kNumLoopKinds - 2, kNumLoopKinds - 1})
+    if (tiles(k, &most) > 0 && most <= loop_capacity(k) && usable(k)) return k;
+  return -1;
+}
+
 bool Batch::resident_available() {
   if (!resident_ || graph_mode_ || persistent_) return false;
   if (loop_skip_ > 0) {
     --loop_skip_;
     return false;
   }
-  if (loop_kind_ == -2) {
-    loop_kind_ = -1;
-    bool able = true;
-    for (auto &m : models_) able = able && m->lean_ok() && m->derived().nx >= 8 && m->derived().nz >= 8;
-    // tiles of all loops and of the largest member
-    auto tiles = [&](int kind, long long *most) {
-      long long sum = 0;
-      *most = 0;
-      for (auto &m : models_) {
-        const long long t =
-            (long long)loop_tiles_x(m->derived().nx) * loop_tiles_z(m->derived().nz, kind);
-        sum += t * n_shots_;
-        *most = std::max(*most, t);
-      }
-      return sum;
-    };
-    auto usable = [&](int kind) {  // the tables of every member
-      for (auto &m : models_)
-        if (m->loop_tile_columns(kind) == 0) return false;
-      return true;
-    };
-    long long most = 0;
-    for (int k = 0; able && k < 3 && loop_kind_ < 0; ++k)
-      if (tiles(k, &most) <= loop_capacity(k) && usable(k)) loop_kind_ = k;
-    for (int k : {2, 3})
-      if (able && loop_kind_ < 0 && tiles(k, &most) > 0 && most <= loop_capacity(k) && usable(k))
-        loop_kind_ = k;
-  }
+  if (loop_kind_ == -2) loop_kind_ = choose_loop_kind(n_shots_);
   return loop_kind_ >= 0;
 }
 
@@ -270,7 +270,8 @@ bool Batch::resident_available() {
 Batch::LoopLaunches *Batch::loop_launches(int which, int i_shot, int steps) {
   LoopLaunches &p = loops_[which + 8 * i_shot];
   if (p.kind >= 0 && which != 4) return &p;
-  const int kind = p.kind = loop_kind_;
+  // (a launch of one shot may have room for smaller tiles than one of all)
+  const int kind = p.kind = which == 0 || which == 4 ? loop_kind_ : choose_loop_kind(1);
   p.forward = which != 3;
   std::vector<LoopRef> refs;
   for (int m = 0; m < size(); ++m)
@@ -299,9 +300,13 @@ Batch::LoopLaunches *Batch::loop_launches(int which, int i_shot, int steps) {
   p.loops.clear(), p.launches.clear(), p.first_block.clear();
   const int cap = loop_capacity(kind);
   const size_t cell_bytes = loop_cells_bytes(kind, 1);
-  if (!loop_cells_) {
-    hip_check(hipMalloc(&loop_cells_, cell_bytes * cap), "hipMalloc");
-    hip_check(launch_fill((double *)loop_cells_, (long long)(cell_bytes * cap / 8), 0.0, stream_),
+  if (!loop_cells_) {  // for every kernel: the launches of all calls keep pointers into them
+    size_t bytes = 0;
+    for (int k = 0; k < kNumLoopKinds; ++k)
+      bytes = std::max(bytes, loop_cells_bytes(k, loop_capacity(k)));
+    hip_check(hipMalloc(&loop_cells_, bytes), "hipMalloc");
+    loop_cells_bytes_ = bytes;
+    hip_check(launch_fill((double *)loop_cells_, (long long)(bytes / 8), 0.0, stream_),
               "clear cells");
   }
   std::vector<LoopArgs> args;
@@ -364,8 +369,7 @@ void Batch::run_loops(LoopLaunches &p, int steps) {
   for (int i = 0; i < n; ++i) {
     if (loop_tag_ + (unsigned)steps < loop_tag_) {  // the tags start over
       hip_check(launch_fill((double *)loop_cells_,
-                            (long long)(loop_cells_bytes(p.kind, loop_capacity(p.kind)) / 8), 0.0,
-                            stream_),
+                            (long long)(loop_cells_bytes_ / 8), 0.0, stream_),
                 "clear cells");
       loop_tag_ = 1;
     }

@@ -18,9 +18,20 @@ namespace psv {
 struct LoopKind {
   int rows, waves;
 };
-constexpr LoopKind kLoopKinds[] = {{1, 8}, {2, 8}, {4, 8}, {4, 16}};
-constexpr int kNumLoopKinds = 4;
+constexpr LoopKind kLoopKinds[] = {{1, 8}, {2, 8}, {3, 8}, {4, 8}, {4, 16}};
+constexpr int kNumLoopKinds = 5;
 constexpr int kLoopTileX = 60;
+// Loop kernels and blocks per compute unit in the order of their time per step
+// (2.9, 3.5, 4.0, 4.3, 5.2, 6.0, 6.5, 7.8 and 7.9 us): launches take the first
+// whose tiles all fit.  Fewer rows a wave make a step shorter, and so does a
+// block alone on its unit, up to a wave of rows less: 960 x 448 points take 6.0
+// us on 256 tiles of 28 rows and 6.5 on 368 of 20, 800 x 700 points 6.5 on 490
+// of 20 rows and 7.7 on 350 of 28.
+struct LoopFit {
+  int kind, per_unit;
+};
+constexpr LoopFit kLoopFits[] = {{0, 1}, {1, 1}, {0, 2}, {2, 1}, {1, 2},
+                                 {3, 1}, {2, 2}, {3, 2}, {4, 1}};
 constexpr int loop_tile_rows(int kind) {
   return kLoopKinds[kind].rows * kLoopKinds[kind].waves - 4;
 }
@@ -99,14 +110,14 @@ inline int loop_tiles_z(int nz, int kind) {
 
 // Rim cells kept for a tile (the points at most three from its edge), and
 // bytes of the exchange cells of one loop.
-constexpr int loop_rim_cells(int kind) { return kind == 3 ? 1024 : 512; }
+constexpr int loop_rim_cells(int kind) { return kLoopKinds[kind].waves == 16 ? 1024 : 512; }
 inline size_t loop_cells_bytes(int kind, int ntiles) {
   return (size_t)ntiles * 4 * loop_rim_cells(kind) * 16;
 }
 
-// Blocks of a loop kernel that the current device holds at once (0: it
-// cannot run them).
-int loop_capacity(int kind);
+// Blocks of a loop kernel that the current device holds at once, at most
+// per_unit of them on a compute unit (0: it cannot run them).
+int loop_capacity(int kind, int per_unit = 2);
 
 // Launches through the gate of the current device: the blocks of all loop
 // launches that may run at the same time fit the device together.

@@ -881,6 +881,7 @@ const LoopDevice &loop_device(int dev) {
     d.per_cu[1] = loop_blocks_per_cu<1>();
     d.per_cu[2] = loop_blocks_per_cu<2>();
     d.per_cu[3] = loop_blocks_per_cu<3>();
+    d.per_cu[4] = loop_blocks_per_cu<4>();
     for (int n : d.per_cu)
       if (n < 1) d.xcds = 0;
     (void)hipGetLastError();
@@ -999,11 +1000,11 @@ hipError_t launch_loop_prepare(LoopArgs *dst, const LoopArgs &a, unsigned *sync,
   return hipGetLastError();
 }
 
-int loop_capacity(int kind) {
+int loop_capacity(int kind, int per_unit) {
   int dev = 0;
   if (hipGetDevice(&dev) != hipSuccess || dev >= kMaxDevices) return 0;
   const LoopDevice &d = loop_device(dev);
-  return d.xcds * kXcdCus * d.per_cu[kind];
+  return d.xcds * kXcdCus * std::min(d.per_cu[kind], per_unit);
 }
 
 void loop_gate_forget(hipStream_t s) {
@@ -1027,6 +1028,7 @@ hipError_t launch_loop(int kind, bool adjoint, const LoopLaunch &l, hipStream_t 
     case 1: launch(resident_loop<1, false>, resident_loop<1, true>); break;
     case 2: launch(resident_loop<2, false>, resident_loop<2, true>); break;
     case 3: launch(resident_loop<3, false>, resident_loop<3, true>); break;
+    case 4: launch(resident_loop<4, false>, resident_loop<4, true>); break;
     default: return hipErrorInvalidValue;
   }
   return hipGetLastError();

@@ -801,17 +801,14 @@ void Model::release(void *p, size_t bytes) {
   device_bytes_ -= (int64_t)bytes;
 }
 
-// The kernel for `loops` loops side by side: the smallest tiles with which
-// the device holds them all (-1: none).  Small tiles shorten a step, since
-// each wave advances fewer rows (680 x 380 points: 4.7 us per step on 12-row
-// tiles, 5.7 on 28-row and 7.6 on 60-row ones); two blocks of 28 rows on a
-// compute unit beat one of 60 rows, which waits for its neighbours with the
-// unit idle (1800 x 450: 7.8 against 8.0 us).
+// The kernel for `loops` loops side by side (-1: the device cannot hold them).
 int Model::loop_kind(int loops) {
   if (d_.nx < 8 || d_.nz < 8) return -1;
-  for (int k = 0; k < kNumLoopKinds; ++k)
-    if (ensure_loop_tables(k) && (long long)loops * loop_tables_[k].tiles() <= loop_capacity(k))
-      return k;
+  for (const LoopFit &f : kLoopFits)
+    if ((long long)loops * loop_tiles_x(d_.nx) * loop_tiles_z(d_.nz, f.kind) <=
+            loop_capacity(f.kind, f.per_unit) &&
+        ensure_loop_tables(f.kind))
+      return f.kind;
   return -1;
 }
 
@@ -1297,10 +1294,9 @@ void Model::enqueue_checkpointed_adjoint(
 // recomputation of segment c - 1 beside the adjoint of segment c.  With the
 // tiles with which the device holds both at once the pair costs less than one
 // after the other on smaller tiles (a gradient of four shots on 680 x 380
-// points, 4000 steps, snapshots every 10 and a checkpoint every 80: 194
-// against 227 ms; by steps 279); where it holds only one, the gate keeps them
-// apart.  The
-// state of the adjoint passes from launch to launch through state_, in turn
+// points, 4000 steps, snapshots every 10 and a checkpoint every 80: 166 ms on
+// 20-row tiles, 194 on 28-row ones, one after the other 227; by steps 279);
+// where it holds only one, the gate keeps them apart.  The state of the adjoint passes from launch to launch through state_, in turn
 // from one buffer to the other (a block may end its segment before another
 // has read its part).  After a launch that did not take place none of the
 // later ones does anything, and the remaining segments run step by step.
