@@ -24,6 +24,7 @@ The gradient is the reference's (``get_kernels`` after the adjoint,
 src/fdModel.cpp:789-969, 1164-1183); the FWI loop follows the descent loop of
 tests/test_descent.py:106-129 with a line search added.
 """
+import math
 import time
 
 import numpy as np
@@ -438,11 +439,22 @@ def learned_direction_ensemble(unets, g, fields, mirror=True):
 def _rearrange(items):
     """Strided copies (dst, src, offset, dims, strides, valid): value (i0, .., i3)
     of dst, contiguous and of shape dims, is src's element offset + sum of
-    ik strides[k], or zero for i3 >= valid.  All of dst have one type, fp32 or
-    bfloat16; on the GPU they go in a launch or two (psv_rearrange)."""
+    ik strides[k], or zero for i3 >= valid.  src is contiguous fp32, all of dst
+    have one type, fp32 or bfloat16; on the GPU they go in a launch or two
+    (psv_rearrange, which takes addresses: hence the checks)."""
     import torch
     if not items:
         return
+    dtype, device = items[0][0].dtype, items[0][0].device
+    if dtype not in (torch.float32, torch.bfloat16):
+        raise ValueError(f"rearrangements are to float32 or bfloat16, not {dtype}")
+    for dst, src, _, dims, _, _ in items:
+        if dst.dtype != dtype or src.dtype != torch.float32:
+            raise ValueError("rearrangements need float32 sources and one type of results")
+        if dst.device != device or src.device != device:
+            raise ValueError("rearrangements need all tensors on one device")
+        if not (dst.is_contiguous() and src.is_contiguous()) or dst.numel() != math.prod(dims):
+            raise ValueError("rearrangements need contiguous tensors and results of their size")
     if items[0][0].is_cuda:
         from . import _lib
         table = (_lib.Rearrangement * len(items))()
@@ -450,15 +462,15 @@ def _rearrange(items):
             t.dst, t.src, t.offset, t.valid = dst.data_ptr(), src.data_ptr(), offset, valid
             t.dims[:], t.strides[:] = dims, strides
         _lib.check(_lib.load().psv_rearrange(
-            table, len(items), int(items[0][0].dtype == torch.bfloat16),
+            table, len(items), int(dtype == torch.bfloat16),
             torch.cuda.current_stream().cuda_stream))
         return
     for dst, src, offset, dims, strides, valid in items:
-        index = torch.tensor(offset)
+        index = torch.tensor(offset, device=device)
         for d, stride in zip(dims, strides):
-            index = index.unsqueeze(-1) + torch.arange(d) * stride
+            index = index.unsqueeze(-1) + torch.arange(d, device=device) * stride
         values = src.reshape(-1)[index[..., :valid]]
-        full = torch.zeros(dims)
+        full = torch.zeros(dims, dtype=torch.float32, device=device)
         full[..., :valid] = values
         dst.copy_(full.view(dst.shape))
 
@@ -483,7 +495,7 @@ class HipUNetTrainer:
         self.net = net.to(device)
         self.opt = torch.optim.AdamW(net.parameters(), lr=lr, weight_decay=weight_decay)
         self.sched = torch.optim.lr_scheduler.CosineAnnealingLR(self.opt, T_max=epochs)
-        self.ws = torch.empty(self.WORKSPACE_FLOATS, device=device)
+        self.ws = torch.empty(self.WORKSPACE_FLOATS, device=device, dtype=torch.float32)
 
     # ---- weight layouts -------------------------------------------------
     @staticmethod
@@ -686,7 +698,7 @@ class HipUNetTrainer:
         out, items = [], []
         for mod, (dw, db) in grads.items():
             wsh = mod.weight.shape
-            g = torch.empty(wsh, device=dw.device)
+            g = torch.empty(wsh, device=dw.device, dtype=torch.float32)
             if isinstance(mod, type(L["up"][0]["mod"])):
                 ci, co = wsh[:2]
                 items.append((g, dw, 0, (ci, co, 2, 2), (1, ci, 2 * co * ci, co * ci), 2))
