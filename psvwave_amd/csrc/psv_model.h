@@ -326,10 +326,12 @@ class Model {
   unsigned loop_tag_ = 1;
   unsigned *loop_status_ = nullptr;  // host memory, one word per job
   static constexpr int kLoopStatusWords = 1024;
+  static constexpr int kLoopTogether = 16;  // loops of a launch at most
   int loop_skip_ = 0;  // forwards still to run step by step after a refused launch
   static constexpr int kLoopSkip = 64;
   void ensure_loop_words();
   bool resident_path(bool dump);
+  bool joins_loops(bool verbose, bool dump);
   void ensure_loop_room(int n, size_t cells, unsigned steps);
   bool ensure_loop_tables(int kind);
   int loop_kind(int loops);

@@ -792,6 +792,21 @@ bool Model::resident_path(bool dump) {
   return loop_kind(1) >= 0;
 }
 
+// Whether the time loop of an asynchronous call joins the resident queue.  Only
+// one of the two queues, loop_jobs_ and the lanes' jobs_, ever holds work: what
+// is left in the other ends first, so that a loop sees the snapshots, traces
+// and kernels of all calls before it and no loop that is run again by steps
+// uses the state of another.
+bool Model::joins_loops(bool verbose, bool dump) {
+  if (!async_ || verbose || timing_stride_ != 0) return false;
+  // with the status words used up the queue ends here, before the choice: it
+  // may find a refused launch
+  if (loop_jobs_.size() + kLoopTogether > (size_t)kLoopStatusWords) settle();
+  if (!resident_path(dump)) return false;
+  if (!jobs_.empty()) settle();
+  return true;
+}
+
 void Model::release(void *p, size_t bytes) {
   if (!p) return;
   sync();
@@ -980,18 +995,15 @@ void Model::push_loop(int kind, int shot, bool store) {
   // with the first call as it does for loops by steps
   if (!lane_stream_) create_stream(&lane_stream_);
   const bool fwd = kind == kJobForward;
-  bool apart = loop_jobs_.size() + 16 > (size_t)kLoopStatusWords;
+  bool apart = false;
   for (size_t i = loop_launched_; i < loop_jobs_.size(); ++i)
     apart = apart || (loop_jobs_[i].kind == kJobForward) != fwd ||
             (fwd && loop_jobs_[i].shot == shot);
-  if (loop_jobs_.size() + 16 > (size_t)kLoopStatusWords)
-    settle_loops();
-  else if (apart)
-    flush_loops();
+  if (apart) flush_loops();
   const int pending = (int)(loop_jobs_.size() - loop_launched_);
   loop_jobs_.push_back({fwd ? kJobForward : pending ? kJobDeferred : kJobAdjoint, shot, store,
                         pending - 1, 0});
-  int together = std::min(16, loop_group(16));
+  int together = loop_group(kLoopTogether);
   if (!fwd && together > 1) {
     // a buffer of kernel terms for all but the first: as many as the device
     // has room for, keeping to a tenth of its memory
@@ -1591,12 +1603,13 @@ void Model::forward(int i_shot, bool store_fields, bool verbose,
   if (store_fields && cfg_.nt % cfg_.snapshot_interval != 0)
     throw ValueError("Snapshot interval and size of accumulator don't match!"
                      " (nt must be a multiple of snapshot_interval)");
-  if (resident_path(output_wavefields) && async_ && !verbose && timing_stride_ == 0) {
+  if (joins_loops(verbose, output_wavefields)) {
     if (store_fields) ensure_snapshots();
     push_loop(kJobForward, i_shot, store_fields);
     return;
   }
   if (async_path(verbose, output_wavefields)) {
+    if (!loop_jobs_.empty()) settle();
     ensure_lane();
     // a pending adjoint may still read this shot's snapshots and a pending
     // forward of the same shot writes the same traces: wait for them; a new
@@ -1638,11 +1651,12 @@ void Model::adjoint(int i_shot, bool verbose) {
   if (!snap_[0])
     throw ValueError("adjoint_simulate needs stored forward wavefields; run "
                      "forward_simulate with store_fields=True first");
-  if (resident_path(false) && async_ && !verbose && timing_stride_ == 0 && ckpt_every_ == 1) {
+  if (ckpt_every_ == 1 && joins_loops(verbose, false)) {
     push_loop(kJobAdjoint, i_shot, false);
     return;
   }
   if (async_path(verbose, false)) {
+    if (!loop_jobs_.empty()) settle();
     ensure_lane();
     if (!defer_ && !no_defer_room_) {
       // a new buffer is zero-filled on the model stream: allocate it on a
