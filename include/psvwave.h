@@ -237,10 +237,6 @@ int psv_set_graph_mode(psv_model *m, int on);
  * `every`, the adjoint costs one extra forward.  get_snapshots is then
  * unavailable.  Changing it discards stored snapshots. */
 int psv_set_checkpointing(psv_model *m, int every);
-/* For tests: the model's next resident time loops find, as if another process
- * held part of the device, that their blocks are not resident together, and
- * run step by step instead (same results). */
-int psv_refuse_resident_loops(psv_model *m);
 int psv_get_step_timing(psv_model *m, double *total_ms, int64_t *timed,
                         int64_t *launches);
 int psv_reset_step_timing(psv_model *m);

@@ -114,7 +114,6 @@ _SIGNATURES = {
     "psv_set_step_variant": [_P, _i, _i],
     "psv_set_timing": [_P, _i],
     "psv_set_graph_mode": [_P, _i],
-    "psv_refuse_resident_loops": [_P],
     "psv_set_checkpointing": [_P, _i],
     "psv_set_async": [_P, _i],
     "psv_synchronize": [_P],

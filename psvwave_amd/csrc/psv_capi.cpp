@@ -1,4 +1,5 @@
-// psv_capi.cpp -- extern "C" entry points declared in include/psvwave.h.
+// psv_capi.cpp -- extern "C" entry points declared in include/psvwave.h (and
+// those of psv_testing.h).
 // Each translates C++ exceptions into a status code plus a thread-local
 // message: ValueError -> PSV_EVALUE (the reference's invalid_argument /
 // length_error / value_error cases), everything else -> PSV_ERUNTIME.
@@ -12,6 +13,7 @@
 
 #include "psv_batch.h"
 #include "psv_model.h"
+#include "psv_testing.h"
 
 struct psv_model {
   psv::Model *impl;

@@ -1,0 +1,19 @@
+/* psv_testing.h -- entry points that the tests force conditions with, which a
+ * program has no use for and the public header therefore does not declare.
+ * They act on one object and leave every result as it is. */
+#pragma once
+
+#include "../../include/psvwave.h"
+
+#ifdef __cplusplus
+extern "C" {
+#endif
+
+/* The model's next resident time loops find, as if another process held part
+ * of the device, that their blocks are not resident together, and run step by
+ * step instead. */
+int psv_refuse_resident_loops(psv_model *m);
+
+#ifdef __cplusplus
+}
+#endif
