@@ -571,6 +571,10 @@ int psv_synchronize(psv_model *m) {
   return guard([&] { M(m); });
 }
 
+int psv_fail_allocation(psv_model *m, int n) {
+  return guard([&] { MA(m).fail_allocation(n); });
+}
+
 int psv_refuse_resident_loops(psv_model *m) {
   return guard([&] { M(m).refuse_next_loops(); });
 }

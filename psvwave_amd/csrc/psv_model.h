@@ -112,6 +112,8 @@ class Model {
   }
   void reset_step_timing() { timed_ms_ = 0, timed_ = 0, launches_ = 0; }
   int64_t device_bytes() const { return device_bytes_; }
+  // As if the device were full at the allocation after the next n (tests).
+  void fail_allocation(int n) { fail_allocation_ = n; }
   // As if another process held part of the device: the blocks of the next
   // resident launches leave at once and their loops run step by step (tests).
   void refuse_next_loops();
@@ -168,6 +170,9 @@ class Model {
   std::vector<InjectionTerm> adjoint_terms() const;
   void ensure_snapshots();
   double *dalloc(size_t n);
+  void dalloc_all(double **p, int count, size_t n);
+  template <class T>
+  void release(T *&p, size_t bytes);
   void upload(double *dst, const double *src, size_t n) const;
   void download(double *dst, const double *src, size_t n) const;
   double *staging(size_t n) const;
@@ -190,6 +195,7 @@ class Model {
   bool owns_stream_ = true;
   std::vector<void *> allocations_;
   int64_t device_bytes_ = 0;
+  int fail_allocation_ = -1;
 
   double *state_[2][5] = {};  // ping-pong: vx, vz, txx, tzz, txz (padded)
   double *lm_ = nullptr, *mu_ = nullptr, *b_ = nullptr;  // padded
@@ -336,7 +342,6 @@ class Model {
   bool ensure_loop_tables(int kind);
   int loop_kind(int loops);
   int loop_group(int limit);
-  void release(void *p, size_t bytes);
   void push_loop(int kind, int shot, bool store);
   void flush_loops();
   void settle_loops();

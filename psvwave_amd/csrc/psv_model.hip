@@ -23,8 +23,9 @@ namespace psv {
 namespace {
 
 void hip_check(hipError_t e, const char *what) {
-  if (e != hipSuccess)
-    throw RuntimeError(std::string(what) + ": " + hipGetErrorString(e));
+  if (e == hipSuccess) return;
+  (void)hipGetLastError();  // reported here, not by the check of a later launch
+  throw RuntimeError(std::string(what) + ": " + hipGetErrorString(e));
 }
 
 long long round_up(long long v, long long m) { return (v + m - 1) / m * m; }
@@ -138,13 +139,27 @@ Model::~Model() {
 double *Model::dalloc(size_t n) {
   void *p = nullptr;
   size_t bytes = std::max<size_t>(n, 1) * sizeof(double);
-  hip_check(hipMalloc(&p, bytes), "hipMalloc");
+  const bool fail = fail_allocation_ >= 0 && fail_allocation_-- == 0;
+  hip_check(fail ? hipErrorOutOfMemory : hipMalloc(&p, bytes), "hipMalloc");
   allocations_.push_back(p);
   device_bytes_ += (int64_t)bytes;
   hip_check(launch_fill((double *)p, (long long)std::max<size_t>(n, 1), 0.0,
                         stream_),
             "zero-fill");
   return (double *)p;
+}
+
+// Buffers of n values each, all `count` of them or none: a caller that tries
+// again after an error finds its pointers null or whole.
+void Model::dalloc_all(double **p, int count, size_t n) {
+  std::vector<double *> got;
+  try {
+    for (int k = 0; k < count; ++k) got.push_back(dalloc(n));
+  } catch (...) {
+    for (double *&q : got) release(q, std::max<size_t>(n, 1) * sizeof(double));
+    throw;
+  }
+  std::copy(got.begin(), got.end(), p);
 }
 
 void Model::sync() const {
@@ -408,7 +423,7 @@ void Model::ensure_snapshots() {
   if (snap_[0]) return;
   clear_graphs();
   long long n = (long long)cfg_.n_shots * stored_snapshots() * ngrid_;
-  for (int f = 0; f < 5; ++f) snap_[f] = dalloc(n);
+  dalloc_all(snap_, 5, n);
 }
 
 void Model::upload(double *dst, const double *src, size_t n) const {
@@ -430,6 +445,7 @@ double *Model::staging(size_t n) const {
     sync();
     if (staging_) (void)hipFree(staging_);
     staging_ = nullptr;
+    staging_n_ = 0;
     hip_check(hipMalloc((void **)&staging_, n * sizeof(double)),
               "hipMalloc staging");
     staging_n_ = n;
@@ -807,13 +823,17 @@ bool Model::joins_loops(bool verbose, bool dump) {
   return true;
 }
 
-void Model::release(void *p, size_t bytes) {
+// Frees a buffer of `bytes` bytes and forgets it, also where what follows fails.
+template <class T>
+void Model::release(T *&p, size_t bytes) {
   if (!p) return;
   sync();
-  auto it = std::find(allocations_.begin(), allocations_.end(), p);
+  void *const freed = p;
+  p = nullptr;
+  auto it = std::find(allocations_.begin(), allocations_.end(), freed);
   if (it != allocations_.end()) allocations_.erase(it);
-  hip_check(hipFree(p), "hipFree");
   device_bytes_ -= (int64_t)bytes;
+  hip_check(hipFree(freed), "hipFree");
 }
 
 // The kernel for `loops` loops side by side (-1: the device cannot hold them).
@@ -1021,11 +1041,13 @@ void Model::push_loop(int kind, int shot, bool store) {
 
 void Model::ensure_loop_words() {
   if (loop_sync_) return;
-  loop_poison_ = (unsigned *)dalloc(1);
-  hip_check(hipHostMalloc((void **)&loop_status_, kLoopStatusWords * sizeof(unsigned),
-                          hipHostMallocDefault),
-            "hipHostMalloc");
-  std::memset(loop_status_, 0, kLoopStatusWords * sizeof(unsigned));
+  if (!loop_poison_) loop_poison_ = (unsigned *)dalloc(1);
+  if (!loop_status_) {
+    hip_check(hipHostMalloc((void **)&loop_status_, kLoopStatusWords * sizeof(unsigned),
+                            hipHostMallocDefault),
+              "hipHostMalloc");
+    std::memset(loop_status_, 0, kLoopStatusWords * sizeof(unsigned));
+  }
   loop_sync_ = (unsigned *)dalloc(2);  // two words for each stream's launches
 }
 
@@ -1035,11 +1057,13 @@ void Model::ensure_loop_room(int n, size_t cells, unsigned steps) {
   ensure_loop_words();
   if (loop_args_n_ < n) {
     release(loop_args_, loop_args_n_ * sizeof(LoopArgs));
+    loop_args_n_ = 0;
     loop_args_ = (LoopArgs *)dalloc(n * sizeof(LoopArgs) / 8);
     loop_args_n_ = n;
   }
   if (loop_cells_bytes_ < cells * n) {  // new cells are zero: no tag matches
     release(loop_cells_, loop_cells_bytes_);
+    loop_cells_bytes_ = 0;
     loop_cells_ = dalloc(cells * n / 8);
     loop_cells_bytes_ = cells * n;
     loop_tag_ = 1;
@@ -1210,15 +1234,9 @@ int Model::checkpoint_segments() const {
 void Model::ensure_segments() {
   const int k = ckpt_every_;
   if (seg_k_ < k) {  // two segment buffers of k snapshot slots
-    for (int f = 0; f < 5; ++f) {
-      if (seg_[f]) {
-        auto it = std::find(allocations_.begin(), allocations_.end(), (void *)seg_[f]);
-        if (it != allocations_.end()) allocations_.erase(it);
-        hip_check(hipFree(seg_[f]), "hipFree");
-        device_bytes_ -= (int64_t)(2LL * seg_k_ * ngrid_ * sizeof(double));
-      }
-      seg_[f] = dalloc((size_t)2 * k * ngrid_);
-    }
+    for (double *&seg : seg_) release(seg, 2 * (size_t)seg_k_ * ngrid_ * sizeof(double));
+    seg_k_ = 0;
+    dalloc_all(seg_, 5, 2 * (size_t)k * ngrid_);
     seg_k_ = k;
   }
   if (!lane_stream_) create_stream(&lane_stream_);
@@ -1243,9 +1261,8 @@ void Model::enqueue_checkpointed_adjoint(
     StepArgs &aa, int i_shot, std::vector<std::pair<hipEvent_t, hipEvent_t>> *pairs, int first,
     int parity) {
   const int nt = cfg_.nt, si = cfg_.snapshot_interval, k = ckpt_every_;
-  if (!state2_[0][0]) {
-    for (int p = 0; p < 2; ++p)
-      for (int f = 0; f < 5; ++f) state2_[p][f] = dalloc(npad_);
+  if (!state2_[0][0]) dalloc_all(&state2_[0][0], 10, npad_);
+  if (!scratch_off_) {
     // all-zero CSR offsets for the finest tiling (64 x 8 tiles)
     const long long max_tiles = (long long)ntx_ * ((d_.nz + 7) / 8);
     scratch_off_ = (int *)dalloc((size_t)(max_tiles + 2) / 2 + 1);
@@ -1500,8 +1517,7 @@ void Model::ensure_state_sets(int n) {
   bool added = false;
   for (int k = 2; k < n; ++k)
     if (!extra_state_[k - 2][0][0]) {
-      for (int p = 0; p < 2; ++p)
-        for (int f = 0; f < 5; ++f) extra_state_[k - 2][p][f] = dalloc(npad_);
+      dalloc_all(&extra_state_[k - 2][0][0], 10, npad_);
       added = true;
     }
   if (added) sync();
@@ -1562,7 +1578,7 @@ StepArgs Model::adjoint_launch_args(int i_shot, int parity) const {
 
 double *const *Model::shot_snapshot_store() {
   if (!shot_snap_[0]) {
-    for (int f = 0; f < 5; ++f) shot_snap_[f] = dalloc((size_t)d_.snapshots * ngrid_);
+    dalloc_all(shot_snap_, 5, (size_t)d_.snapshots * ngrid_);
     sync();
   }
   return shot_snap_;
@@ -1583,8 +1599,7 @@ void Model::state_arrays(int set, std::vector<double *> &out) const {
 
 void Model::ensure_second_state() {
   if (!lane_state_[0][0]) {
-    for (int p = 0; p < 2; ++p)
-      for (int f = 0; f < 5; ++f) lane_state_[p][f] = dalloc(npad_);
+    dalloc_all(&lane_state_[0][0], 10, npad_);
     sync();
   }
 }
@@ -1885,9 +1900,7 @@ void Model::run_model_two_lanes(bool adj) {
   const int ns = cfg_.n_shots, nt = cfg_.nt;
   ensure_snapshots();
   if (!lane_stream_) create_stream(&lane_stream_);
-  if (!lane_state_[0][0])
-    for (int p = 0; p < 2; ++p)
-      for (int f = 0; f < 5; ++f) lane_state_[p][f] = dalloc(npad_);
+  if (!lane_state_[0][0]) dalloc_all(&lane_state_[0][0], 10, npad_);
   while ((int)lane_events_.size() < ns + 3) {
     hipEvent_t e;
     hip_check(hipEventCreateWithFlags(&e, hipEventDisableTiming), "hipEventCreate");

@@ -14,6 +14,9 @@ extern "C" {
  * step instead. */
 int psv_refuse_resident_loops(psv_model *m);
 
+/* The model's allocation after the next n fails as if the device were full. */
+int psv_fail_allocation(psv_model *m, int n);
+
 #ifdef __cplusplus
 }
 #endif

@@ -1,0 +1,121 @@
+"""Calls that run out of device memory part of the way: the next call finds
+nothing half-built, and its outputs are those of a model that never failed."""
+import ctypes as C
+
+import numpy as np
+import pytest
+
+from test_gpu_resident_loop import _cfg, _fields, _gradient, _same
+
+pytestmark = pytest.mark.gpu
+
+
+def _fail(m, n):
+    """The model's allocation after the next n fails."""
+    from psvwave_amd import _lib
+    lib = _lib.load()
+    lib.psv_fail_allocation.argtypes = [C.c_void_p, C.c_int]
+    _lib.check(lib.psv_fail_allocation(m._h, n))
+
+
+def _run(m, cfg, seed, every=1):
+    import psvwave_amd
+    # (relative to the configuration's background, not to what m holds)
+    m.set_parameter_fields(*_fields(psvwave_amd.fdModel(cfg), seed))
+    rng = np.random.default_rng(9)
+    shape = (m.n_shots, m.nr, m.nt)
+    m.set_observed_data(rng.standard_normal(shape), rng.standard_normal(shape))
+    for s in range(m.n_shots):
+        m.forward_simulate(s)
+    m.calculate_l2_misfit()
+    m.calculate_l2_adjoint_sources()
+    m.reset_kernels()
+    for s in range(m.n_shots):
+        m.adjoint_simulate(s)
+    return [np.array(m.misfit), *m.get_synthetic_data(), *m.get_lame_kernels(),
+            *(m.get_snapshots() if every == 1 else ())]
+
+
+def _reference(cfg, seed):
+    import psvwave_amd
+    m = psvwave_amd.fdModel(cfg)
+    m.set_step_variant(27)
+    m.set_async(False)
+    return _run(m, cfg, seed)
+
+
+@pytest.mark.parametrize("variant", [None, 27])
+@pytest.mark.parametrize("n", [0, 1, 4])
+def test_snapshot_store(variant, n):
+    """The n-th of the five arrays of the store; by steps, of the second
+    lane's state first."""
+    import psvwave_amd
+    print(f"[allocation] store {variant} {n}", flush=True)
+    cfg = _cfg(131, 77, nt=60, shots=3)
+    m = psvwave_amd.fdModel(cfg)
+    if variant is not None:
+        m.set_step_variant(variant)
+        _fail(m, n)
+        with pytest.raises(RuntimeError, match="memory"):
+            m.forward_simulate(0, store_fields=False)
+        m.forward_simulate(0, store_fields=False)
+        m.synchronize()
+    _fail(m, n)
+    with pytest.raises(RuntimeError, match="memory"):
+        m.forward_simulate(0)
+        m.synchronize()
+    _same(_run(m, cfg, 6), _reference(cfg, 6), (variant, n))
+
+
+@pytest.mark.parametrize("n", [0, 1])
+def test_room_of_a_larger_launch(n):
+    """Three loops after a launch of one: their arguments, then their exchange
+    cells; a launch of one afterwards, then three again."""
+    import psvwave_amd
+    print(f"[allocation] room {n}", flush=True)
+    cfg = _cfg(131, 77, nt=60, shots=3)
+    m = psvwave_amd.fdModel(cfg)
+    m.forward_simulate(0)
+    m.synchronize()
+    _fail(m, n)
+    try:
+        for s in range(m.n_shots):
+            m.forward_simulate(s)
+        m.synchronize()
+    except RuntimeError as e:
+        assert "memory" in str(e)
+    for _ in range(70):  # past the forwards by steps that may follow
+        m.forward_simulate(0)
+        m.synchronize()
+    _same(_run(m, cfg, 6), _reference(cfg, 6), n)
+
+
+@pytest.mark.parametrize("variant, n", [(None, 0), (None, 3), (None, 4), (27, 0), (27, 9),
+                                        (27, 10), (27, 13)])
+def test_checkpoint_segments(variant, n):
+    """Segment buffers that grow; by steps the recomputation's state first."""
+    import psvwave_amd
+    print(f"[allocation] segments {variant} {n}", flush=True)
+    cfg = _cfg(131, 77, nt=60, shots=2)
+    m = psvwave_amd.fdModel(cfg)
+    if variant is not None:
+        m.set_step_variant(variant)
+    if variant is None:  # segments of two snapshots first
+        m.set_checkpointing(2)
+        _run(m, cfg, 7, 2)
+    m.set_checkpointing(5)
+    m.forward_simulate(0)
+    m.synchronize()
+    _fail(m, n)
+    with pytest.raises(RuntimeError, match="memory"):
+        m.adjoint_simulate(0)
+    if variant is None:  # smaller segments, then the larger ones
+        m.set_checkpointing(2)
+        _same(_run(m, cfg, 7, 2), _reference(cfg, 7)[:6], "smaller")
+        m.set_checkpointing(5)
+    _same(_run(m, cfg, 6, 5), _reference(cfg, 6)[:6], (variant, n))
+
+
+def test_nothing_changes_without_a_failure():
+    cfg = _cfg(131, 77, nt=60, shots=3)
+    _same(_gradient(cfg), _gradient(cfg, 27), "gradient")
