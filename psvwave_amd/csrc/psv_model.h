@@ -344,7 +344,9 @@ class Model {
   int loop_group(int limit);
   void push_loop(int kind, int shot, bool store);
   void flush_loops();
+  void launch_loops(int first, int n);
   void settle_loops();
+  void finish_loops();
   void redo_loops(const std::vector<LoopJob> &jobs);
   void run_resident(int kind, int i_shot, bool store);
   void enqueue_replay(const double *d, unsigned *status);

@@ -1021,8 +1021,6 @@ void Model::push_loop(int kind, int shot, bool store) {
             (fwd && loop_jobs_[i].shot == shot);
   if (apart) flush_loops();
   const int pending = (int)(loop_jobs_.size() - loop_launched_);
-  loop_jobs_.push_back({fwd ? kJobForward : pending ? kJobDeferred : kJobAdjoint, shot, store,
-                        pending - 1, 0});
   int together = loop_group(kLoopTogether);
   if (!fwd && together > 1) {
     // a buffer of kernel terms for all but the first: as many as the device
@@ -1033,9 +1031,16 @@ void Model::push_loop(int kind, int shot, bool store) {
            hipMemGetInfo(&free_b, &total_b) == hipSuccess &&
            (double)n * sizeof(double) + (double)(2ull << 30) <= (double)free_b &&
            (double)n * sizeof(double) * (double)(loop_defer_.size() + 1) <= 0.1 * (double)total_b)
-      loop_defer_.push_back(dalloc((size_t)n));
+      try {
+        loop_defer_.push_back(dalloc((size_t)n));
+      } catch (const RuntimeError &) {
+        break;  // (free memory in pieces)
+      }
     together = loop_group((int)loop_defer_.size() + 1);
   }
+  // queued last: where the above throws, this call has left nothing behind
+  loop_jobs_.push_back({fwd ? kJobForward : pending ? kJobDeferred : kJobAdjoint, shot, store,
+                        pending - 1, 0});
   if (pending + 1 >= together) flush_loops();
 }
 
@@ -1084,18 +1089,37 @@ void Model::refuse_next_loops() {
 }
 
 // Launches the pending jobs side by side, then adds deferred kernel terms.
+// Where that fails (the device has no room for the launch, say) they run by
+// steps at once, behind all jobs before them.
 void Model::flush_loops() {
   const int first = (int)loop_launched_, n = (int)loop_jobs_.size() - first;
   if (n == 0) return;
-  loop_launched_ = loop_jobs_.size();
   const bool fwd = loop_jobs_[first].kind == kJobForward;
+  // every job has its status word, still zero, before anything can fail
+  for (int i = 0; i < n; ++i) loop_jobs_[first + i].word = first;
+  for (int i = 1; i < n && !fwd; ++i)
+    loop_jobs_.push_back({kJobReplay, -1, false, loop_jobs_[first + i].defer,
+                          (int)loop_jobs_.size()});
+  loop_launched_ = loop_jobs_.size();
+  try {
+    launch_loops(first, n);
+    for (size_t r = first + n; r < loop_jobs_.size(); ++r)
+      enqueue_replay(loop_defer_[loop_jobs_[r].defer], loop_status_ + r);
+  } catch (const RuntimeError &) {
+    finish_loops();
+  }
+}
+
+// One launch of the n jobs from `first` on.
+void Model::launch_loops(int first, int n) {
+  const bool fwd = loop_jobs_[first].kind == kJobForward;
+  ensure_loop_words();
   const int kind = loop_kind(n);
   const LoopTables &t = loop_tables_[kind];
   const size_t cells = loop_cells_bytes(kind, t.tiles());
   ensure_loop_room(n, cells, (unsigned)cfg_.nt);
   for (int i = 0; i < n; ++i) {
-    LoopJob &j = loop_jobs_[first + i];
-    j.word = first;
+    const LoopJob &j = loop_jobs_[first + i];
     LoopArgs a = loop_args(kind, j.shot, fwd);
     a.slot_every = ckpt_every_;
     if ((j.store || !fwd) && snap_[0])
@@ -1122,13 +1146,6 @@ void Model::flush_loops() {
   gated_launch_loop(kind, !fwd, l, stream_);
   loop_tag_ += (unsigned)cfg_.nt;
   launches_ += (int64_t)n * cfg_.nt;
-  for (int i = 1; i < n && !fwd; ++i) {
-    const LoopJob r = {kJobReplay, -1, false, loop_jobs_[first + i].defer,
-                       (int)loop_jobs_.size()};
-    loop_jobs_.push_back(r);
-    ++loop_launched_;
-    enqueue_replay(loop_defer_[r.defer], loop_status_ + r.word);
-  }
 }
 
 // The kernel terms deferred to d, in their adjoint's order.
@@ -1144,8 +1161,14 @@ void Model::enqueue_replay(const double *d, unsigned *status) {
 }
 
 void Model::settle_loops() {
-  if (loop_jobs_.empty()) return;
   flush_loops();
+  finish_loops();
+}
+
+// Waits for the launched jobs, which are all there are, and runs those that
+// did not take place.
+void Model::finish_loops() {
+  if (loop_jobs_.empty()) return;
   sync();
   std::vector<LoopJob> ended;
   ended.swap(loop_jobs_);
@@ -1157,12 +1180,15 @@ void Model::settle_loops() {
 // step by step, in order.  A resident loop does not take place when its
 // blocks were not resident together in time (another process holds part of
 // the device); it then sets the poison word, at which every job after it
-// does nothing either.
+// does nothing either.  The last launch may also not have been enqueued.
 // The next jobs then run step by step from the start, since whoever holds
 // the device is likely still there.
 void Model::redo_loops(const std::vector<LoopJob> &jobs) {
-  const std::vector<unsigned> ran(loop_status_, loop_status_ + jobs.size());
-  std::memset(loop_status_, 0, jobs.size() * sizeof(unsigned));
+  std::vector<unsigned> ran(jobs.size(), kLoopNotRun);
+  if (loop_status_) {
+    std::copy_n(loop_status_, jobs.size(), ran.begin());
+    std::memset(loop_status_, 0, jobs.size() * sizeof(unsigned));
+  }
   bool missing = false;
   for (const LoopJob &j : jobs) {
     if (ran[j.word] == kLoopStalled)
@@ -1174,7 +1200,8 @@ void Model::redo_loops(const std::vector<LoopJob> &jobs) {
     return;
   }
   loop_skip_ = kLoopSkip;
-  hip_check(launch_fill((double *)loop_poison_, 1, 0.0, stream_), "clear poison");
+  if (loop_poison_)
+    hip_check(launch_fill((double *)loop_poison_, 1, 0.0, stream_), "clear poison");
   for (const LoopJob &j : jobs) {
     if (ran[j.word] != kLoopNotRun) continue;
     if (j.kind == kJobReplay) {

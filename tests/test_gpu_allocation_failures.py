@@ -119,3 +119,46 @@ def test_checkpoint_segments(variant, n):
 def test_nothing_changes_without_a_failure():
     cfg = _cfg(131, 77, nt=60, shots=3)
     _same(_gradient(cfg), _gradient(cfg, 27), "gradient")
+
+
+@pytest.mark.parametrize("n", [0, 1])
+def test_loops_without_room_run_by_steps(n):
+    """No room for the arguments or the cells of three loops: the calls, which
+    were all accepted, run by steps."""
+    import psvwave_amd
+    print(f"[allocation] forwards {n}", flush=True)
+    cfg = _cfg(131, 77, nt=60, shots=3)
+    m = psvwave_amd.fdModel(cfg)
+    m.forward_simulate(0)
+    m.synchronize()
+    m.set_parameter_fields(*_fields(psvwave_amd.fdModel(cfg), 6))
+    _fail(m, n)
+    for s in range(m.n_shots):
+        m.forward_simulate(s)
+    want = _reference(cfg, 6)
+    _same([*m.get_synthetic_data(), *m.get_snapshots()], want[1:3] + want[6:], n)
+
+
+@pytest.mark.parametrize("n", [0, 1, 2, 3])
+def test_adjoints_without_room(n):
+    """Three adjoints after single forwards: no room for the first or second
+    buffer of deferred kernel terms (fewer then share a launch), or for the
+    arguments or cells of three loops (all by steps, terms in their order)."""
+    import psvwave_amd
+    print(f"[allocation] adjoints {n}", flush=True)
+    cfg = _cfg(131, 77, nt=60, shots=3)
+    m = psvwave_amd.fdModel(cfg)
+    m.set_parameter_fields(*_fields(m, 6))
+    rng = np.random.default_rng(9)
+    shape = (m.n_shots, m.nr, m.nt)
+    m.set_observed_data(rng.standard_normal(shape), rng.standard_normal(shape))
+    for s in range(m.n_shots):
+        m.forward_simulate(s)
+        m.synchronize()
+    m.calculate_l2_adjoint_sources()
+    m.reset_kernels()
+    _fail(m, n)
+    for s in range(m.n_shots):
+        m.adjoint_simulate(s)
+    _same(m.get_lame_kernels(), _reference(cfg, 6)[3:6], n)
+    _same(_run(m, cfg, 7), _reference(cfg, 7), "afterwards")
