@@ -85,6 +85,9 @@ class Batch {
   void clear_gradient_tables();
   // Resident loops (psv_loop.h), the default when every member fits the
   // device: the loops of a call packed into as few launches as hold them.
+  struct DeviceFree {
+    void operator()(void *p) const { (void)hipFree(p); }
+  };
   struct LoopRef {
     int member, shot;
     bool forward, snaps;
@@ -95,14 +98,15 @@ class Batch {
     std::vector<LoopRef> loops;                // in launch order
     std::vector<std::pair<int, int>> launches; // first loop, blocks
     std::vector<int> first_block;              // of each launch
-    LoopArgs *args = nullptr;
-    int4 *blocks = nullptr;
+    std::unique_ptr<LoopArgs, DeviceFree> args;
+    std::unique_ptr<int4, DeviceFree> blocks;
   };
   int choose_loop_kind(int shots);
   bool resident_available();
   LoopLaunches *loop_launches(int which, int i_shot, int steps);
+  LoopLaunches plan_loops(int which, int i_shot, int steps);
+  void ensure_loop_words(int launches);
   void run_loops(LoopLaunches &p, int steps);
-  void clear_loops();
   void end_timing();
   bool resident_ = true;  // until a step variant is chosen
   int loop_skip_ = 0;     // calls still to run step by step after a refused launch

@@ -16,8 +16,19 @@ namespace psv {
 
 namespace {
 void hip_check(hipError_t e, const char *what) {
-  if (e != hipSuccess)
-    throw RuntimeError(std::string(what) + ": " + hipGetErrorString(e));
+  if (e == hipSuccess) return;
+  (void)hipGetLastError();  // reported here, not by the check of a later launch
+  throw RuntimeError(std::string(what) + ": " + hipGetErrorString(e));
+}
+
+// n doubles of device memory, zero in the stream's order.
+void *zeroed(size_t n, hipStream_t s) {
+  void *p = nullptr;
+  hip_check(hipMalloc(&p, n * sizeof(double)), "hipMalloc");
+  const hipError_t e = launch_fill((double *)p, (long long)n, 0.0, s);
+  if (e != hipSuccess) (void)hipFree(p);
+  hip_check(e, "zero-fill");
+  return p;
 }
 }  // namespace
 
@@ -57,7 +68,7 @@ Batch::~Batch() {
     if (p) (void)hipFree(p);
   if (zero_lens_) (void)hipFree(zero_lens_);
   clear_gradient_tables();
-  clear_loops();
+  loops_.clear();
   if (loop_cells_) (void)hipFree(loop_cells_);
   if (loop_sync_) (void)hipFree(loop_sync_);
   if (loop_poison_) (void)hipFree(loop_poison_);
@@ -214,14 +225,6 @@ void Batch::enqueue_loop(int i_shot, int nsteps) {
 
 // ---- resident loops ----
 
-void Batch::clear_loops() {
-  for (auto &kv : loops_) {
-    if (kv.second.args) (void)hipFree(kv.second.args);
-    if (kv.second.blocks) (void)hipFree(kv.second.blocks);
-  }
-  loops_.clear();
-}
-
 // The kernel for launches of `shots` loops of every member: the first that
 // holds them all (kLoopFits), or where several launches are needed 28-row tiles,
 // two blocks per compute unit: the blocks of a unit mostly belong to different
@@ -264,12 +267,27 @@ bool Batch::resident_available() {
   return loop_kind_ >= 0;
 }
 
-// The launches of a call, built on first use.  which: 0 forward_all, 1
-// forward of i_shot, 2 / 3 forward / adjoint of i_shot with the one-shot
-// snapshot stores, 4 the first `steps` steps of forward_all.
+// The launches of a call, built on first use and kept only once they are
+// whole.  Null where the device has no room for them: the call then runs by
+// steps, and the next one tries again.
 Batch::LoopLaunches *Batch::loop_launches(int which, int i_shot, int steps) {
-  LoopLaunches &p = loops_[which + 8 * i_shot];
-  if (p.kind >= 0 && which != 4) return &p;
+  const int key = which + 8 * i_shot;
+  auto it = loops_.find(key);
+  if (it != loops_.end() && which != 4) return &it->second;
+  hip_check(hipStreamSynchronize(stream_), "sync");
+  try {
+    LoopLaunches p = plan_loops(which, i_shot, steps);
+    ensure_loop_words((int)p.launches.size());
+    return &(loops_[key] = std::move(p));
+  } catch (const RuntimeError &) {
+    return nullptr;
+  }
+}
+
+// which: 0 forward_all, 1 forward of i_shot, 2 / 3 forward / adjoint of i_shot
+// with the one-shot snapshot stores, 4 the first `steps` steps of forward_all.
+Batch::LoopLaunches Batch::plan_loops(int which, int i_shot, int steps) {
+  LoopLaunches p;
   // (a launch of one shot may have room for smaller tiles than one of all)
   const int kind = p.kind = which == 0 || which == 4 ? loop_kind_ : choose_loop_kind(1);
   p.forward = which != 3;
@@ -297,17 +315,13 @@ Batch::LoopLaunches *Batch::loop_launches(int which, int i_shot, int steps) {
     bins[b].push_back(r);
     room[b] -= tiles(r);
   }
-  p.loops.clear(), p.launches.clear(), p.first_block.clear();
-  const int cap = loop_capacity(kind);
   const size_t cell_bytes = loop_cells_bytes(kind, 1);
   if (!loop_cells_) {  // for every kernel: the launches of all calls keep pointers into them
     size_t bytes = 0;
     for (int k = 0; k < kNumLoopKinds; ++k)
       bytes = std::max(bytes, loop_cells_bytes(k, loop_capacity(k)));
-    hip_check(hipMalloc(&loop_cells_, bytes), "hipMalloc");
+    loop_cells_ = zeroed(bytes / 8, stream_);
     loop_cells_bytes_ = bytes;
-    hip_check(launch_fill((double *)loop_cells_, (long long)(bytes / 8), 0.0, stream_),
-              "clear cells");
   }
   std::vector<LoopArgs> args;
   std::vector<int4> blocks;
@@ -333,35 +347,37 @@ Batch::LoopLaunches *Batch::loop_launches(int which, int i_shot, int steps) {
     p.launches.emplace_back(first, (int)blocks.size() - block0);
     p.first_block.push_back(block0);
   }
-  auto put = [&](auto *&dst, const auto &v) {
-    hip_check(hipStreamSynchronize(stream_), "sync");
-    if (dst) hip_check(hipFree(dst), "hipFree");
-    dst = nullptr;
-    hip_check(hipMalloc((void **)&dst, v.size() * sizeof(v[0])), "hipMalloc");
-    hip_check(hipMemcpy(dst, v.data(), v.size() * sizeof(v[0]), hipMemcpyHostToDevice), "upload");
+  auto put = [&](auto &dst, const auto &v) {
+    void *d = nullptr;
+    hip_check(hipMalloc(&d, v.size() * sizeof(v[0])), "hipMalloc");
+    dst.reset((typename std::remove_reference_t<decltype(dst)>::pointer)d);
+    hip_check(hipMemcpy(d, v.data(), v.size() * sizeof(v[0]), hipMemcpyHostToDevice), "upload");
   };
   put(p.args, args);
   put(p.blocks, blocks);
-  const int n = (int)p.launches.size();
-  if (n > loop_words_) {
-    if (loop_sync_) hip_check(hipFree(loop_sync_), "hipFree");
-    if (loop_status_) hip_check(hipHostFree(loop_status_), "hipHostFree");
-    loop_sync_ = loop_status_ = nullptr;
-    loop_words_ = 0;
-    hip_check(hipMalloc((void **)&loop_sync_, (size_t)n * 8), "hipMalloc");
-    hip_check(hipHostMalloc((void **)&loop_status_, n * sizeof(unsigned), hipHostMallocDefault),
-              "hipHostMalloc");
-    loop_words_ = n;
-  }
-  if (!loop_poison_) {
-    hip_check(hipMalloc((void **)&loop_poison_, 8), "hipMalloc");
-    hip_check(launch_fill((double *)loop_poison_, 1, 0.0, stream_), "clear poison");
-  }
-  return &p;
+  return p;
+}
+
+// Meeting and status words of as many launches, and the poison word.
+void Batch::ensure_loop_words(int launches) {
+  if (!loop_poison_) loop_poison_ = (unsigned *)zeroed(1, stream_);
+  if (launches <= loop_words_) return;
+  // the words there are go last: launches already planned use them
+  void *sync = nullptr, *status = nullptr;
+  hip_check(hipMalloc(&sync, (size_t)launches * 8), "hipMalloc");
+  const hipError_t e = hipHostMalloc(&status, launches * sizeof(unsigned), hipHostMallocDefault);
+  if (e != hipSuccess) (void)hipFree(sync);
+  hip_check(e, "hipHostMalloc");
+  if (loop_sync_) (void)hipFree(loop_sync_);
+  if (loop_status_) (void)hipHostFree(loop_status_);
+  loop_sync_ = (unsigned *)sync;
+  loop_status_ = (unsigned *)status;
+  loop_words_ = launches;
 }
 
 // Runs the launches of a call (`steps` time steps each) and waits for them;
-// loops whose launch was refused (psv_loop.h) run step by step.
+// loops whose launch was refused (psv_loop.h) or could not be made run step by
+// step.
 void Batch::run_loops(LoopLaunches &p, int steps) {
   const int n = (int)p.launches.size();
   for (int i = 0; i < n; ++i) loop_status_[i] = kLoopNotRun;
@@ -374,14 +390,18 @@ void Batch::run_loops(LoopLaunches &p, int steps) {
       loop_tag_ = 1;
     }
     LoopLaunch l;
-    l.loops = p.args + p.launches[i].first;
-    l.blocks = p.blocks + p.first_block[i];
+    l.loops = p.args.get() + p.launches[i].first;
+    l.blocks = p.blocks.get() + p.first_block[i];
     l.nblocks = p.launches[i].second;
     l.tag0 = loop_tag_;
     l.sync = loop_sync_ + 2 * i;
     l.poison = loop_poison_;
     l.status = loop_status_ + i;
-    gated_launch_loop(p.kind, !p.forward, l, stream_);
+    try {
+      gated_launch_loop(p.kind, !p.forward, l, stream_);
+    } catch (const RuntimeError &) {
+      break;
+    }
     loop_tag_ += (unsigned)steps;
   }
   hip_check(hipStreamSynchronize(stream_), "hipStreamSynchronize");
@@ -407,8 +427,7 @@ void Batch::run_loops(LoopLaunches &p, int steps) {
 void Batch::forward(int i_shot) {
   if (i_shot < 0 || i_shot >= n_shots_)
     throw ValueError("i_shot is outside [0, n_shots)");
-  if (resident_available()) {
-    LoopLaunches *p = loop_launches(1, i_shot, nt_);
+  if (LoopLaunches *p = resident_available() ? loop_launches(1, i_shot, nt_) : nullptr) {
     hip_check(hipEventRecord(ev_[0], stream_), "hipEventRecord");
     run_loops(*p, nt_);
     end_timing();
@@ -499,8 +518,7 @@ void Batch::end_timing() {
 }
 
 void Batch::forward_all() {
-  if (resident_available()) {
-    LoopLaunches *p = loop_launches(0, 0, nt_);
+  if (LoopLaunches *p = resident_available() ? loop_launches(0, 0, nt_) : nullptr) {
     hip_check(hipEventRecord(ev_[0], stream_), "hipEventRecord");
     run_loops(*p, nt_);
     end_timing();
@@ -573,7 +591,10 @@ void Batch::gradients() {
   if (nt_ % si_ != 0)
     throw ValueError("Snapshot interval and size of accumulator don't match! "
                      "(nt must be a multiple of snapshot_interval)");
-  const bool resident = resident_available();
+  // everything is allocated before anything is changed
+  bool resident = resident_available();
+  for (int s = 0; s < n_shots_ && resident; ++s)
+    resident = loop_launches(2, s, nt_) && loop_launches(3, s, nt_);
   if (!resident && !gfwd_) {
     std::vector<StepArgs> f, a;
     for (auto &m : models_) {
@@ -585,12 +606,17 @@ void Batch::gradients() {
           for (int q = 0; q < 5; ++q) f.back().snap[q] = a.back().snap[q] = store[q];
         }
     }
-    hip_check(hipMalloc((void **)&gfwd_, f.size() * sizeof(StepArgs)), "hipMalloc");
-    hip_check(hipMalloc((void **)&gadj_, a.size() * sizeof(StepArgs)), "hipMalloc");
-    hip_check(hipMemcpy(gfwd_, f.data(), f.size() * sizeof(StepArgs), hipMemcpyHostToDevice),
-              "upload");
-    hip_check(hipMemcpy(gadj_, a.data(), a.size() * sizeof(StepArgs), hipMemcpyHostToDevice),
-              "upload");
+    try {
+      hip_check(hipMalloc((void **)&gfwd_, f.size() * sizeof(StepArgs)), "hipMalloc");
+      hip_check(hipMalloc((void **)&gadj_, a.size() * sizeof(StepArgs)), "hipMalloc");
+      hip_check(hipMemcpy(gfwd_, f.data(), f.size() * sizeof(StepArgs), hipMemcpyHostToDevice),
+                "upload");
+      hip_check(hipMemcpy(gadj_, a.data(), a.size() * sizeof(StepArgs), hipMemcpyHostToDevice),
+                "upload");
+    } catch (...) {
+      clear_gradient_tables();
+      throw;
+    }
   }
   for (auto &m : models_) m->reset_kernels();
   hip_check(hipEventRecord(ev_[0], stream_), "hipEventRecord");
@@ -668,9 +694,8 @@ double Batch::autotune(int steps, int *best, double *ms_per_variant) {
   if (best) *best = best_v;
   // resident loops where they are faster still
   resident_ = true;
-  if (resident_available()) {
-    const int n = std::min(steps, nt_);
-    LoopLaunches *p = loop_launches(4, 0, n);
+  const int n = std::min(steps, nt_);
+  if (LoopLaunches *p = resident_available() ? loop_launches(4, 0, n) : nullptr) {
     run_loops(*p, n);  // warm up
     hip_check(hipEventRecord(ev_[0], stream_), "hipEventRecord");
     run_loops(*p, n);

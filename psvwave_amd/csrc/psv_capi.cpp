@@ -571,8 +571,8 @@ int psv_synchronize(psv_model *m) {
   return guard([&] { M(m); });
 }
 
-int psv_fail_allocation(psv_model *m, int n) {
-  return guard([&] { MA(m).fail_allocation(n); });
+int psv_fail_allocation(psv_model *m, int n, int times) {
+  return guard([&] { MA(m).fail_allocation(n, times); });
 }
 
 int psv_refuse_resident_loops(psv_model *m) {
@@ -763,6 +763,10 @@ int psv_batch_lockstep(psv_batch *b, int *on) {
     need(on, "on");
     *on = B(b).lockstep_available() ? 1 : 0;
   });
+}
+
+int psv_batch_fail_allocation(psv_batch *b, int m, int n, int times) {
+  return guard([&] { B(b).model(m).fail_allocation(n, times); });
 }
 
 int psv_batch_resident(psv_batch *b, int *on) {

@@ -112,8 +112,8 @@ class Model {
   }
   void reset_step_timing() { timed_ms_ = 0, timed_ = 0, launches_ = 0; }
   int64_t device_bytes() const { return device_bytes_; }
-  // As if the device were full at the allocation after the next n (tests).
-  void fail_allocation(int n) { fail_allocation_ = n; }
+  // As if the device were full at `times` allocations after the next n (tests).
+  void fail_allocation(int n, int times) { fail_after_ = n, fail_times_ = times; }
   // As if another process held part of the device: the blocks of the next
   // resident launches leave at once and their loops run step by step (tests).
   void refuse_next_loops();
@@ -195,7 +195,7 @@ class Model {
   bool owns_stream_ = true;
   std::vector<void *> allocations_;
   int64_t device_bytes_ = 0;
-  int fail_allocation_ = -1;
+  int fail_after_ = 0, fail_times_ = 0;
 
   double *state_[2][5] = {};  // ping-pong: vx, vz, txx, tzz, txz (padded)
   double *lm_ = nullptr, *mu_ = nullptr, *b_ = nullptr;  // padded

@@ -139,7 +139,7 @@ Model::~Model() {
 double *Model::dalloc(size_t n) {
   void *p = nullptr;
   size_t bytes = std::max<size_t>(n, 1) * sizeof(double);
-  const bool fail = fail_allocation_ >= 0 && fail_allocation_-- == 0;
+  const bool fail = fail_times_ > 0 && fail_after_-- <= 0 && fail_times_-- > 0;
   hip_check(fail ? hipErrorOutOfMemory : hipMalloc(&p, bytes), "hipMalloc");
   allocations_.push_back(p);
   device_bytes_ += (int64_t)bytes;

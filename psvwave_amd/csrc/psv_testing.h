@@ -14,8 +14,10 @@ extern "C" {
  * step instead. */
 int psv_refuse_resident_loops(psv_model *m);
 
-/* The model's allocation after the next n fails as if the device were full. */
-int psv_fail_allocation(psv_model *m, int n);
+/* `times` allocations of the model (of member m of the batch) after the next n
+ * fail as if the device were full. */
+int psv_fail_allocation(psv_model *m, int n, int times);
+int psv_batch_fail_allocation(psv_batch *b, int m, int n, int times);
 
 #ifdef __cplusplus
 }

@@ -5,7 +5,7 @@ import ctypes as C
 import numpy as np
 import pytest
 
-from test_gpu_resident_loop import _cfg, _fields, _gradient, _same
+from test_gpu_resident_loop import _batch, _cfg, _fields, _gradient, _same
 
 pytestmark = pytest.mark.gpu
 
@@ -14,8 +14,8 @@ def _fail(m, n):
     """The model's allocation after the next n fails."""
     from psvwave_amd import _lib
     lib = _lib.load()
-    lib.psv_fail_allocation.argtypes = [C.c_void_p, C.c_int]
-    _lib.check(lib.psv_fail_allocation(m._h, n))
+    lib.psv_fail_allocation.argtypes = [C.c_void_p, C.c_int, C.c_int]
+    _lib.check(lib.psv_fail_allocation(m._h, n, 1))
 
 
 def _run(m, cfg, seed, every=1):
@@ -162,3 +162,31 @@ def test_adjoints_without_room(n):
         m.adjoint_simulate(s)
     _same(m.get_lame_kernels(), _reference(cfg, 6)[3:6], n)
     _same(_run(m, cfg, 7), _reference(cfg, 7), "afterwards")
+
+
+@pytest.mark.parametrize("n, times", [(0, 1), (3, 1), (0, 2), (0, 3), (3, 2)])
+def test_batch_gradients(n, times):
+    """The second member's snapshot store: after one failure the call runs by
+    steps, after a second it is raised and leaves the kernels as they were,
+    and the next one builds its launches anew."""
+    from psvwave_amd import _lib
+    print(f"[allocation] batch {n} {times}", flush=True)
+    lib = _lib.load()
+    lib.psv_batch_fail_allocation.argtypes = [C.c_void_p, C.c_int, C.c_int, C.c_int]
+    cfgs = [_cfg(133, 71, shots=2, nt=40), _cfg(90, 61, shots=2, nt=40)]
+    want = _batch(cfgs, 28)
+    misfits = want.gradients()
+    b = _batch(cfgs)
+    zero = [b.get_kernels(m) for m in range(2)]
+    # (a store that failed is tried again from its first array)
+    _lib.check(lib.psv_batch_fail_allocation(b._h, 1, n, times))
+    if times > 1:
+        with pytest.raises(RuntimeError, match="memory"):
+            b.gradients()
+        for m in range(2):
+            _same(b.get_kernels(m), zero[m], "untouched")
+    for k in range(3):
+        _same([b.gradients()], [misfits], (n, times, k))
+        for m in range(2):
+            _same(b.get_kernels(m), want.get_kernels(m), (n, times, k, m))
+    assert b.resident()
