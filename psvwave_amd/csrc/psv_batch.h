@@ -50,6 +50,7 @@ class Batch {
   // Seismograms are those of forward(0), forward(1), ... bit for bit.
   void forward_all();
   bool lockstep_available();
+  void refuse_next_loops();  // as Model's (tests)
   bool runs_resident() { return loop_skip_ == 0 && resident_available(); }
   // Per-member L2 misfit over all shots (calculate_l2_misfit of each).
   void misfits(double *out);

@@ -375,6 +375,16 @@ void Batch::ensure_loop_words(int launches) {
   loop_words_ = launches;
 }
 
+// The next launches are refused, whatever the step variant.
+void Batch::refuse_next_loops() {
+  ensure_loop_words(0);
+  hip_check(hipStreamSynchronize(stream_), "sync");
+  const unsigned one = 1;
+  hip_check(hipMemcpy(loop_poison_, &one, sizeof(one), hipMemcpyHostToDevice), "poison");
+  resident_ = true;
+  loop_skip_ = 0;
+}
+
 // Runs the launches of a call (`steps` time steps each) and waits for them;
 // loops whose launch was refused (psv_loop.h) or could not be made run step by
 // step.

@@ -765,6 +765,10 @@ int psv_batch_lockstep(psv_batch *b, int *on) {
   });
 }
 
+int psv_batch_refuse_resident_loops(psv_batch *b) {
+  return guard([&] { B(b).refuse_next_loops(); });
+}
+
 int psv_batch_fail_allocation(psv_batch *b, int m, int n, int times) {
   return guard([&] { B(b).model(m).fail_allocation(n, times); });
 }

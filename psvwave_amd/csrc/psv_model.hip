@@ -1222,11 +1222,14 @@ void Model::redo_loops(const std::vector<LoopJob> &jobs) {
 void Model::enqueue_loop_by_steps(int shot, bool forward, bool snaps, const SlotFn &slot,
                                   double *defer) {
   StepArgs a = forward ? forward_args(shot) : adjoint_args(shot);
-  a.rec_increments = 0;
+  // a batch's members may run a two-step kernel, whose receivers record
+  // increments (enqueue_loop)
+  a.rec_increments = forward && step_is_two_step(variant_) ? 1 : 0;
   a.rec_off = adj_off_;
   a.rec_entries = adj_entries_;
   enqueue_zero_state(stream_);
   enqueue_range(a, state_, 0, forward, 0, cfg_.nt, snaps, slot, nullptr, false, stream_, defer);
+  if (a.rec_increments) enqueue_receiver_scan(shot, stream_);
 }
 
 void Model::enqueue_store_loop(int i_shot, bool forward, bool snaps) {

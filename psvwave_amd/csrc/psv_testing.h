@@ -13,6 +13,9 @@ extern "C" {
  * of the device, that their blocks are not resident together, and run step by
  * step instead. */
 int psv_refuse_resident_loops(psv_model *m);
+/* The same of a batch, which then starts resident loops under any step
+ * variant. */
+int psv_batch_refuse_resident_loops(psv_batch *b);
 
 /* `times` allocations of the model (of member m of the batch) after the next n
  * fail as if the device were full. */
