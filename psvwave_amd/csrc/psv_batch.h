@@ -107,7 +107,7 @@ class Batch {
   LoopLaunches *loop_launches(int which, int i_shot, int steps);
   LoopLaunches plan_loops(int which, int i_shot, int steps);
   void ensure_loop_words(int launches);
-  void run_loops(LoopLaunches &p, int steps);
+  bool run_loops(LoopLaunches &p, int steps, bool redo = true);
   void end_timing();
   bool resident_ = true;  // until a step variant is chosen
   int loop_skip_ = 0;     // calls still to run step by step after a refused launch

@@ -385,10 +385,10 @@ void Batch::refuse_next_loops() {
   loop_skip_ = 0;
 }
 
-// Runs the launches of a call (`steps` time steps each) and waits for them;
-// loops whose launch was refused (psv_loop.h) or could not be made run step by
-// step.
-void Batch::run_loops(LoopLaunches &p, int steps) {
+// Runs the launches of a call (`steps` time steps each) and waits for them:
+// whether all took place.  Those that were refused (psv_loop.h) or could not be
+// made are, with `redo`, run step by step as whole loops.
+bool Batch::run_loops(LoopLaunches &p, int steps, bool redo) {
   const int n = (int)p.launches.size();
   for (int i = 0; i < n; ++i) loop_status_[i] = kLoopNotRun;
   hip_check(launch_fill((double *)loop_sync_, n, 0.0, stream_), "clear loop words");
@@ -421,10 +421,10 @@ void Batch::run_loops(LoopLaunches &p, int steps) {
       throw RuntimeError("a resident time loop made no progress");
     missing = missing || loop_status_[i] == kLoopNotRun;
   }
-  if (!missing) return;
+  if (!missing) return true;
   loop_skip_ = 64;
   hip_check(launch_fill((double *)loop_poison_, 1, 0.0, stream_), "clear poison");
-  for (int i = 0; i < n; ++i) {
+  for (int i = 0; i < n && redo; ++i) {
     if (loop_status_[i] != kLoopNotRun) continue;
     const int last = i + 1 < n ? p.launches[i + 1].first : (int)p.loops.size();
     for (int k = p.launches[i].first; k < last; ++k)
@@ -432,6 +432,7 @@ void Batch::run_loops(LoopLaunches &p, int steps) {
                                                      p.loops[k].snaps);
   }
   hip_check(hipStreamSynchronize(stream_), "hipStreamSynchronize");
+  return false;
 }
 
 void Batch::forward(int i_shot) {
@@ -702,21 +703,22 @@ double Batch::autotune(int steps, int *best, double *ms_per_variant) {
   }
   set_variant(best_v, keep_remap);
   if (best) *best = best_v;
-  // resident loops where they are faster still
+  // resident loops where they are faster still; not where a launch is refused,
+  // since whoever holds the device is likely still there
   resident_ = true;
   const int n = std::min(steps, nt_);
-  if (LoopLaunches *p = resident_available() ? loop_launches(4, 0, n) : nullptr) {
-    run_loops(*p, n);  // warm up
+  LoopLaunches *const p = resident_available() ? loop_launches(4, 0, n) : nullptr;
+  bool faster = p && run_loops(*p, n, false);  // warm up
+  if (faster) {
     hip_check(hipEventRecord(ev_[0], stream_), "hipEventRecord");
-    run_loops(*p, n);
+    faster = run_loops(*p, n, false);
     hip_check(hipEventRecord(ev_[1], stream_), "hipEventRecord");
     hip_check(hipStreamSynchronize(stream_), "hipStreamSynchronize");
     float ms = 0.f;
     hip_check(hipEventElapsedTime(&ms, ev_[0], ev_[1]), "hipEventElapsedTime");
-    resident_ = ms / (n * n_shots_) < best_ms;
-  } else {
-    resident_ = false;
+    faster = faster && ms / (n * n_shots_) < best_ms;
   }
+  resident_ = faster;
   return best_ms;
 }
 

@@ -75,3 +75,16 @@ def test_the_end_of_the_stepwise_calls():
         if k in (0, 1, 62, 63, 64, 65, 69):
             _same(_traces(b), _traces(want), k)
     assert b.resident()
+
+
+def test_autotune_goes_on_by_steps():
+    print("[refused] autotune", flush=True)
+    cfgs = _configs(40)
+    want = _batch(cfgs, 28)
+    want.forward_all()
+    b = _batch(cfgs)
+    _refuse(b)
+    b.autotune(steps=6)
+    assert not b.resident()
+    b.forward_all()
+    _same(_traces(b), _traces(want), "autotune")
