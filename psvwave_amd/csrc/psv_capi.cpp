@@ -575,6 +575,13 @@ int psv_fail_allocation(psv_model *m, int n, int times) {
   return guard([&] { MA(m).fail_allocation(n, times); });
 }
 
+int psv_resident_rows(psv_model *m, int loops, int *rows) {
+  return guard([&] {
+    need(rows, "rows");
+    *rows = M(m).resident_rows(loops);
+  });
+}
+
 int psv_refuse_resident_loops(psv_model *m) {
   return guard([&] { M(m).refuse_next_loops(); });
 }

@@ -114,6 +114,11 @@ class Model {
   int64_t device_bytes() const { return device_bytes_; }
   // As if the device were full at `times` allocations after the next n (tests).
   void fail_allocation(int n, int times) { fail_after_ = n, fail_times_ = times; }
+  // Rows of the tiles on which `loops` loops run side by side (0: by steps).
+  int resident_rows(int loops) {
+    const int kind = resident_path(false) ? loop_kind(loops) : -1;
+    return kind < 0 ? 0 : loop_tile_rows(kind);
+  }
   // As if another process held part of the device: the blocks of the next
   // resident launches leave at once and their loops run step by step (tests).
   void refuse_next_loops();

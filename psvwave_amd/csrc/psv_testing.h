@@ -1,6 +1,6 @@
-/* psv_testing.h -- entry points that the tests force conditions with, which a
- * program has no use for and the public header therefore does not declare.
- * They act on one object and leave every result as it is. */
+/* psv_testing.h -- entry points with which the tests force a condition or learn
+ * of a choice; a program has no use for them, so the public header does not
+ * declare them.  They act on one object and leave every result as it is. */
 #pragma once
 
 #include "../../include/psvwave.h"
@@ -17,6 +17,9 @@ int psv_refuse_resident_loops(psv_model *m);
  * variant. */
 int psv_batch_refuse_resident_loops(psv_batch *b);
 
+/* Rows of the tiles on which `loops` of the model's time loops run side by side;
+ * 0: they run by steps. */
+int psv_resident_rows(psv_model *m, int loops, int *rows);
 /* `times` allocations of the model (of member m of the batch) after the next n
  * fail as if the device were full. */
 int psv_fail_allocation(psv_model *m, int n, int times);
