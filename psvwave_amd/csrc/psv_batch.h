@@ -111,7 +111,7 @@ class Batch {
   void end_timing();
   bool resident_ = true;  // until a step variant is chosen
   int loop_skip_ = 0;     // calls still to run step by step after a refused launch
-  int loop_kind_ = -2;    // -2 not chosen, -1 some member does not fit
+  int loop_kind_ = -1;    // -1: not chosen, or some member does not fit
   std::map<int, LoopLaunches> loops_;
   void *loop_cells_ = nullptr;
   size_t loop_cells_bytes_ = 0;

@@ -263,7 +263,7 @@ bool Batch::resident_available() {
     --loop_skip_;
     return false;
   }
-  if (loop_kind_ == -2) loop_kind_ = choose_loop_kind(n_shots_);
+  if (loop_kind_ < 0) loop_kind_ = choose_loop_kind(n_shots_);
   return loop_kind_ >= 0;
 }
 

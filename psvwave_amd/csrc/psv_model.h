@@ -174,6 +174,7 @@ class Model {
   std::vector<InjectionTerm> forward_terms(int shot) const;
   std::vector<InjectionTerm> adjoint_terms() const;
   void ensure_snapshots();
+  void *raw_alloc(size_t bytes);
   double *dalloc(size_t n);
   void dalloc_all(double **p, int count, size_t n);
   template <class T>

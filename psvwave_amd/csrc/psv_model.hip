@@ -136,13 +136,18 @@ Model::~Model() {
   if (owns_stream_) destroy_stream(stream_);
 }
 
-double *Model::dalloc(size_t n) {
+// Device memory that the model owns, its contents undefined.
+void *Model::raw_alloc(size_t bytes) {
   void *p = nullptr;
-  size_t bytes = std::max<size_t>(n, 1) * sizeof(double);
   const bool fail = fail_times_ > 0 && fail_after_-- <= 0 && fail_times_-- > 0;
   hip_check(fail ? hipErrorOutOfMemory : hipMalloc(&p, bytes), "hipMalloc");
   allocations_.push_back(p);
   device_bytes_ += (int64_t)bytes;
+  return p;
+}
+
+double *Model::dalloc(size_t n) {
+  void *const p = raw_alloc(std::max<size_t>(n, 1) * sizeof(double));
   hip_check(launch_fill((double *)p, (long long)std::max<size_t>(n, 1), 0.0,
                         stream_),
             "zero-fill");
@@ -943,28 +948,34 @@ bool Model::ensure_loop_tables(int kind) {
   const int loops = std::min(std::max(cfg_.n_shots, 1), loop_capacity(kind) / ntiles);
   for (int l = 0; l < loops; ++l)
     for (int i = 0; i < ntiles; ++i) blocks.push_back(make_int4(l, i % ntx, i / ntx, 0));
+  std::vector<std::pair<void *, size_t>> put_bytes;
   auto put = [&](auto *&dst, const auto &v) {
     const size_t bytes = std::max<size_t>(v.size() * sizeof(v[0]), 16);
-    void *p = nullptr;
-    hip_check(hipMalloc(&p, bytes), "hipMalloc");
-    allocations_.push_back(p);
-    device_bytes_ += (int64_t)bytes;
+    void *const p = raw_alloc(bytes);
+    put_bytes.emplace_back(p, bytes);
     dst = (typename std::remove_reference<decltype(dst)>::type)p;
     if (!v.empty())
       hip_check(hipMemcpy(p, v.data(), v.size() * sizeof(v[0]), hipMemcpyHostToDevice),
                 "upload");
   };
-  put(t.blocks, blocks);
-  put(t.fwd_off, foff);
-  put(t.fwd_first, ffirst);
-  put(t.fwd, fent);
-  put(t.fwd_head, fhead);
-  put(t.adj_off, aoff);
-  put(t.adj_first, afirst);
-  put(t.adj, aent);
-  put(t.adj_head, ahead);
-  put(t.rec_off, roff);
-  put(t.rec, rent);
+  try {
+    put(t.blocks, blocks);
+    put(t.fwd_off, foff);
+    put(t.fwd_first, ffirst);
+    put(t.fwd, fent);
+    put(t.fwd_head, fhead);
+    put(t.adj_off, aoff);
+    put(t.adj_first, afirst);
+    put(t.adj, aent);
+    put(t.adj_head, ahead);
+    put(t.rec_off, roff);
+    put(t.rec, rent);
+  } catch (const RuntimeError &) {
+    // no room now: another kernel or loops by steps, and another try next time
+    for (auto &b : put_bytes) release(b.first, b.second);
+    t = LoopTables();
+    return false;
+  }
   t.state = 1;
   return true;
 }

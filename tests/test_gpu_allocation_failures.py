@@ -18,6 +18,13 @@ def _fail(m, n):
     _lib.check(lib.psv_fail_allocation(m._h, n, 1))
 
 
+def _warm(m):
+    """The tables of the resident loops, which count as allocations too."""
+    for s in range(m.n_shots):
+        m.forward_simulate(s, store_fields=False)
+    m.synchronize()
+
+
 def _run(m, cfg, seed, every=1):
     import psvwave_amd
     # (relative to the configuration's background, not to what m holds)
@@ -60,6 +67,8 @@ def test_snapshot_store(variant, n):
             m.forward_simulate(0, store_fields=False)
         m.forward_simulate(0, store_fields=False)
         m.synchronize()
+    else:
+        _warm(m)
     _fail(m, n)
     with pytest.raises(RuntimeError, match="memory"):
         m.forward_simulate(0)
@@ -177,6 +186,8 @@ def test_batch_gradients(n, times):
     want = _batch(cfgs, 28)
     misfits = want.gradients()
     b = _batch(cfgs)
+    b.forward_all()
+    b.forward(0)  # (the members' tables are there)
     zero = [b.get_kernels(m) for m in range(2)]
     # (a store that failed is tried again from its first array)
     _lib.check(lib.psv_batch_fail_allocation(b._h, 1, n, times))
@@ -190,3 +201,59 @@ def test_batch_gradients(n, times):
         for m in range(2):
             _same(b.get_kernels(m), want.get_kernels(m), (n, times, k, m))
     assert b.resident()
+
+
+@pytest.mark.parametrize("n, times", [(0, 1), (4, 1), (10, 1), (11, 1), (12, 1), (13, 1), (14, 1),
+                                      (0, 30)])
+def test_tables_of_a_loop_kernel(n, times):
+    """A kernel's 11 tables that find no room: another kernel or, where none has
+    room, loops by steps; and the first kernel again the next time.  Then the
+    words, the arguments and the cells of the first launch."""
+    import psvwave_amd
+    from psvwave_amd import _lib
+    from test_gpu_loop_kernels import _rows
+    print(f"[allocation] tables {n} {times}", flush=True)
+    cfg = _cfg(131, 77, nt=60, shots=3)
+    m = psvwave_amd.fdModel(cfg)
+    lib = _lib.load()
+    lib.psv_fail_allocation.argtypes = [C.c_void_p, C.c_int, C.c_int]
+    _lib.check(lib.psv_fail_allocation(m._h, n, times))
+    fields = _fields(psvwave_amd.fdModel(cfg), 6)
+    m.set_parameter_fields(*fields)
+    try:
+        for s in range(m.n_shots):
+            m.forward_simulate(s, store_fields=False)
+        m.synchronize()
+    except RuntimeError as e:  # the loops by steps found no room either
+        assert times > 1 and "memory" in str(e)
+    else:
+        _same(m.get_synthetic_data(), _reference(cfg, 6)[1:3], (n, times))
+    _lib.check(lib.psv_fail_allocation(m._h, 0, 0))
+    for _ in range(64):  # the forwards by steps that may follow
+        m.forward_simulate(0, store_fields=False)
+    rows = C.c_int()
+    lib.psv_resident_rows.argtypes = [C.c_void_p, C.c_int, C.POINTER(C.c_int)]
+    for loops in (1, 3):
+        _lib.check(lib.psv_resident_rows(m._h, loops, C.byref(rows)))
+        assert rows.value == _rows(cfg, loops) > 0
+    _same(_run(m, cfg, 7), _reference(cfg, 7), "afterwards")
+
+
+def test_tables_of_a_batch():
+    """No room for a member's tables: by steps, and resident the next time."""
+    from psvwave_amd import _lib
+    print("[allocation] batch tables", flush=True)
+    lib = _lib.load()
+    lib.psv_batch_fail_allocation.argtypes = [C.c_void_p, C.c_int, C.c_int, C.c_int]
+    cfgs = [_cfg(133, 71, shots=2, nt=40), _cfg(90, 61, shots=2, nt=40)]
+    b, want = _batch(cfgs), _batch(cfgs, 28)
+    want.forward_all()
+    # every kernel's tables, then the state of a lockstep by steps
+    _lib.check(lib.psv_batch_fail_allocation(b._h, 1, 0, 30))
+    b.forward_all()
+    _lib.check(lib.psv_batch_fail_allocation(b._h, 1, 0, 0))
+    for k in range(2):
+        for m in range(2):
+            _same(b.get_synthetic_data(m), want.get_synthetic_data(m), (k, m))
+        assert b.resident()
+        b.forward_all()
