@@ -215,7 +215,9 @@ int psv_load_model(psv_model *m, const char *de_path, const char *vp_path,
  * the 64 x 16 lean kernel with ring-point operands in LDS (four waves per
  * SIMD), 27 / 28 variants 24 / 26 with their loads capped to the grid (the
  * tiles on the right and bottom edges read no padding; 27 is the default
- * when dx, dz lie in [2^-40, 2^40]).
+ * when dx, dz lie in [2^-40, 2^40]).  Without this call grids that fit the
+ * device run as resident time loops (one launch per time loop) instead; with
+ * it the model runs the chosen kernel step by step from then on.
  * All variants give bitwise identical results.  xcd_remap: 1 keeps
  * neighbouring tiles on one XCD.
  * timing_stride k > 0 records the kernel start and end of every k-th step
@@ -278,7 +280,9 @@ int psv_stream_pressure(int *live_streams, int *hw_queues);
  * Monte-Carlo purpose; copy() at src/psvWave.cpp:421-425 is its only way to
  * multiply models).  A batch holds n independent models of possibly
  * different sizes sharing nt and n_shots; psv_batch_forward advances every
- * model of one shot with one launch per time step over all their tiles.
+ * model of one shot, in resident time loops packed into as few launches as hold
+ * them (psv_batch_resident) or with one launch per time step over all their
+ * tiles.
  * Each member behaves as the model psv_create(&params[m]) would:
  * seismograms are bit-identical to running the members one by one. */
 typedef struct psv_batch psv_batch;
@@ -295,7 +299,7 @@ int psv_batch_get_synthetic_data(const psv_batch *b, int m, double *ux,
 /* Forward simulation of shot i_shot for every model (no snapshots). */
 int psv_batch_forward(psv_batch *b, int i_shot);
 /* Forward simulation of every shot of every model (what psv_batch_forward
- * for shots 0 .. n_shots-1 does, bit for bit).  With 2 to 8 shots and a
+ * for shots 0 .. n_shots-1 does, bit for bit).  By steps with 2 to 8 shots and a
  * lean step variant the shots advance together, one launch per time step
  * over every (tile, shot) of every model, shot s in the model's state buffer
  * set s (10 padded grids more per model and extra shot; shot by shot when
@@ -318,7 +322,7 @@ int psv_batch_set_variant(psv_batch *b, int variant, int xcd_remap);
 /* FWI gradient of every member against its observed data (what
  * psv_run_model(m, 0, 1) does for one model): kernels reset, then shot by
  * shot the forward storing snapshots, the adjoint sources and the adjoint
- * with kernel correlation -- one launch per time step over every member --
+ * with kernel correlation -- by steps with one launch over every member each --
  * then misfits (psv_batch_misfits) and velocity kernels
  * (psv_batch_get_kernels, (nx, nz) each).  Needs one snapshot_interval for
  * all members, dividing nt, and step variant 0, 1, 8-13 or 18-28; each
@@ -334,7 +338,9 @@ int psv_batch_set_persistent(psv_batch *b, int on);
 /* Times `steps` batched steps of variants 0, 1, 6, 7, 8-13, 18-20, 22-24,
  * 26-28 (ms_per_step[19]: ms per time step of one shot, -1 for a variant the batch
  * cannot use) in the loop psv_batch_forward_all runs with each, and keeps
- * the fastest (*best).  Overwrites the synthetic data. */
+ * the fastest (*best) -- or the resident time loops where they are faster
+ * still (psv_batch_resident; psv_batch_set_variant would give them up).
+ * Overwrites the synthetic data. */
 int psv_batch_autotune(psv_batch *b, int steps, int *best,
                        double *ms_per_step);
 /* Summed wall time of psv_batch_forward time loops (HIP events) and the

@@ -2,8 +2,9 @@
 
 The reference runs one ``fdModel`` at a time (its stated purpose is
 Monte-Carlo simulation, README.md:16-17).  A ``Batch`` holds n members that
-share ``nt`` and ``n_shots``; ``forward(i_shot)`` advances every member with
-one kernel launch per time step over the tiles of all members.  Each
+share ``nt`` and ``n_shots``; ``forward(i_shot)`` advances every member, in
+resident time loops packed into as few launches as hold them, or with one
+kernel launch per time step over the tiles of all members.  Each
 member's results equal those of ``fdModel(config)`` run alone, bit for bit.
 """
 import ctypes as C
@@ -109,7 +110,7 @@ class Batch:
         """FWI gradient of every member against its observed data (each
         member's run_model: forward with snapshots, misfit, adjoint sources,
         kernel reset, adjoint with correlation, kernel mapping), shot by
-        shot with one launch per time step over all members.  Returns the
+        shot over all members at once.  Returns the
         misfits; the velocity kernels come from get_kernels(m)."""
         _lib.check(self._lib.psv_batch_gradients(self._h))
         out = np.empty(len(self))
@@ -139,8 +140,11 @@ class Batch:
     def autotune(self, steps=20):
         """Time variants 0, 1, 6, 7, 8-13, 18-20, 22-24, 26-28 over `steps` steps,
         each in the loop forward_all runs with it (all shots in lockstep
-        where that applies), and keep the fastest.  Returns (best variant,
-        {variant: ms per time step of one shot})."""
+        where that applies), and keep the fastest, or the resident time loops
+        where they are faster still.  Returns (best variant,
+        {variant: ms per time step of one shot}) of the step kernels;
+        resident() tells whether the batch runs the resident loops, which
+        set_variant would give up."""
         best = C.c_int()
         ms = np.zeros(len(AUTOTUNE_VARIANTS))
         _lib.check(self._lib.psv_batch_autotune(self._h, int(steps), C.byref(best),

@@ -22,11 +22,15 @@ constexpr LoopKind kLoopKinds[] = {{1, 8}, {2, 8}, {3, 8}, {4, 8}, {4, 16}};
 constexpr int kNumLoopKinds = 5;
 constexpr int kLoopTileX = 60;
 // Loop kernels and blocks per compute unit in the order of their time per step
-// (2.9, 3.5, 4.0, 4.3, 5.2, 6.0, 6.5, 7.8 and 7.9 us): launches take the first
-// whose tiles all fit.  Fewer rows a wave make a step shorter, and so does a
-// block alone on its unit, up to a wave of rows less: 960 x 448 points take 6.0
-// us on 256 tiles of 28 rows and 6.5 on 368 of 20, 800 x 700 points 6.5 on 490
-// of 20 rows and 7.7 on 350 of 28.
+// (3.1, 3.9, 3.7, 4.8 to 5.1, 5.3, 5.9, 6.2, 7.6 and 7.8 to 8.1 us, a forward
+// with 19 receivers on a grid that each of them holds and the one before does
+// not): launches take the first whose tiles all fit.  Fewer rows a wave make a
+// step shorter, and so does a block alone on its unit, up to a wave of rows
+// less: compared in one run each, 960 x 448 points took 6.0 us on 256 tiles of
+// 28 rows and 6.5 on 368 of 20, 800 x 700 points 6.5 on 490 of 20 rows and 7.7
+// on 350 of 28.  (The third,
+// two blocks of 4 rows, comes up only where a tile of 12 rows has too many
+// receivers.)
 struct LoopFit {
   int kind, per_unit;
 };

@@ -12,10 +12,11 @@
 // What bounds a step is FP64 issue (about 111 FP64 instructions per point and
 // 40 others, at 1.8 ns per wave and instruction) plus one exchange, about 2 us
 // from the last store to the first value read.  The exchange is hidden only
-// where two blocks share a compute unit.  us per step: 250 x 150 points 2.9
-// (a launch per step: 7.7), 680 x 380 4.7, 960 x 448 on one block per compute
-// unit 5.8 and two such loops on two 8.1 (107e9 points per second), 1800 x
-// 450 7.8 (27).
+// where two blocks share a compute unit.  us per step of a forward (19
+// receivers, no snapshots): 250 x 150 points 3.1 (a launch per step: 8.6),
+// 680 x 380 4.8 to 5.1, 960 x 448 on one block per compute unit 5.9 and two
+// such loops on two 8.0 (108e9 points per second), 1800 x 450 7.6 (a launch
+// per step: 27).
 //
 // Tile.  Lane l of every wave is column x0 - 2 + l, wave w holds the rows
 // q = w P .. w P + P - 1 of the tile, row q being z0 - 2 + q.  The velocity
@@ -775,8 +776,9 @@ resident_loop(LoopLaunch l) {
       };
       begin_step(k + 1);
       // polls share the fabric with the cells they wait for: asking at once
-      // and without pause cost 960 x 448 points 6.8 us per step, these pauses
-      // (of 64 cycles each) make it 6.0, longer ones no less
+      // and without pause cost 960 x 448 points 6.8 us per step against 6.0 with
+      // these pauses (of 64 cycles each; both measured together), longer ones no
+      // less
       __builtin_amdgcn_s_sleep(P == 4 ? 8 : 4);
       poll();
       for (unsigned spin = 0;;) {

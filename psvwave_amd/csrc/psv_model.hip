@@ -1022,8 +1022,9 @@ LoopArgs Model::loop_args(int kind, int i_shot, bool forward) const {
 // Adds a job; launches the pending ones before a job they cannot share a
 // launch with, and once there are as many as run together.
 void Model::push_loop(int kind, int shot, bool store) {
-  // the second stream, which checkpointed adjoints use beside this one, opens
-  // with the first call as it does for loops by steps
+  // the second stream opens with the first call, as it does for loops by steps:
+  // checkpointed adjoints and loops after a refused launch use it, and the count
+  // of live streams does not depend on the way a loop runs
   if (!lane_stream_) create_stream(&lane_stream_);
   const bool fwd = kind == kJobForward;
   bool apart = false;

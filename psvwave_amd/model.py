@@ -423,7 +423,9 @@ class fdModel:
         with halo columns and ring operands by DMA (6 waves per SIMD); 25
         the same without the halo columns; 26 lean 64x16 with ring operands
         by DMA (4 waves per SIMD); 27 (the default), 28 variants 24, 26 with
-        their loads capped to the grid (edge tiles read no padding)."""
+        their loads capped to the grid (edge tiles read no padding).  A model
+        that has not been given one runs resident time loops where its grid
+        fits the device; one that has runs by steps from then on."""
         _lib.check(self._lib.psv_set_step_variant(self._h, int(variant),
                                                   int(bool(xcd_remap))))
 

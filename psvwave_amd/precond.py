@@ -7,9 +7,9 @@ the surface.  Models are a smooth Gaussian-random-field background plus a
 +-5 % random perturbation inside the kernel region.
 
 * ``gradient_pairs``: (gradient at the background, true perturbation) pairs,
-  computed for many models at once by the batched solver (``Batch``: one
-  launch per time step over every member, forward and adjoint with kernel
-  correlation).
+  computed for many models at once by the batched solver (``Batch``: the
+  members' time loops packed into common launches, forward and adjoint with
+  kernel correlation).
 * ``UNet``: a 4-level U-Net (32 base channels) mapping the normalised
   velocity kernels to a relative model update.  ``train_hip`` /
   ``HipUNetTrainer`` train it and ``HipUNet`` runs it on this library's
@@ -128,8 +128,8 @@ def gradient_pairs(n, seed=7, batch_size=256, cfg=None, log=None, along_path=0.0
 
     The device solver runs `batch_size` pairs at once as one Batch: the
     true models' forward runs give the observed data, then Batch.gradients
-    computes every member's gradient (bitwise each model's run_model) with
-    one launch per time step over all members.  The next batch's models are
+    computes every member's gradient (bitwise each model's run_model), all
+    members at once.  The next batch's models are
     drawn on a host thread meanwhile.  Pair k depends only on (seed, k)."""
     from concurrent.futures import ThreadPoolExecutor
     from .batch import Batch
