@@ -407,12 +407,12 @@ bool Batch::run_loops(LoopLaunches &p, int steps, bool redo) {
     l.sync = loop_sync_ + 2 * i;
     l.poison = loop_poison_;
     l.status = loop_status_ + i;
+    loop_tag_ += (unsigned)steps;  // spent, also where an error follows the launch
     try {
       gated_launch_loop(p.kind, !p.forward, l, stream_);
     } catch (const RuntimeError &) {
       break;
     }
-    loop_tag_ += (unsigned)steps;
   }
   hip_check(hipStreamSynchronize(stream_), "hipStreamSynchronize");
   bool missing = false;

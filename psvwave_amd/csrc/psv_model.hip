@@ -1155,8 +1155,8 @@ void Model::launch_loops(int first, int n) {
   l.sync = loop_sync_;
   l.poison = loop_poison_;
   l.status = loop_status_ + first;
+  loop_tag_ += (unsigned)cfg_.nt;  // spent, also where an error follows the launch
   gated_launch_loop(kind, !fwd, l, stream_);
-  loop_tag_ += (unsigned)cfg_.nt;
   launches_ += (int64_t)n * cfg_.nt;
 }
 
@@ -1399,8 +1399,8 @@ void Model::run_checkpointed_resident(int i_shot) {
     l.sync = sync_words;
     l.poison = loop_poison_;
     l.status = loop_status_ + word;
-    gated_launch_loop(kind, !fwd, l, s);
     loop_tag_ += (unsigned)(a.k1 - a.k0);
+    gated_launch_loop(kind, !fwd, l, s);
     launches_ += a.k1 - a.k0;
   };
   hip_check(hipEventRecord(ev_start, stream_), "hipEventRecord");
